@@ -230,8 +230,8 @@ spt_status spt_bvh_export(const spt_bvh* bvh, spt_node64* nodes, spt_tri48* tris
                           float* root_box);
 /* Writes the reference's tree dump text format (acceleration/sbvh.cpp:577-620). */
 spt_status spt_bvh_dump(const spt_bvh* bvh, const char* path);
-/* The four-wide compressed tree the throughput traversal reads, for
- * inspection (no reference counterpart). Node (64 B, 16 u32): grid origin
+/* A compressed four-wide form of the tree, for inspection (no reference
+ * counterpart; the traversal reads its own four-wide tree with smaller boxes). Node (64 B, 16 u32): grid origin
  * x y z (f32); biased exponent bytes of the per-axis grid step 2^e (bytes
  * 0-2); six words of child bytes q (lo.x hi.x lo.y hi.y lo.z hi.z, byte i =
  * child i; bound = origin + q * 2^e, lo rounded down, hi up); two words of
@@ -371,7 +371,7 @@ typedef struct spt_tuning {
                                       a render allocates min(paths of the call, capacity), halved
                                       while the device has no room, down to 2^20) */
     uint32_t extend_blocks_per_cu; /* persistent traversal grid (default: the occupancy limit on
-                                      one wavefront, at most 4 each for two, 2 for more) */
+                                      one wavefront, at most 5 each for two, 4 for more) */
     uint32_t shade_blocks_per_cu;  /* shading grid, at most 1024 (default 128 on one wavefront,
                                       64 with several) */
     uint32_t use_graph;            /* 1: bounce loop captured once in a HIP graph and replayed;
@@ -379,9 +379,10 @@ typedef struct spt_tuning {
     uint32_t tile_pixels;          /* multi-scene calls: pixels per generation tile (default 4096) */
     uint32_t tile_samples;         /* multi-scene calls: samples per tile (default 16) */
     uint32_t check_every;          /* bounces the host may run ahead of the device (default 4) */
-    uint32_t refill_lanes;         /* a traversal wave fetches new rays once this many of
-                                      its 64 lanes are idle (default in path tracing 48 on one
-                                      wavefront, 20 with several; 16 in spt_trace) */
+    uint32_t refill_lanes;         /* a traversal wave fetches new rays once this many of its 64
+                                      lanes (four per ray) are idle; more than 24 act as 24
+                                      (default in path tracing 48 on one wavefront, 20 with
+                                      several; 20 in spt_trace) */
     uint32_t wavefronts;           /* unguided renders: independent wavefronts run at once on
                                       their own streams, each with a share of the paths and of
                                       the queue capacity, so one's traversal overlaps another's

@@ -181,7 +181,7 @@ class Bvh:
         return nodes, tris, leaf, box
 
     def wide(self):
-        """The compressed four-wide tree the traversal reads (spt_bvh_wide):
+        """A compressed four-wide form of the tree (spt_bvh_wide):
         nodes (n, 16) uint32 and leaf records (m, 8) uint32 (float fields as
         their bits)."""
         nn, nl = C.c_uint64(0), C.c_uint64(0)

@@ -8,7 +8,7 @@
 #include <cstring>
 #include <new>
 
-#include "spt_device.h"
+#include "spt_quad.h"
 
 namespace spt {
 
@@ -87,14 +87,15 @@ namespace {
 
 void free_scene(spt_ctx* ctx) {
     if (ctx->d_nodes) (void)hipFree(ctx->d_nodes);
-    if (ctx->d_nodesq) (void)hipFree(ctx->d_nodesq);
-    if (ctx->d_leaves) (void)hipFree(ctx->d_leaves);
+    if (ctx->d_qnodes) (void)hipFree(ctx->d_qnodes);
+    if (ctx->d_qprims) (void)hipFree(ctx->d_qprims);
+    if (ctx->d_qboxes) (void)hipFree(ctx->d_qboxes);
     if (ctx->d_tris) (void)hipFree(ctx->d_tris);
     if (ctx->d_shading) (void)hipFree(ctx->d_shading);
     ctx->d_nodes = nullptr;
-    ctx->d_nodesq = nullptr;
-    ctx->d_leaves = nullptr;
-    ctx->n_nodesq = ctx->n_leaves = 0;
+    ctx->d_qnodes = nullptr;
+    ctx->d_qprims = nullptr;
+    ctx->d_qboxes = nullptr;
     ctx->d_tris = nullptr;
     ctx->d_shading = nullptr;
     ctx->n_nodes = ctx->n_tris = 0;
@@ -171,7 +172,56 @@ void scene_arrays(const spt_bvh* bvh, const float* verts, const float* normals, 
 
 uint32_t tree_stack_cap(const spt_node64* nodes, uint32_t n) { return tree_depth(nodes, n) + 1; }
 
+// ---------------------------------------------------------------------------
+// The compressed four-wide tree spt_bvh_wide returns (for inspection; the
+// kernels read the quad tree).
+// ---------------------------------------------------------------------------
 namespace {
+
+// Four-wide node collapsed from the binary
+// tree (children are binary-tree nodes or leaves two levels down, with their
+// own padded boxes): child boxes as six float4 (lo.x of the 4 children, hi.x,
+// lo.y, hi.y, lo.z, hi.z), then the child words and leaf counts.
+struct Node4 {
+    float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];
+    uint32_t child[4];  // inner: Node4 index; leaf: first triangle; unused: kNoChild
+    uint32_t count[4];  // leaf: triangle count (> 0); inner or unused: 0
+};
+static_assert(sizeof(Node4) == 128, "Node4 layout");
+constexpr uint32_t kNoChild = 0xFFFFFFFFu;
+
+// Compressed four-wide node (64 B):
+// each axis has a per-node grid origin + q * 2^e, and every child bound is
+// rounded outward to a byte q (lo down, hi up), so the decoded boxes contain
+// the exact padded child boxes (the traversal visits a superset of the exact
+// four-wide tree's boxes; results do not depend on visit order).
+//   word 0-2: grid origin x y z (float); word 3: biased exponent bytes of
+//   2^e_x, 2^e_y, 2^e_z (float exponent field, bytes 0-2)
+//   words 4-9: q of lo.x, hi.x, lo.y, hi.y, lo.z, hi.z (byte i = child i)
+//   words 10-11: 16-bit triangle counts of the children (0: inner or unused;
+//   0xFFFF: 65535 or more, the full count is in the leaf's box record)
+//   words 12-15: children: NodeQ index (inner), first triangle (leaf), kNoChild
+// A leaf's range is read from the node that holds it, which the traversal
+// has just visited; its exact box (the reference's hit-point-inside-leaf
+// test) sits in a side array at 4 * node + slot and is read only when a
+// triangle of the leaf passes the t tests.
+struct NodeQ {
+    float ox, oy, oz;
+    uint32_t exps;
+    uint32_t q[6];
+    uint32_t cnt[2];
+    uint32_t child[4];
+};
+static_assert(sizeof(NodeQ) == 64, "NodeQ layout");
+
+// Exact padded box of the leaf in slot s of node i, at index 4 i + s (32 B).
+struct LeafRec {
+    float mn[3];
+    uint32_t cnt;  // full triangle count
+    float mx[3];
+    uint32_t pad;
+};
+static_assert(sizeof(LeafRec) == 32, "LeafRec layout");
 
 struct Entry4 {
     float lo[3], hi[3];
@@ -194,22 +244,20 @@ void side(const spt_node64& nd, int s, Entry4& e) {
     e.cnt = s == 0 ? nd.lcnt : nd.rcnt;
 }
 
-}  // namespace
-
-uint32_t collapse4(const spt_node64* nodes, uint32_t n, std::vector<Node4>& out) {
+// Collapses a pre-order pair-node tree into four-wide nodes (pre-order, root
+// first).
+void collapse4(const spt_node64* nodes, uint32_t n, std::vector<Node4>& out) {
     out.clear();
-    if (n == 0) return 1;
-    // work list: binary node, the Node4 slot it fills, its depth
+    if (n == 0) return;
+    // work list: binary node, the Node4 slot it fills
     struct Item {
-        uint32_t bin, slot, depth;
+        uint32_t bin, slot;
     };
-    std::vector<Item> work{{0u, 0u, 1u}};
+    std::vector<Item> work{{0u, 0u}};
     out.emplace_back();
-    uint32_t max_depth = 1;
     while (!work.empty()) {
         const Item j = work.back();
         work.pop_back();
-        max_depth = std::max(max_depth, j.depth);
         // the binary node's two children, then the inner child with the
         // largest surface area is opened until there are four
         Entry4 e[4];
@@ -244,7 +292,7 @@ uint32_t collapse4(const spt_node64* nodes, uint32_t n, std::vector<Node4>& out)
                 } else {
                     q.child[i] = (uint32_t)out.size();
                     out.emplace_back();
-                    work.push_back({e[i].ref, q.child[i], j.depth + 1});
+                    work.push_back({e[i].ref, q.child[i]});
                 }
             } else {
                 q.lox[i] = q.loy[i] = q.loz[i] = 0.0f;
@@ -255,10 +303,7 @@ uint32_t collapse4(const spt_node64* nodes, uint32_t n, std::vector<Node4>& out)
         }
         out[j.slot] = q;
     }
-    return 3 * max_depth + 1;
 }
-
-namespace {
 
 // The value the traversal decodes for byte q (qdec): origin + q * scale in
 // float, q * scale exact.
@@ -301,8 +346,9 @@ uint32_t quantize_axis(const float* lo, const float* hi, const bool* used, float
     return (uint32_t)(e + 127);
 }
 
-}  // namespace
-
+// Appends the compressed form of a four-wide tree (and four leaf box slots
+// per node): inner children rebased by the node array's size, leaf ranges by
+// tri_base. Returns false when an index would not fit its field.
 bool compress4(const std::vector<Node4>& in, uint32_t tri_base, std::vector<NodeQ>& nodes, std::vector<LeafRec>& leaves) {
     const uint64_t node_base = nodes.size();
     // leaf stack entries hold node << 2 | slot below kLeafBit
@@ -341,6 +387,8 @@ bool compress4(const std::vector<Node4>& in, uint32_t tri_base, std::vector<Node
     return true;
 }
 
+}  // namespace
+
 }  // namespace spt
 
 using namespace spt;
@@ -351,7 +399,7 @@ spt_status spt_bvh_wide(const spt_bvh* bvh, void* nodes, uint64_t* n_nodes, void
     if (!bvh || !n_nodes || !n_leaves) return SPT_ERR_INVALID;
     const std::vector<spt_node64>& bn = bvh_nodes(bvh);
     std::vector<Node4> n4;
-    (void)collapse4(bn.data(), (uint32_t)bn.size(), n4);
+    collapse4(bn.data(), (uint32_t)bn.size(), n4);
     std::vector<NodeQ> nq;
     std::vector<LeafRec> lr;
     if (!compress4(n4, 0u, nq, lr)) return SPT_ERR_UNSUPPORTED;
@@ -394,6 +442,10 @@ spt_status spt_create(int device, spt_ctx** out) {
         delete ctx;
         return SPT_ERR_DEVICE;
     }
+    if (hipMalloc(&ctx->d_rays, kRayCounterWords * 4) != hipSuccess) {
+        spt_destroy(ctx);
+        return SPT_ERR_DEVICE;
+    }
     // status words the bounce loop writes for the host (mapped host memory)
     void* hs = nullptr;
     if (hipHostMalloc(&hs, 256, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) hs = nullptr;
@@ -424,6 +476,7 @@ void spt_destroy(spt_ctx* ctx) {
     if (ctx->d_mats) (void)hipFree(ctx->d_mats);
     if (ctx->d_spill) (void)hipFree(ctx->d_spill);
     if (ctx->d_flags) (void)hipFree(ctx->d_flags);
+    if (ctx->d_rays) (void)hipFree(ctx->d_rays);
     if (ctx->d_paths) (void)hipFree(ctx->d_paths);
     if (ctx->guide.d_theta) (void)hipFree(ctx->guide.d_theta);
     if (ctx->guide.d_records) (void)hipFree(ctx->guide.d_records);
@@ -518,14 +571,13 @@ spt_status spt_upload_scene(spt_ctx* ctx, const spt_node64* nodes, uint32_t n_no
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     free_scene(ctx);
-    std::vector<Node4> n4;
-    const uint32_t cap4 = collapse4(nodes, n_nodes, n4);
-    std::vector<NodeQ> nq;
-    std::vector<LeafRec> leaves;
-    if (!compress4(n4, 0u, nq, leaves)) return set_error(ctx, SPT_ERR_INVALID, "tree over 2^29 four-wide nodes");
+    QuadTree qt;
+    const uint32_t cap4 = append_quad_tree(nodes, n_nodes, tris, n_tris, root_box, 0u, qt);
+    if (cap4 == 0) return set_error(ctx, SPT_ERR_INVALID, "tree over 2^31 four-wide nodes");
     spt_status s = upload(ctx, &ctx->d_nodes, nodes, (size_t)n_nodes * sizeof(spt_node64), "nodes");
-    if (s == SPT_OK) s = upload(ctx, &ctx->d_nodesq, nq.data(), nq.size() * sizeof(NodeQ), "compressed nodes");
-    if (s == SPT_OK) s = upload(ctx, &ctx->d_leaves, leaves.data(), leaves.size() * sizeof(LeafRec), "leaf records");
+    if (s == SPT_OK) s = upload(ctx, &ctx->d_qnodes, qt.nodes.data(), qt.nodes.size() * sizeof(QuadNode), "quad nodes");
+    if (s == SPT_OK) s = upload(ctx, &ctx->d_qprims, qt.prims.data(), qt.prims.size() * sizeof(QuadPrim), "quad blocks");
+    if (s == SPT_OK) s = upload(ctx, &ctx->d_qboxes, qt.boxes.data(), qt.boxes.size() * sizeof(QuadBox), "leaf boxes");
     if (s == SPT_OK) s = upload(ctx, &ctx->d_tris, tris, (size_t)n_tris * sizeof(spt_tri48), "triangles");
     std::vector<float> flat;
     if (s == SPT_OK) {
@@ -562,9 +614,9 @@ spt_status spt_upload_scene(spt_ctx* ctx, const spt_node64* nodes, uint32_t n_no
     std::memcpy(ctx->root_box, root_box, sizeof(ctx->root_box));
     ctx->root_leaf = n_nodes == 0 ? n_tris : 0;
     ctx->stack_cap = tree_depth(nodes, n_nodes) + 1;
-    ctx->n_nodesq = (uint32_t)nq.size();
-    ctx->n_leaves = (uint32_t)leaves.size();
     ctx->stack_cap4 = cap4;
+    ctx->small_coords = quad_small_coords(tris, n_tris);
+    ctx->small_tree = qt.small();
     ctx->max_mat = 0;
     ctx->has_spheres = false;
     for (uint32_t i = 0; i < n_tris; ++i) {

@@ -15,8 +15,8 @@ namespace spt {
 namespace {
 
 void free_batch(BatchData& b) {
-    void* ptrs[] = {b.d_nodes, b.d_nodesq, b.d_leaves,     b.d_tris, b.d_shading, b.d_mats,
-                    b.d_jobs,  b.d_tiles,  b.d_tile_start, b.d_done, b.d_clock};
+    void* ptrs[] = {b.d_nodes, b.d_qnodes, b.d_qprims,     b.d_qboxes, b.d_tris, b.d_shading, b.d_mats,
+                    b.d_jobs,  b.d_tiles,  b.d_tile_start, b.d_done,   b.d_clock};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     b = BatchData{};
@@ -80,7 +80,7 @@ spt_status tune(spt_ctx* ctx, bool batch, F run, spt_tuning* out) {
         {&spt_tuning::shade_blocks_per_cu, {16u, 32u, 64u, 128u}},
         {&spt_tuning::use_graph, {2u, 1u}},
         {&spt_tuning::check_every, {2u, 4u, 8u}},
-        {&spt_tuning::refill_lanes, {16u, 32u, 48u, 56u}},
+        {&spt_tuning::refill_lanes, {8u, 16u, 24u}},
         {&spt_tuning::wavefronts, {3u, 2u, 1u}},
     };
     if (batch) {
@@ -165,8 +165,7 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
     if (!ctx || !scenes || n == 0 || !out) return SPT_ERR_INVALID;
     *out = nullptr;
     std::vector<spt_node64> nodes;
-    std::vector<NodeQ> nodesq;
-    std::vector<LeafRec> leaves;
+    QuadTree qt;
     std::vector<spt_tri48> tris;
     std::vector<float> sh;
     std::vector<spt_material> mats;
@@ -208,16 +207,18 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
             nd.rref += (nd.rcnt == 0) ? (uint32_t)node_base : (uint32_t)tri_base;
             nodes.push_back(nd);
         }
-        std::vector<Node4> b4;
-        d.stack_cap4 = std::max(d.stack_cap4, collapse4(bn.data(), (uint32_t)bn.size(), b4));
-        const uint64_t node4_base = nodesq.size();
-        if (!compress4(b4, (uint32_t)tri_base, nodesq, leaves))
-            return fail(set_error(ctx, SPT_ERR_UNSUPPORTED, "batch exceeds 2^31 four-wide nodes or leaves"));
-        for (spt_tri48 t : bt) {
+        for (spt_tri48& t : bt) {
             t.pad[0] += (uint32_t)mat_base;
             d.has_spheres = d.has_spheres || t.pad[1] == SPT_PRIM_SPHERE;
-            tris.push_back(t);
         }
+        tris.insert(tris.end(), bt.begin(), bt.end());
+        d.small_coords = d.small_coords && quad_small_coords(bt.data(), (uint32_t)bt.size());
+        const float* rb = bvh_root_box(sc.bvh);
+        const uint64_t qnode_base = qt.nodes.size();
+        const uint32_t cap4 = append_quad_tree(bn.data(), (uint32_t)bn.size(), bt.data(), (uint32_t)bt.size(), rb,
+                                               (uint32_t)tri_base, qt);
+        if (cap4 == 0) return fail(set_error(ctx, SPT_ERR_UNSUPPORTED, "batch exceeds 2^31 four-wide nodes or blocks"));
+        d.stack_cap4 = std::max(d.stack_cap4, cap4);
         for (size_t k = 0; k < bt.size(); ++k) {
             float* o = &bs[k * 12];
             uint32_t m;
@@ -227,22 +228,20 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
         }
         sh.insert(sh.end(), bs.begin(), bs.end());
         mats.insert(mats.end(), sc.mats, sc.mats + sc.n_mats);
-        const float* rb = bvh_root_box(sc.bvh);
         for (int k = 0; k < 3; ++k) {
             jb.rmin[k] = rb[k];
             jb.rmax[k] = rb[3 + k];
         }
-        jb.root_leaf = bn.empty() ? (uint32_t)bt.size() : 0u;
-        jb.node0 = (uint32_t)node4_base;  // persistent traversal starts at the scene's NodeQ root
-        jb.tri0 = (uint32_t)tri_base;
+        jb.node0 = (uint32_t)qnode_base;  // the traversal starts at the scene's root
         d.stack_cap = std::max(d.stack_cap, tree_stack_cap(bn.data(), (uint32_t)bn.size()));
         d.jobs.push_back(jb);
     }
     (void)hipSetDevice(ctx->device);
     uint64_t bytes = 0;
     spt_status s = upload_vec(ctx, reinterpret_cast<spt_node64**>(&d.d_nodes), nodes, "batch nodes", bytes);
-    if (s == SPT_OK) s = upload_vec(ctx, &d.d_nodesq, nodesq, "batch compressed nodes", bytes);
-    if (s == SPT_OK) s = upload_vec(ctx, &d.d_leaves, leaves, "batch leaf records", bytes);
+    if (s == SPT_OK) s = upload_vec(ctx, &d.d_qnodes, qt.nodes, "batch quad nodes", bytes);
+    if (s == SPT_OK) s = upload_vec(ctx, &d.d_qprims, qt.prims, "batch quad blocks", bytes);
+    if (s == SPT_OK) s = upload_vec(ctx, &d.d_qboxes, qt.boxes, "batch leaf boxes", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, reinterpret_cast<spt_tri48**>(&d.d_tris), tris, "batch triangles", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, reinterpret_cast<float**>(&d.d_shading), sh, "batch shading", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, &d.d_mats, mats, "batch materials", bytes);
@@ -250,6 +249,7 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
     if (s == SPT_OK) s = check_hip(ctx, hipMalloc(&d.d_done, n * sizeof(uint32_t)), "batch counters");
     if (s == SPT_OK) s = check_hip(ctx, hipMalloc(&d.d_clock, (n + 1) * sizeof(uint64_t)), "batch clocks");
     if (s != SPT_OK) return fail(s);
+    d.small_tree = qt.small();
     d.n_nodes = (uint32_t)nodes.size();
     d.n_tris = (uint32_t)tris.size();
     d.n_mats = (uint32_t)mats.size();

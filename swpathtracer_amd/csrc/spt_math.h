@@ -57,6 +57,21 @@ SPT_HD float sqrt_rn(float x) {
     return std::sqrt(x);
 #endif
 }
+// Correctly rounded 1 / x. On gfx950 v_rcp_f32 (at most 1 ulp off) followed
+// by one Newton step in two FMAs gives the IEEE quotient's bits for every
+// float with 2^-100 <= |x| <= 2^100 (all of them compared on the device); the
+// general expansion takes twice the instructions. Outside that range the
+// general form.
+SPT_HD float rcp_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float ax = __builtin_fabsf(x);
+    if (__builtin_expect(!(ax >= 0x1p-100f && ax <= 0x1p100f), 0)) return 1.0f / x;
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+#else
+    return 1.0f / x;
+#endif
+}
 SPT_HD V3 normalize(V3 v) { return v * (1.0f / sqrt_rn(dot(v, v))); }
 
 // 3x3 basis by columns; l2w = (u, v, w), w2l = its transpose.
@@ -131,7 +146,14 @@ SPT_HD bool tri_test(V3 o, V3 d, V3 v0, V3 e1, V3 e2, float& t, float& u, float&
     const V3 pvec = cross(d, e2);
     const float det = dot(e1, pvec);
     const bool det_ok = !((det > -1e-6f) && (det < 1e-6f));
+#if defined(__HIP_DEVICE_COMPILE__)
+    // rcp_rn without its lower bound: a smaller det is rejected whatever follows
+    const float r = __builtin_amdgcn_rcpf(det);
+    float inv_det = __builtin_fmaf(__builtin_fmaf(-det, r, 1.0f), r, r);
+    if (__builtin_expect(__builtin_fabsf(det) > 0x1p100f, 0)) inv_det = 1.0f / det;
+#else
     const float inv_det = 1.0f / det;
+#endif
     const V3 tvec = o - v0;
     u = dot(tvec, pvec) * inv_det;
     const bool u_ok = !((u < 0.0f) || (u > 1.0f));

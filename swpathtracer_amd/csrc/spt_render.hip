@@ -15,6 +15,7 @@
 
 #include "spt_bsdf.h"
 #include "spt_guide.h"
+#include "spt_quad.h"
 
 namespace spt {
 
@@ -46,7 +47,8 @@ struct Work {
     uint32_t* perm;    // shading order (stable counting sort by skey)
     uint32_t* bhist;   // [key][block] histogram, then exclusive offsets
     uint32_t* cnt;     // [0], [1]: live counts of the two buffers; [2]: replay overflows;
-                       // [8]: ray-fetch counter of the extend kernel; u64 at [10]: rays, u64 at [12]: bounces
+                       // u64 at [10]: rays, u64 at [12]: bounces
+    uint32_t* rays;    // ray counters of the extend kernel (kRayCounterWords)
 };
 constexpr size_t kWorkBytes = 16 + 4 + 4;
 
@@ -228,26 +230,25 @@ __global__ __launch_bounds__(kBlock) void k_generate(RenderArgs a, PathBuf A, Wo
 }
 
 // Work-word layout (w.cnt, 64 words): [0], [1] live counts of the two
-// buffers; [2] replay overflows; [8] ray-fetch counter of the extend kernel;
-// u64 [10] rays, u64 [12] bounces; [16] guide records, [17] candidates;
+// buffers; [2] replay overflows; u64 [10] rays, u64 [12] bounces; [16] guide records, [17] candidates;
 // u64 [20] next path to generate; [24] first slot and [25] number of the
 // planned new paths, u64 [26] their first path index; [28] plans made;
 // u64 [30] hits evaluated by the guide network.
 constexpr int kGen = 20, kPlanSlot = 24, kPlanN = 25, kPlanPath = 26, kPlanSeq = 28;
 
-// Between bounces (one thread): the consumed buffer's count and the
-// ray-fetch counter go back to zero (a kernel, not a memset, so the bounce
+// Between bounces (one wave): the consumed buffer's count and the extend
+// kernel's ray counters go back to zero (a kernel, not a memset, so the bounce
 // can be graph-captured), and new camera paths are planned into the free
 // tail of the survivors' buffer B: n = min(capacity - survivors, paths not
 // yet generated). Progress goes to mapped host memory: status[1] = live
 // paths after the refill, status[2] = all paths generated, then status[0] =
 // the plan's sequence number, so the host can stop issuing bounces without
 // waiting on the stream.
-__global__ void k_plan(uint32_t* cntA, uint32_t* cntB, uint32_t* cnt, uint32_t cap, uint64_t total,
+__global__ void k_plan(uint32_t* cntA, uint32_t* cntB, uint32_t* cnt, uint32_t* rays, uint32_t cap, uint64_t total,
                        uint32_t* status, uint64_t* job_clock) {
+    if (threadIdx.x < kRayCounters) rays[threadIdx.x * kRayCounterStride] = 0;
     if (threadIdx.x != 0) return;
     if (cntA) *cntA = 0;
-    cnt[8] = 0;
     const uint32_t have = *cntB;
     uint64_t* gen = reinterpret_cast<uint64_t*>(cnt + kGen);
     const uint64_t g0 = *gen;
@@ -283,38 +284,34 @@ __global__ __launch_bounds__(kBlock) void k_refill(RenderArgs a, PathBuf B, Work
 // traversal; hit record and sort key written at the path's slot. FETCH adds
 // node / triangle record fetch counts to the two 64-bit counters at flags + 4.
 template <bool FETCH, bool MULTI>
-__global__ __launch_bounds__(kBlock) void k_extend(RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_extend(RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA,
                                                    uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
-    __shared__ uint32_t lds[kLdsStack * kBlock];
+    __shared__ QuadLds lds;
     __shared__ unsigned long long fetched[2];
     const uint32_t n = *cntA;
     if (n == 0) return;
-    const uint32_t gthreads = gridDim.x * kBlock;
-    const uint32_t gtid = blockIdx.x * kBlock + threadIdx.x;
-    if (gtid == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         atomicAdd(reinterpret_cast<unsigned long long*>(w.cnt + 10), (unsigned long long)n);
         atomicAdd(reinterpret_cast<unsigned long long*>(w.cnt + 12), 1ull);
     }
-    Stack st(lds + threadIdx.x, spill + gtid, gthreads, a.sc.stack_cap4);
     bool overflow = false;
     unsigned long long my_nodes = 0, my_tris = 0;
     if (FETCH) {
         if (threadIdx.x < 2) fetched[threadIdx.x] = 0;
         __syncthreads();
     }
-    trace_persistent<FETCH>(
-        a.sc, n, w.cnt + 8, st, overflow, a.refill,
+    trace_quads<FETCH>(
+        a.sc, n, w.rays, lds, spill + (size_t)blockIdx.x * quad_spill_words(a.sc.stack_cap4), overflow, a.refill,
         [&](uint32_t i, V3& o, V3& d, Root& root) {
             const float4 o4 = A.o[i], d4 = A.d[i];
             o = V3{o4.x, o4.y, o4.z};
             d = V3{d4.x, d4.y, d4.z};
             if (MULTI) {
                 const Job& jb = a.jobs[__float_as_uint(d4.w)];
-                root = Root{V3{jb.rmin[0], jb.rmin[1], jb.rmin[2]}, V3{jb.rmax[0], jb.rmax[1], jb.rmax[2]},
-                            jb.root_leaf, jb.node0, jb.tri0};
+                root = Root{V3{jb.rmin[0], jb.rmin[1], jb.rmin[2]}, V3{jb.rmax[0], jb.rmax[1], jb.rmax[2]}, jb.node0};
             }
         },
-        [&](uint32_t i, const Hit& h, uint32_t nn, uint32_t nt) {
+        [&](uint32_t i, const Hit& h, V3, V3, uint32_t nn, uint32_t nt) {
             w.hit[i] = make_float4(h.t, __uint_as_float(h.idx), h.u, h.v);
             w.skey[i] = (h.idx == kNoHit) ? a.sc.n_mats : h.mat;
             if (FETCH) {
@@ -836,14 +833,13 @@ size_t guide_paths_lds_bytes() {
 }  // namespace
 
 // Defaults for the zero fields of a tuning.
-// Shading grid and traversal refill threshold by wavefront count: one
-// wavefront waits for 48 idle lanes before refilling and shades with 128
-// blocks per CU; with other wavefronts to cover a refill's stall, eager
-// refills and a smaller shading grid measured faster (902-908 against 843
-// Mpaths/s at three wavefronts).
+// Shading grid by wavefront count: one wavefront shades with 128 blocks per
+// CU; with other wavefronts beside it a smaller grid measured faster (1024-spp
+// mesh image, three wavefronts: 64 blocks 910 Mpaths/s, 32 893, 128 891). The
+// refill threshold of one wavefront acts as kMaxRefillLanes.
 void resolve_front_defaults(const spt_tuning& raw, spt_tuning& r, uint32_t fronts) {
     r.shade_blocks_per_cu = raw.shade_blocks_per_cu ? raw.shade_blocks_per_cu : (fronts > 1 ? 64u : 128u);
-    r.refill_lanes = raw.refill_lanes ? raw.refill_lanes : (fronts > 1 ? 20u : 48u);
+    r.refill_lanes = raw.refill_lanes ? raw.refill_lanes : (fronts > 1 ? kRefillLanes : 48u);
 }
 
 spt_tuning resolve_tuning(const spt_tuning& t) {
@@ -938,7 +934,7 @@ template <bool MULTI>
 spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuning& tn, spt_render_stats& stats) {
     uint64_t cap = std::min<uint64_t>(total, tn.path_capacity);
     auto state_bytes = [](uint64_t c) {
-        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + (size_t)kMaxSortKeys * kMaxSortBlocks * 4 + 4096;
+        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + (size_t)kMaxSortKeys * kMaxSortBlocks * 4 + 8192;
     };
     if (state_bytes(cap) > ctx->paths_bytes) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -979,10 +975,11 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     w.perm = (uint32_t*)take(cap * 4);
     w.bhist = (uint32_t*)take((size_t)kMaxSortKeys * kMaxSortBlocks * 4);
     w.cnt = (uint32_t*)take(256);
+    w.rays = (uint32_t*)take(kRayCounterWords * 4);
     if ((size_t)(base - reinterpret_cast<char*>(ctx->d_paths)) > ctx->paths_bytes)
         return set_error(ctx, SPT_ERR_NOMEM, "path state layout exceeds its allocation");
     a.rec_count = a.rec_shared ? a.rec_shared : w.cnt + 16;
-    a.refill = std::min<uint32_t>(64, std::max<uint32_t>(1, tn.refill_lanes));
+    a.refill = std::min<uint32_t>(kMaxRefillLanes, std::max<uint32_t>(1, tn.refill_lanes));
     if (a.guided) {
         const size_t need = (size_t)cap * guide::kOut * sizeof(unsigned short);
         if (need > ctx->guide.gout_cap) {
@@ -1004,21 +1001,21 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         per_cu = 4;
     if (tn.extend_blocks_per_cu)
         per_cu = std::min<int>(per_cu, (int)tn.extend_blocks_per_cu);
-    else if (tn.wavefronts > 1)  // concurrent wavefronts share the CUs (measured: 4 each for two, 2 for three)
-        per_cu = std::min<int>(per_cu, tn.wavefronts == 2 ? 4 : 2);
+    else if (tn.wavefronts > 1)  // concurrent wavefronts share the CUs: three with 3, 4, 5, 7 blocks each ran
+                                 // the 1024-spp mesh image at 911, 948, 897, 914 Mpaths/s
+        per_cu = std::min<int>(per_cu, tn.wavefronts == 2 ? 5 : 4);
     const uint32_t ext_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)(per_cu * ctx->num_cus));
     const uint32_t shade_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * tn.shade_blocks_per_cu);
     const uint32_t refill_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * 8);
     // sort chunks: many (latency hiding) unless many keys would make the scan long
     const uint32_t sort_blocks =
         a.keys ? std::max<uint32_t>(1024, std::min<uint32_t>(kMaxSortBlocks, 16384 / a.keys)) : 256;
-    spt_status s = ensure_spill(ctx, (size_t)ext_grid * kBlock *
-                                         (a.sc.stack_cap4 > kLdsStack ? a.sc.stack_cap4 - kLdsStack : 1));
+    spt_status s = ensure_spill(ctx, std::max<size_t>(1, (size_t)ext_grid * quad_spill_words(a.sc.stack_cap4)));
     if (s != SPT_OK) return s;
     hipStream_t st = ctx->stream;
     const bool timed = (a.flags & SPT_RENDER_TIME_KERNELS) != 0;
     const bool fetch_stats = (a.flags & SPT_RENDER_FETCH_STATS) != 0;
-    s = check_hip(ctx, hipMemsetAsync(w.cnt, 0, 256, st), "counters");
+    s = check_hip(ctx, hipMemsetAsync(w.cnt, 0, 256, st), "counters");  // the ray counters: k_plan
     if (s != SPT_OK) return s;
     if (a.train && !a.rec_shared) {  // records continue after those collected since the last training step
         s = check_hip(ctx,
@@ -1084,7 +1081,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         else
             hipLaunchKernelGGL((k_shade<MULTI, false>), dim3(shade_grid), dim3(kBlock), 0, st, a, A, B, w, cntA, cntB);
         // regeneration: the survivors' buffer is topped up with new camera paths
-        hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, cntA, cntB, w.cnt, (uint32_t)cap, total, ctx->d_status,
+        hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, cntA, cntB, w.cnt, w.rays, (uint32_t)cap, total, ctx->d_status,
                            a.job_clock);
         hipLaunchKernelGGL((k_refill<MULTI>), dim3(refill_grid), dim3(kBlock), 0, st, a, B, w);
         return check_hip(ctx, hipGetLastError(), "bounce launch");
@@ -1130,7 +1127,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         }
     } else {
         ctx->h_status[0] = 0;
-        hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, nullptr, w.cnt, w.cnt, (uint32_t)cap, total, ctx->d_status,
+        hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, nullptr, w.cnt, w.cnt, w.rays, (uint32_t)cap, total, ctx->d_status,
                            a.job_clock);
         hipLaunchKernelGGL((k_refill<MULTI>), dim3(refill_grid), dim3(kBlock), 0, st, a, buf[0], w);
         s = check_hip(ctx, hipGetLastError(), "generate launch");
@@ -1346,7 +1343,6 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
         a.job.rmin[i] = ctx->root_box[i];
         a.job.rmax[i] = ctx->root_box[3 + i];
     }
-    a.job.root_leaf = ctx->root_leaf;
     a.flags = prm->flags;
     a.per_path = a.job.path_rgb ? 1u : 0u;
     a.guided = (prm->flags & SPT_RENDER_GUIDED) ? 1u : 0u;
@@ -1468,8 +1464,11 @@ spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
 
     RenderArgs a{};
     a.sc.nodes = b.d_nodes;
-    a.sc.nodesq = reinterpret_cast<const uint4*>(b.d_nodesq);
-    a.sc.leaves = reinterpret_cast<const float4*>(b.d_leaves);
+    a.sc.qnodes = reinterpret_cast<const uint32_t*>(b.d_qnodes);
+    a.sc.qprims = reinterpret_cast<const float4*>(b.d_qprims);
+    a.sc.qboxes = reinterpret_cast<const float4*>(b.d_qboxes);
+    a.sc.small_coords = b.small_coords ? 1u : 0u;
+    a.sc.small_tree = b.small_tree ? 1u : 0u;
     a.sc.stack_cap4 = b.stack_cap4;
     a.sc.tris = b.d_tris;
     a.sc.shading = b.d_shading;

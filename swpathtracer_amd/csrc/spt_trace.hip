@@ -3,13 +3,14 @@
 // three ray casters (integrators/raycaster.h:61-99).
 #include <mutex>
 
-#include "spt_device.h"
+#include "spt_quad.h"
 
 namespace spt {
 
 namespace {
 
-template <bool PRUNE, bool COUNT, bool FETCH>
+// The reference's own node set on the binary tree (COUNT: with its counters).
+template <bool COUNT>
 __global__ __launch_bounds__(kBlock) void k_trace(DevScene sc, const float4* __restrict__ rays, uint64_t n,
                                                   uint2* __restrict__ hits, uint32_t* __restrict__ tests_out,
                                                   uint32_t* __restrict__ isects_out, uint32_t* __restrict__ spill,
@@ -23,10 +24,9 @@ __global__ __launch_bounds__(kBlock) void k_trace(DevScene sc, const float4* __r
         const float4 ro = rays[2 * i], rd = rays[2 * i + 1];
         Hit h;
         uint32_t tests, isects;
-        trace_ray<PRUNE, COUNT, FETCH>(sc, V3{ro.x, ro.y, ro.z}, V3{rd.x, rd.y, rd.z}, st, h, tests, isects,
-                                       overflow);
+        trace_ray<COUNT>(sc, V3{ro.x, ro.y, ro.z}, V3{rd.x, rd.y, rd.z}, st, h, tests, isects, overflow);
         hits[i] = make_uint2(__float_as_uint(h.t), h.prim);
-        if (COUNT || FETCH) {
+        if (COUNT) {
             if (tests_out) tests_out[i] = tests;
             if (isects_out) isects_out[i] = isects;
         }
@@ -34,27 +34,30 @@ __global__ __launch_bounds__(kBlock) void k_trace(DevScene sc, const float4* __r
     if (overflow) atomicOr(flags, 1u);
 }
 
-// Persistent closest-hit kernel: rays[i] -> hits[i] (FETCH: per-ray node and
-// triangle record counts into nodes_out / tris_out).
+// Scene-order id of the primitive at a leaf-order index.
+__device__ inline uint32_t prim_of(const DevScene& sc, uint32_t idx) {
+    return idx == kNoHit ? SPT_MISS : __float_as_uint(sc.tris[3 * (size_t)idx + 2].y);
+}
+
+// Closest-hit kernel: rays[i] -> hits[i] (FETCH: per-ray node and triangle
+// record counts into nodes_out / tris_out).
 template <bool FETCH>
-__global__ __launch_bounds__(kBlock) void k_trace_p(DevScene sc, const float4* __restrict__ rays, uint32_t n,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_trace_q(DevScene sc, const float4* __restrict__ rays, uint32_t n,
                                                     uint2* __restrict__ hits, uint32_t* __restrict__ nodes_out,
                                                     uint32_t* __restrict__ tris_out, uint32_t* __restrict__ spill,
-                                                    uint32_t* __restrict__ flags, uint32_t refill) {
-    __shared__ uint32_t lds[kLdsStack * kBlock];
-    const uint32_t gthreads = gridDim.x * kBlock;
-    const uint32_t gtid = blockIdx.x * kBlock + threadIdx.x;
-    Stack st(lds + threadIdx.x, spill + gtid, gthreads, sc.stack_cap4);
+                                                    uint32_t* __restrict__ flags, uint32_t* __restrict__ rays_taken,
+                                                    uint32_t refill) {
+    __shared__ QuadLds lds;
     bool overflow = false;
-    trace_persistent<FETCH>(
-        sc, n, flags + 8, st, overflow, refill,
+    trace_quads<FETCH>(
+        sc, n, rays_taken, lds, spill + (size_t)blockIdx.x * quad_spill_words(sc.stack_cap4), overflow, refill,
         [&](uint32_t i, V3& o, V3& d, Root&) {
             const float4 ro = rays[2 * (size_t)i], rd = rays[2 * (size_t)i + 1];
             o = V3{ro.x, ro.y, ro.z};
             d = V3{rd.x, rd.y, rd.z};
         },
-        [&](uint32_t i, const Hit& h, uint32_t nn, uint32_t nt) {
-            hits[i] = make_uint2(__float_as_uint(h.t), h.prim);
+        [&](uint32_t i, const Hit& h, V3, V3, uint32_t nn, uint32_t nt) {
+            hits[i] = make_uint2(__float_as_uint(h.t), prim_of(sc, h.idx));
             if (FETCH) {
                 nodes_out[i] = nn;
                 tris_out[i] = nt;
@@ -63,12 +66,42 @@ __global__ __launch_bounds__(kBlock) void k_trace_p(DevScene sc, const float4* _
     if (overflow) atomicOr(flags, 1u);
 }
 
-// One ray per pixel centre (RegularPixelSampler(1) gives (0.5, 0.5),
-// regular_pixel_sampler.cpp:3-14); value per normal_raycaster.cpp:19-31,
-// depth_raycaster.cpp:36-48, int_test_count_raycaster.cpp:75-85.
+// Camera ray of pixel i: one ray per pixel centre (RegularPixelSampler(1)
+// gives (0.5, 0.5), regular_pixel_sampler.cpp:3-14).
+__device__ inline void pixel_ray(const DevCamera& cam, uint64_t i, V3& o, V3& d) {
+    const uint32_t x = (uint32_t)(i % cam.width), y = (uint32_t)(i / cam.width);
+    camera_ray(cam, x + 0.5f, y + 0.5f, o, d);
+}
+
+// Normal (normal_raycaster.cpp:19-31) and depth (depth_raycaster.cpp:36-48)
+// ray casters over pixels [base, base + n).
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_raycast(DevScene sc, DevCamera cam, void* __restrict__ out,
-                                                    uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_raycast(DevScene sc, DevCamera cam, uint64_t base, uint32_t n,
+                                                    float* __restrict__ out, uint32_t* __restrict__ spill,
+                                                    uint32_t* __restrict__ flags, uint32_t* __restrict__ rays_taken,
+                                                    uint32_t refill) {
+    __shared__ QuadLds lds;
+    bool overflow = false;
+    trace_quads<false>(
+        sc, n, rays_taken, lds, spill + (size_t)blockIdx.x * quad_spill_words(sc.stack_cap4), overflow, refill,
+        [&](uint32_t i, V3& o, V3& d, Root&) { pixel_ray(cam, base + i, o, d); },
+        [&](uint32_t i, const Hit& h, V3 o, V3 d, uint32_t, uint32_t) {
+            if (KIND == SPT_RAYCAST_DEPTH) {
+                out[base + i] = (h.idx != kNoHit) ? h.t : -1.0f;
+            } else {
+                const V3 nrm = (h.idx != kNoHit) ? shading_normal(sc, h, o + d * h.t) : V3{0.0f, 0.0f, 0.0f};
+                float* o3 = out + 3 * (base + i);
+                o3[0] = nrm.x;
+                o3[1] = nrm.y;
+                o3[2] = nrm.z;
+            }
+        });
+    if (overflow) atomicOr(flags, 1u);
+}
+
+// Intersection-test count ray caster (int_test_count_raycaster.cpp:75-85).
+__global__ __launch_bounds__(kBlock) void k_raycast_count(DevScene sc, DevCamera cam, uint32_t* __restrict__ out,
+                                                          uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
     __shared__ uint32_t lds[kLdsStack * kBlock];
     const uint32_t gthreads = gridDim.x * kBlock;
     const uint32_t gtid = blockIdx.x * kBlock + threadIdx.x;
@@ -76,26 +109,12 @@ __global__ __launch_bounds__(kBlock) void k_raycast(DevScene sc, DevCamera cam, 
     bool overflow = false;
     const uint64_t n = (uint64_t)cam.width * cam.height;
     for (uint64_t i = gtid; i < n; i += gthreads) {
-        const uint32_t x = (uint32_t)(i % cam.width), y = (uint32_t)(i / cam.width);
         V3 o, d;
-        camera_ray(cam, x + 0.5f, y + 0.5f, o, d);
+        pixel_ray(cam, i, o, d);
         Hit h;
         uint32_t tests, isects;
-        if (KIND == SPT_RAYCAST_COUNT) {
-            trace_ray<false, true>(sc, o, d, st, h, tests, isects, overflow);
-            reinterpret_cast<uint32_t*>(out)[i] = tests;
-        } else {
-            trace_ray<true, false>(sc, o, d, st, h, tests, isects, overflow);
-            if (KIND == SPT_RAYCAST_DEPTH) {
-                reinterpret_cast<float*>(out)[i] = (h.idx != kNoHit) ? h.t : -1.0f;
-            } else {
-                V3 nrm = (h.idx != kNoHit) ? shading_normal(sc, h, o + d * h.t) : V3{0.0f, 0.0f, 0.0f};
-                float* o3 = reinterpret_cast<float*>(out) + 3 * i;
-                o3[0] = nrm.x;
-                o3[1] = nrm.y;
-                o3[2] = nrm.z;
-            }
-        }
+        trace_ray<true>(sc, o, d, st, h, tests, isects, overflow);
+        out[i] = tests;
     }
     if (overflow) atomicOr(flags, 1u);
 }
@@ -104,23 +123,21 @@ __global__ __launch_bounds__(kBlock) void k_camera_rays(DevCamera cam, float4* _
     const uint64_t n = (uint64_t)cam.width * cam.height;
     const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    const uint32_t x = (uint32_t)(i % cam.width), y = (uint32_t)(i / cam.width);
     V3 o, d;
-    camera_ray(cam, x + 0.5f, y + 0.5f, o, d);
+    pixel_ray(cam, i, o, d);
     rays[2 * i] = make_float4(o.x, o.y, o.z, 0.0f);
     rays[2 * i + 1] = make_float4(d.x, d.y, d.z, 0.0f);
 }
 
 // Scratch of the allocation-free closest-hit entry point
-// (spt_trace_noalloc): words [0, 16) hold the overflow flag (word 0) and the
-// persistent kernel's ray counter (word 8), words [64, ...) the traversal
-// stacks' spill area. Each device holds its own copy; host code reaches it
+// (spt_trace_noalloc): word 0 holds the overflow flag, then come the
+// traversal's ray counters and the traversal stacks' spill area. Each device holds its own copy; host code reaches it
 // only through the address hipGetSymbolAddress returns for that device.
 static __device__ __align__(256) uint32_t scratch[SPT_NOALLOC_SCRATCH_WORDS];
-constexpr uint32_t kScratchSpill = 64;
+constexpr uint32_t kScratchRays = 64, kScratchSpill = kScratchRays + kRayCounterWords;
 
 __global__ void k_scratch_reset(uint32_t* __restrict__ ctl) {
-    if (threadIdx.x < kScratchSpill) ctl[threadIdx.x] = 0u;
+    ctl[threadIdx.x] = 0u;
 }
 
 __global__ void k_scratch_fold_overflow(const uint32_t* __restrict__ ctl, uint32_t* __restrict__ ctx_flags) {
@@ -137,58 +154,79 @@ uint32_t grid_for(const spt_ctx* ctx, uint64_t n) {
 
 }  // namespace
 
-uint32_t persistent_grid(spt_ctx* ctx, const void* kernel) {
+namespace {
+
+// Idle lanes of a wave that make it take new rays (spt_tuning.refill_lanes).
+uint32_t refill_of(const spt_ctx* ctx) {
+    const uint32_t want = ctx->tuning.refill_lanes ? ctx->tuning.refill_lanes : kRefillLanes;
+    return std::min<uint32_t>(kMaxRefillLanes, std::max<uint32_t>(1, want));
+}
+
+// Grid of a quad kernel over n rays: what the chip holds at once, or a block
+// per 16 rays when that is fewer (a wave takes at least 4).
+uint32_t quad_grid(spt_ctx* ctx, const void* kernel, uint64_t n) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess || per_cu <= 0)
         per_cu = 4;
-    return (uint32_t)(per_cu * ctx->num_cus);
+    return (uint32_t)std::min<uint64_t>((uint64_t)per_cu * ctx->num_cus, (n + 15) / 16);
 }
+
+constexpr uint64_t kMaxLaunchRays = 1ull << 31;  // rays of one launch (32-bit ray counter)
+
+// Launches `launch(base, n, grid)` over [0, total) with the ray counters
+// reset before each launch that uses them.
+template <typename Launch>
+spt_status quad_launches(spt_ctx* ctx, const void* kernel, uint64_t total, Launch launch, const char* what) {
+    for (uint64_t base = 0; base < total; base += kMaxLaunchRays) {
+        const uint32_t n = (uint32_t)std::min(kMaxLaunchRays, total - base);
+        const uint32_t grid = quad_grid(ctx, kernel, n);
+        spt_status s = ensure_spill(ctx, std::max<size_t>(1, (size_t)grid * quad_spill_words(ctx->stack_cap4)));
+        if (s != SPT_OK) return s;
+        if (RayShares(n, grid * (kBlock / 64)).fixed < n) {  // only larger launches use the counters
+            s = check_hip(ctx, hipMemsetAsync(ctx->d_rays, 0, kRayCounterWords * 4, ctx->stream), "ray counters");
+            if (s != SPT_OK) return s;
+        }
+        launch(base, n, grid);
+        s = check_hip(ctx, hipGetLastError(), what);
+        if (s != SPT_OK) return s;
+    }
+    return SPT_OK;
+}
+
+}  // namespace
 
 spt_status launch_trace(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t n, spt_hit* d_hits, uint32_t mode,
                         uint32_t* d_tests, uint32_t* d_isects) {
     if (n == 0) return SPT_OK;
-    if ((mode == SPT_TRACE_CLOSEST || mode == SPT_TRACE_FETCH) && n < 0xFFFFFF00ull) {
-        const void* kern = (mode == SPT_TRACE_FETCH) ? reinterpret_cast<const void*>(&k_trace_p<true>)
-                                                    : reinterpret_cast<const void*>(&k_trace_p<false>);
-        const uint32_t grid = persistent_grid(ctx, kern);
-        spt_status s =
-            ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap4 > kLdsStack ? ctx->stack_cap4 - kLdsStack : 1));
-        if (s != SPT_OK) return s;
-        s = check_hip(ctx, hipMemsetAsync(ctx->d_flags + 8, 0, 4, ctx->stream), "ray counter");
-        if (s != SPT_OK) return s;
-        DevScene sc = ctx->scene();
-        const float4* rays = reinterpret_cast<const float4*>(d_rays);
-        uint2* hits = reinterpret_cast<uint2*>(d_hits);
-        // incoherent ray batches prefer eager refills (16 idle lanes); the path
-        // tracer's default (48) is for its extension rays
-        const uint32_t want = ctx->tuning.refill_lanes ? ctx->tuning.refill_lanes : 16u;
-        const uint32_t refill = std::min<uint32_t>(64, std::max<uint32_t>(1, want));
-        if (mode == SPT_TRACE_FETCH)
-            hipLaunchKernelGGL(k_trace_p<true>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, (uint32_t)n, hits,
-                               d_tests, d_isects, ctx->d_spill, ctx->d_flags, refill);
-        else
-            hipLaunchKernelGGL(k_trace_p<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, (uint32_t)n,
-                               hits, nullptr, nullptr, ctx->d_spill, ctx->d_flags, refill);
-        return check_hip(ctx, hipGetLastError(), "trace launch");
-    }
-    const uint32_t grid = grid_for(ctx, n);
-    spt_status s = ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap > kLdsStack ? ctx->stack_cap - kLdsStack : 1));
-    if (s != SPT_OK) return s;
     DevScene sc = ctx->scene();
     const float4* rays = reinterpret_cast<const float4*>(d_rays);
     uint2* hits = reinterpret_cast<uint2*>(d_hits);
     if (mode == SPT_TRACE_CLOSEST)
-        hipLaunchKernelGGL((k_trace<true, false, false>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n,
-                           hits, nullptr, nullptr, ctx->d_spill, ctx->d_flags);
-    else if (mode == SPT_TRACE_COUNT)
-        hipLaunchKernelGGL((k_trace<false, true, false>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n,
-                           hits, d_tests, d_isects, ctx->d_spill, ctx->d_flags);
-    else if (mode == SPT_TRACE_FETCH)
-        hipLaunchKernelGGL((k_trace<true, false, true>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n,
-                           hits, d_tests, d_isects, ctx->d_spill, ctx->d_flags);
+        return quad_launches(
+            ctx, reinterpret_cast<const void*>(&k_trace_q<false>), n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL(k_trace_q<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
+                                   hits + base, nullptr, nullptr, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
+            },
+            "trace launch");
+    if (mode == SPT_TRACE_FETCH)
+        return quad_launches(
+            ctx, reinterpret_cast<const void*>(&k_trace_q<true>), n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL(k_trace_q<true>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
+                                   hits + base, d_tests + base, d_isects + base, ctx->d_spill, ctx->d_flags,
+                                   ctx->d_rays, refill_of(ctx));
+            },
+            "trace launch");
+    const uint32_t grid = grid_for(ctx, n);
+    spt_status s = ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap > kLdsStack ? ctx->stack_cap - kLdsStack : 1));
+    if (s != SPT_OK) return s;
+    if (mode == SPT_TRACE_COUNT)
+        hipLaunchKernelGGL((k_trace<true>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n, hits, d_tests,
+                           d_isects, ctx->d_spill, ctx->d_flags);
     else
-        hipLaunchKernelGGL((k_trace<false, false, false>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n,
-                           hits, nullptr, nullptr, ctx->d_spill, ctx->d_flags);
+        hipLaunchKernelGGL((k_trace<false>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays, n, hits, nullptr,
+                           nullptr, ctx->d_spill, ctx->d_flags);
     return check_hip(ctx, hipGetLastError(), "trace launch");
 }
 
@@ -225,25 +263,27 @@ spt_status launch_trace_noalloc(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t 
         return set_error(ctx, SPT_ERR_INVALID, "spt_trace_noalloc: more than SPT_NOALLOC_MAX_RAYS rays");
     if (!ctx->scratch) return set_error(ctx, SPT_ERR_STATE, "spt_trace_noalloc: no static scratch on this device");
     if (n == 0) return SPT_OK;
-    const void* kern = reinterpret_cast<const void*>(&k_trace_p<false>);
-    // spill words per lane: the stack entries beyond the LDS part
-    const uint64_t per_lane = ctx->stack_cap4 > kLdsStack ? ctx->stack_cap4 - kLdsStack : 1;
+    const void* kern = reinterpret_cast<const void*>(&k_trace_q<false>);
+    // blocks whose stack entries beyond the LDS part fit the scratch
+    const uint64_t per_block = quad_spill_words(ctx->stack_cap4);
     const uint64_t room = (uint64_t)SPT_NOALLOC_SCRATCH_WORDS - kScratchSpill;
-    const uint64_t max_blocks = room / (per_lane * kBlock);
+    const uint64_t max_blocks = per_block ? room / per_block : ~0ull;
     if (max_blocks == 0)
         return set_error(ctx, SPT_ERR_UNSUPPORTED, "spt_trace_noalloc: the tree is too deep for the static scratch");
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(persistent_grid(ctx, kern), max_blocks);
     uint32_t* ctl = ctx->scratch;
     uint32_t* spill = ctx->scratch + kScratchSpill;
-    // a fill kernel, not a memset node: callers may capture this in a graph
-    hipLaunchKernelGGL(k_scratch_reset, dim3(1), dim3(kScratchSpill), 0, ctx->stream, ctl);
-    const uint32_t want = ctx->tuning.refill_lanes ? ctx->tuning.refill_lanes : 16u;
-    const uint32_t refill = std::min<uint32_t>(64, std::max<uint32_t>(1, want));
-    hipLaunchKernelGGL(k_trace_p<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->scene(),
-                       reinterpret_cast<const float4*>(d_rays), (uint32_t)n, reinterpret_cast<uint2*>(d_hits), nullptr,
-                       nullptr, spill, ctl, refill);
-    // a stack overflow is reported by spt_sync, as for spt_trace
-    hipLaunchKernelGGL(k_scratch_fold_overflow, dim3(1), dim3(64), 0, ctx->stream, ctl, ctx->d_flags);
+    const float4* rays = reinterpret_cast<const float4*>(d_rays);
+    uint2* hits = reinterpret_cast<uint2*>(d_hits);
+    for (uint64_t base = 0; base < n; base += kMaxLaunchRays) {
+        const uint32_t cnt = (uint32_t)std::min(kMaxLaunchRays, n - base);
+        const uint32_t grid = (uint32_t)std::min<uint64_t>(quad_grid(ctx, kern, cnt), max_blocks);
+        // a fill kernel, not a memset node: callers may capture this in a graph
+        hipLaunchKernelGGL(k_scratch_reset, dim3(1), dim3(kScratchSpill), 0, ctx->stream, ctl);
+        hipLaunchKernelGGL(k_trace_q<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->scene(), rays + 2 * base,
+                           cnt, hits + base, nullptr, nullptr, spill, ctl, ctl + kScratchRays, refill_of(ctx));
+        // a stack overflow is reported by spt_sync, as for spt_trace
+        hipLaunchKernelGGL(k_scratch_fold_overflow, dim3(1), dim3(64), 0, ctx->stream, ctl, ctx->d_flags);
+    }
     return check_hip(ctx, hipGetLastError(), "trace (no allocation) launch");
 }
 
@@ -258,20 +298,30 @@ spt_status launch_camera_rays(spt_ctx* ctx, const spt_camera* cam, spt_ray32* d_
 spt_status launch_raycast(spt_ctx* ctx, const spt_camera* cam, uint32_t kind, void* d_out) {
     const uint64_t n = (uint64_t)cam->width * cam->height;
     if (n == 0) return SPT_OK;
+    DevScene sc = ctx->scene();
+    DevCamera dc = make_camera(*cam);
+    float* out = reinterpret_cast<float*>(d_out);
+    if (kind == SPT_RAYCAST_NORMAL)
+        return quad_launches(
+            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_NORMAL>), n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_NORMAL>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
+                                   base, cnt, out, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
+            },
+            "raycast launch");
+    if (kind == SPT_RAYCAST_DEPTH)
+        return quad_launches(
+            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_DEPTH>), n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_DEPTH>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
+                                   base, cnt, out, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
+            },
+            "raycast launch");
     const uint32_t grid = grid_for(ctx, n);
     spt_status s = ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap > kLdsStack ? ctx->stack_cap - kLdsStack : 1));
     if (s != SPT_OK) return s;
-    DevScene sc = ctx->scene();
-    DevCamera dc = make_camera(*cam);
-    if (kind == SPT_RAYCAST_NORMAL)
-        hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_NORMAL>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, d_out,
-                           ctx->d_spill, ctx->d_flags);
-    else if (kind == SPT_RAYCAST_DEPTH)
-        hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_DEPTH>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, d_out,
-                           ctx->d_spill, ctx->d_flags);
-    else
-        hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_COUNT>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, d_out,
-                           ctx->d_spill, ctx->d_flags);
+    hipLaunchKernelGGL(k_raycast_count, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
+                       reinterpret_cast<uint32_t*>(d_out), ctx->d_spill, ctx->d_flags);
     return check_hip(ctx, hipGetLastError(), "raycast launch");
 }
 
