@@ -383,10 +383,10 @@ typedef struct spt_tuning {
                                       lanes (four per ray) are idle; more than 24 act as 24
                                       (default in path tracing 48 on one wavefront, 20 with
                                       several; 20 in spt_trace) */
-    uint32_t wavefronts;           /* unguided renders: independent wavefronts run at once on
-                                      their own streams, each with a share of the paths and of
-                                      the queue capacity, so one's traversal overlaps another's
-                                      shading (1..4, default 3) */
+    uint32_t wavefronts;           /* independent wavefronts run at once on their own streams, each
+                                      with a share of the paths and of the queue capacity, so
+                                      one's traversal overlaps another's shading (1..4, default 3;
+                                      left at the default, a plain render of one scene uses one) */
 } spt_tuning;
 spt_status spt_set_tuning(spt_ctx* ctx, const spt_tuning* t);
 spt_status spt_get_tuning(spt_ctx* ctx, spt_tuning* t);

@@ -224,27 +224,6 @@ __device__ inline V3 shading_normal(const DevScene& sc, const Hit& h, V3 pos) {
     return normalize(n0 * (1.0f - h.u - h.v) + n1 * h.u + n2 * h.v);
 }
 
-// Wave-aggregated counter increment: lanes of the wave that carry the same
-// key share one global atomicAdd (one per distinct key per wave instead of one
-// per lane); returns this lane's slot (old value + rank among equal keys).
-// Must be called by every active lane of the wave together.
-__device__ inline uint32_t wave_add(uint32_t* counters, uint32_t key) {
-    uint64_t todo = __ballot(1);
-    const uint64_t lt = __lanemask_lt();
-    uint32_t slot = 0;
-    while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const uint32_t lkey = __shfl(key, leader);
-        const uint64_t group = __ballot(key == lkey) & todo;
-        uint32_t base = 0;
-        if (__lane_id() == (unsigned)leader) base = atomicAdd(&counters[lkey], (uint32_t)__popcll(group));
-        base = __shfl(base, leader);
-        if (key == lkey) slot = base + (uint32_t)__popcll(group & lt);
-        todo &= ~group;
-    }
-    return slot;
-}
-
 // One scene's share of a render call: camera, sampling, termination,
 // outputs and where its tree starts in the (shared) node/triangle arrays.
 struct Job {

@@ -59,6 +59,7 @@ struct RenderArgs {
     const BatchTile* tiles;     // multi-scene call: generation order
     const uint64_t* tile_start; // first path of each tile (n_tiles + 1 entries)
     uint32_t n_tiles;
+    uint32_t n_jobs;
     uint32_t* job_done;         // paths finished per job
     uint64_t* job_clock;        // [0] start, [1 + j] finish of job j (device wall clock)
     uint32_t flags;
@@ -117,15 +118,26 @@ __device__ inline const Job& job_of(const RenderArgs& a, uint32_t j) {
     return a.job;
 }
 
-// Film and per-path output of a finished path; in a multi-scene call also
-// counts the job's finished paths and stamps the job's finish time when its
-// last path ends. Called by every active lane of the branch together.
+// Adds finished paths to a job's count and stamps the job's finish time when
+// its last path is counted.
+__device__ inline void count_done(const RenderArgs& a, uint32_t jid, uint32_t n) {
+    const uint32_t k = atomicAdd(&a.job_done[jid], n);
+    if ((uint64_t)k + n == a.jobs[jid].n_paths) a.job_clock[1 + jid] = wall_clock64();
+}
+
+// Film and per-path output of a finished path. A multi-scene call also counts
+// the job's finished paths: in the block's LDS counters (`done`, added to the
+// job's at the block's end: one global atomic per block and job instead of one
+// per wave, whose addresses all XCDs share) when the jobs fit them.
+constexpr uint32_t kDoneJobs = 512;
 template <bool MULTI>
 __device__ inline void finish_path(const RenderArgs& a, const Job& jb, uint32_t jid, uint32_t pix, uint64_t local,
-                                   float4 L) {
+                                   float4 L, uint32_t* done) {
     if (MULTI) {
-        const uint32_t k = wave_add(a.job_done, jid);
-        if ((uint64_t)k + 1 == jb.n_paths) a.job_clock[1 + jid] = wall_clock64();
+        if (a.n_jobs <= kDoneJobs)
+            atomicAdd(&done[jid], 1u);
+        else
+            count_done(a, jid, 1u);
     }
     if (jb.film32) {
         float* f = jb.film32 + 3 * (size_t)pix;
@@ -209,7 +221,7 @@ __device__ inline void gen_path(const RenderArgs& a, PathBuf& A, const Work& w, 
     camera_ray(jb.cam, xs, ys, o, d);
     if (r.overflow) atomicAdd(&w.cnt[2], 1u);
     if (jb.max_depth == 0) {  // depth >= path_length before the first trace
-        finish_path<MULTI>(a, jb, jid, pix, local, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+        finish_path<MULTI>(a, jb, jid, pix, local, make_float4(0.0f, 0.0f, 0.0f, 0.0f), nullptr);
         return;
     }
     A.o[s] = make_float4(o.x, o.y, o.z, __uint_as_float(pix));
@@ -634,8 +646,200 @@ __device__ inline void layered_eval_guided(const spt_material& m, V3 wo, const F
     }
 }
 
+// What a path that goes on carries into the next bounce.
+struct Survivor {
+    float4 o, d, thr, rad;
+    uint64_t key, local;
+    uint4 gr;
+};
+
+template <bool GUIDED>
+__device__ inline void store_survivor(const RenderArgs& a, const PathBuf& B, const Survivor& sv, uint32_t slot) {
+    B.o[slot] = sv.o;
+    B.d[slot] = sv.d;
+    B.thr[slot] = sv.thr;
+    B.rad[slot] = sv.rad;
+    B.key[slot] = sv.key;
+    if (a.per_path) B.local[slot] = sv.local;
+    if (GUIDED && a.train) B.grec[slot] = sv.gr;
+}
+
+// Shading of one vertex (integrators/pathtracer.cpp:21-54) of path j in
+// shading order; go_on(survivor) is called for a path that does not end here.
+template <bool MULTI, bool GUIDED, typename GoOn>
+__device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const Work& w, const spt_material* smats,
+                                  bool lds_mats, uint32_t j, uint32_t* done, GoOn go_on) {
+    const uint32_t i = a.keys ? w.perm[j] : j;
+    const float4 hv = w.hit[i];
+    float4 rad = A.rad[i];
+    const float4 thr = A.thr[i];
+    const float4 o4 = A.o[i], d4 = A.d[i];
+    const uint32_t pix = __float_as_uint(o4.w), jid = __float_as_uint(d4.w);
+    const Job& jb = job_of<MULTI>(a, jid);
+    const uint32_t depth = __float_as_uint(rad.w);
+    const uint32_t idx = __float_as_uint(hv.y);
+    if (idx == kNoHit) {  // miss: background at depth 0, else 0 (pathtracer.cpp:21-26)
+        if (depth == 0) {
+            rad.x += thr.x * jb.bg[0];
+            rad.y += thr.y * jb.bg[1];
+            rad.z += thr.z * jb.bg[2];
+        }
+        if (GUIDED && a.train) finish_records(a, A.grec[i], rad, A.key[i]);
+        finish_path<MULTI>(a, jb, jid, pix, a.per_path ? A.local[i] : 0ull, rad, done);
+        return;
+    }
+    const V3 o{o4.x, o4.y, o4.z}, d{d4.x, d4.y, d4.z};
+    Hit h;
+    h.t = hv.x;
+    h.idx = idx;
+    h.u = hv.z;
+    h.v = hv.w;
+    const V3 pos = o + d * h.t;  // triangle.cpp:69
+    const V3 nrm = shading_normal(a.sc, h, pos);
+    const uint32_t mid = w.skey[i];
+    const spt_material& m = lds_mats ? smats[mid] : a.sc.mats[mid];
+    const Frame fr = frame_from_up(nrm);          // pathtracer.cpp:28
+    const V3 wo = normalize(to_local(fr, -d));    // pathtracer.cpp:30
+    const uint64_t key = A.key[i];
+    Draws r = make_draws(jb, key, __float_as_uint(thr.w));
+    V3 bsdf, refl, wi;
+    float pdf;
+    const uint32_t gmode = GUIDED ? guide_mode(a, mid) : 0u;
+    const bool prod = GUIDED && (a.gflags & SPT_GUIDE_PRODUCT);
+    const bool guided = gmode != 0u;
+    bool via = true;  // the sampled direction came from a guided step
+    float pmarg = 0.0f;  // PRODUCT: density of wi, the training weight's 1/p
+    if (gmode == kGuideCoated) {
+        // with PRODUCT: the learned incident radiance times the coated
+        // lobe in exit space
+        using namespace guide;
+        Lobe lobes[kLobes];
+        mixture_params(HalfRow{a.gout + (size_t)i * kOut}, lobes);
+        V3 mb;
+        float kb;
+        bsdf_lobe(m.layers[1], wo, m.layers[0].ior, mb, kb);
+        const V3 mbw = to_world(fr, mb);
+        if (prod) mixture_product(lobes, mbw, kb);
+        layered_eval_guided(m, wo, fr, lobes, a.bsdf_frac, bsdf, refl, pdf, wi, r, via);
+        if (prod && a.train && via && wi.y > 0.0f) {  // exit density, the lobe standing in for the walk
+            const V3 e = to_world(fr, wi);
+            Lobe bl;
+            bl.mu = mbw;
+            bl.kappa = kb;
+            pmarg = a.bsdf_frac * expf(log_vmf(bl, e)) + (1.0f - a.bsdf_frac) * mixture_pdf(lobes, e);
+        }
+    } else if (guided) {
+        // one-sample mixture of the layer's sampler and the learned
+        // incident radiance times a vMF stand-in of the layer's lobe
+        using namespace guide;
+        const spt_layer& l = m.layers[0];
+        Lobe lobes[kLobes];
+        mixture_params(HalfRow{a.gout + (size_t)i * kOut}, lobes);
+        if (prod) {
+            V3 mb;
+            float kb;
+            bsdf_lobe(l, wo, 1.0f, mb, kb);
+            mixture_product(lobes, to_world(fr, mb), kb);
+        }
+        if (r.next() < a.bsdf_frac) {
+            wi = layer_sample(l, wo, r).wi;
+        } else {
+            const float u0 = r.next(), u1 = r.next(), u2 = r.next();
+            wi = to_local(fr, mixture_sample(lobes, u0, u1, u2));
+        }
+        pdf = a.bsdf_frac * layer_density(l, wo, wi) +
+              (1.0f - a.bsdf_frac) * mixture_pdf(lobes, to_world(fr, wi));
+        pmarg = pdf;
+        if (wi.y > 0.0f && pdf > 0.0f) {
+            bsdf = layer_f(l, wo, wi);
+            refl = layer_reflectance(l, wo, wi);
+        } else {
+            bsdf = V3{0.0f, 0.0f, 0.0f};
+            refl = V3{0.0f, 0.0f, 0.0f};
+            pdf = 1.0f;
+        }
+    } else {
+        layered_eval(m, wo, bsdf, refl, pdf, wi, r);  // pathtracer.cpp:36
+    }
+    const V3 wwi = to_world(fr, wi);              // pathtracer.cpp:37
+    const V3 no = pos + wwi * 1e-3f;              // pathtracer.cpp:38
+    rad.x += thr.x * m.emission[0];
+    rad.y += thr.y * m.emission[1];
+    rad.z += thr.z * m.emission[2];
+    const float kk = gmax(gmax(refl.x, refl.y), refl.z);  // pathtracer.cpp:41
+    // training weight before roulette: L_i / p (PRODUCT, radiance target)
+    // or f cos / p L_i (the product target)
+    const float rec_w = prod ? ((pmarg > 0.0f) ? 1.0f / pmarg : 0.0f) : lum(bsdf) * wi.y / pdf;
+    bool alive = true;
+    if ((jb.rr_depth >= 0) && ((int32_t)depth >= jb.rr_depth)) {  // pathtracer.cpp:43-49
+        if ((r.next() < kk) && (depth < 1000u))
+            bsdf = bsdf / kk;
+        else
+            alive = false;
+    }
+    if (r.overflow) atomicAdd(&w.cnt[2], 1u);
+    const uint32_t nd = depth + 1;
+    if (alive && (jb.max_depth >= 0) && ((int32_t)nd >= jb.max_depth)) alive = false;  // pathtracer.cpp:18
+    if (!alive) {
+        if (GUIDED && a.train) finish_records(a, A.grec[i], rad, A.key[i]);
+        finish_path<MULTI>(a, jb, jid, pix, a.per_path ? A.local[i] : 0ull, rad, done);
+        return;
+    }
+    // pathtracer.cpp:52-54, forwards: throughput *= f * cos / pdf
+    const V3 wgt = (bsdf * wi.y) / pdf;
+    uint4 gr = (GUIDED && a.train) ? A.grec[i] : make_uint4(0u, 0u, 0u, 0u);
+    const bool cand = GUIDED && a.train && guided && via && gr.w < 3u && wi.y > 0.0f && bsdf.x + bsdf.y + bsdf.z > 0.0f;
+    const bool take = cand && (a.rec_stride <= 1u ||
+                               mix64(key + (uint64_t)(depth + 1) * 0x9E3779B97F4A7C15ull) % a.rec_stride == 0u);
+    uint32_t rs = 0;
+    if (GUIDED && a.train) {
+        // one 64-bit atomic per wave adds the wave's candidates (high
+        // word) and records (low word); the record slots of the wave are
+        // consecutive from the old low word
+        const uint64_t cb = __ballot(cand), tb = __ballot(take);
+        const int leader = __ffsll((unsigned long long)cb) - 1;
+        const unsigned long long inc = ((unsigned long long)__popcll(cb) << 32) | (unsigned long long)__popcll(tb);
+        unsigned long long* rc = reinterpret_cast<unsigned long long*>(a.rec_count);
+        if (tb) {
+            unsigned long long old = 0;
+            if (__lane_id() == (unsigned)leader) old = atomicAdd(rc, inc);
+            rs = __shfl((uint32_t)old, leader) + (uint32_t)__popcll(tb & __lanemask_lt());
+        } else if (cb && __lane_id() == (unsigned)leader) {
+            atomicAdd(rc, inc);
+        }
+    }
+    if (take) {
+        if (a.rec_ring) rs %= a.rec_cap;
+        if (rs < a.rec_cap) {
+            float* rec = a.records + (size_t)rs * guide::kRecord;
+            rec[20] = __uint_as_float(rec_tag(key, gr.w));
+            const V3 wdir = to_world(fr, wi);
+            const float vals[20] = {pos.x, pos.y, pos.z, nrm.x, nrm.y, nrm.z, -d.x, -d.y, -d.z, wdir.x, wdir.y,
+                                    wdir.z, 0.0f, rec_w, rad.x, rad.y, rad.z,
+                                    thr.x * wgt.x, thr.y * wgt.y, thr.z * wgt.z};
+            for (int k = 0; k < 20; ++k) rec[k] = vals[k];
+            if (gr.w == 0) gr.x = rs;
+            else if (gr.w == 1) gr.y = rs;
+            else gr.z = rs;
+            ++gr.w;
+        }
+    }
+    Survivor sv;
+    sv.o = make_float4(no.x, no.y, no.z, __uint_as_float(pix));
+    sv.d = make_float4(wwi.x, wwi.y, wwi.z, __uint_as_float(jid));
+    sv.thr = make_float4(thr.x * wgt.x, thr.y * wgt.y, thr.z * wgt.z, __uint_as_float(r.k));
+    sv.rad = make_float4(rad.x, rad.y, rad.z, __uint_as_float(nd));
+    sv.key = key;
+    if (a.per_path) sv.local = A.local[i];
+    if (GUIDED && a.train) sv.gr = gr;
+    go_on(sv);
+}
+
 // Shading of one bounce (integrators/pathtracer.cpp:21-54) for every live
-// path of A, in material order when sorted; survivors are appended to B.
+// path of A, in material order when sorted; survivors are appended to B, with
+// one atomic on B's count per block and 256 paths: one per wave (the
+// compiler's aggregation) made that address the limit, about 10 ns per atomic
+// that all XCDs share (61M paths: 950k atomics in a 10.2-ms launch).
 // GUIDED instantiates the guide's sampling and record capture; the plain
 // instantiation carries none of their registers. Four waves per SIMD (128
 // VGPRs, a few spills) measured 2% faster than the two the register count
@@ -653,176 +857,54 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         uint32_t* dst = reinterpret_cast<uint32_t*>(smats);
         for (uint32_t k = threadIdx.x; k < words; k += kBlock) dst[k] = src[k];
     }
+    __shared__ uint32_t done[MULTI ? kDoneJobs : 1];  // finished paths of the block per job
+    if (MULTI)
+        for (uint32_t k = threadIdx.x; k < kDoneJobs; k += kBlock) done[k] = 0;
     __syncthreads();
+    // survivors of the block's four waves (two sets, used in turn) and their first slot
+    __shared__ uint32_t survivors[2][kBlock / 64 + 1];
     const uint32_t n = *cntA;
     const uint32_t gthreads = gridDim.x * kBlock;
-    for (uint32_t j = blockIdx.x * kBlock + threadIdx.x; j < n; j += gthreads) {
-        const uint32_t i = a.keys ? w.perm[j] : j;
-        const float4 hv = w.hit[i];
-        float4 rad = A.rad[i];
-        const float4 thr = A.thr[i];
-        const float4 o4 = A.o[i], d4 = A.d[i];
-        const uint32_t pix = __float_as_uint(o4.w), jid = __float_as_uint(d4.w);
-        const Job& jb = job_of<MULTI>(a, jid);
-        const uint32_t depth = __float_as_uint(rad.w);
-        const uint32_t idx = __float_as_uint(hv.y);
-        if (idx == kNoHit) {  // miss: background at depth 0, else 0 (pathtracer.cpp:21-26)
-            if (depth == 0) {
-                rad.x += thr.x * jb.bg[0];
-                rad.y += thr.y * jb.bg[1];
-                rad.z += thr.z * jb.bg[2];
-            }
-            if (GUIDED && a.train) finish_records(a, A.grec[i], rad, A.key[i]);
-            finish_path<MULTI>(a, jb, jid, pix, a.per_path ? A.local[i] : 0ull, rad);
+    const uint32_t wave = threadIdx.x / 64;
+    uint32_t turn = 0;
+    for (uint32_t j0 = blockIdx.x * kBlock; j0 < n; j0 += gthreads, turn ^= 1u) {
+        const uint32_t j = j0 + threadIdx.x;
+        if (GUIDED) {  // a slot per lane (per wave, as the compiler aggregates them): holding the survivors
+                       // across the barriers would spill 72 VGPRs instead of 22, which costs guided
+                       // passes as much as the shared address
+            if (j < n)
+                shade_path<MULTI, GUIDED>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& sv) {
+                    store_survivor<GUIDED>(a, B, sv, atomicAdd(cntB, 1u));
+                });
             continue;
         }
-        const V3 o{o4.x, o4.y, o4.z}, d{d4.x, d4.y, d4.z};
-        Hit h;
-        h.t = hv.x;
-        h.idx = idx;
-        h.u = hv.z;
-        h.v = hv.w;
-        const V3 pos = o + d * h.t;  // triangle.cpp:69
-        const V3 nrm = shading_normal(a.sc, h, pos);
-        const uint32_t mid = w.skey[i];
-        const spt_material& m = lds_mats ? smats[mid] : a.sc.mats[mid];
-        const Frame fr = frame_from_up(nrm);          // pathtracer.cpp:28
-        const V3 wo = normalize(to_local(fr, -d));    // pathtracer.cpp:30
-        const uint64_t key = A.key[i];
-        Draws r = make_draws(jb, key, __float_as_uint(thr.w));
-        V3 bsdf, refl, wi;
-        float pdf;
-        const uint32_t gmode = GUIDED ? guide_mode(a, mid) : 0u;
-        const bool prod = GUIDED && (a.gflags & SPT_GUIDE_PRODUCT);
-        const bool guided = gmode != 0u;
-        bool via = true;  // the sampled direction came from a guided step
-        float pmarg = 0.0f;  // PRODUCT: density of wi, the training weight's 1/p
-        if (gmode == kGuideCoated) {
-            // with PRODUCT: the learned incident radiance times the coated
-            // lobe in exit space
-            using namespace guide;
-            Lobe lobes[kLobes];
-            mixture_params(HalfRow{a.gout + (size_t)i * kOut}, lobes);
-            V3 mb;
-            float kb;
-            bsdf_lobe(m.layers[1], wo, m.layers[0].ior, mb, kb);
-            const V3 mbw = to_world(fr, mb);
-            if (prod) mixture_product(lobes, mbw, kb);
-            layered_eval_guided(m, wo, fr, lobes, a.bsdf_frac, bsdf, refl, pdf, wi, r, via);
-            if (prod && a.train && via && wi.y > 0.0f) {  // exit density, the lobe standing in for the walk
-                const V3 e = to_world(fr, wi);
-                Lobe bl;
-                bl.mu = mbw;
-                bl.kappa = kb;
-                pmarg = a.bsdf_frac * expf(log_vmf(bl, e)) + (1.0f - a.bsdf_frac) * mixture_pdf(lobes, e);
-            }
-        } else if (guided) {
-            // one-sample mixture of the layer's sampler and the learned
-            // incident radiance times a vMF stand-in of the layer's lobe
-            using namespace guide;
-            const spt_layer& l = m.layers[0];
-            Lobe lobes[kLobes];
-            mixture_params(HalfRow{a.gout + (size_t)i * kOut}, lobes);
-            if (prod) {
-                V3 mb;
-                float kb;
-                bsdf_lobe(l, wo, 1.0f, mb, kb);
-                mixture_product(lobes, to_world(fr, mb), kb);
-            }
-            if (r.next() < a.bsdf_frac) {
-                wi = layer_sample(l, wo, r).wi;
-            } else {
-                const float u0 = r.next(), u1 = r.next(), u2 = r.next();
-                wi = to_local(fr, mixture_sample(lobes, u0, u1, u2));
-            }
-            pdf = a.bsdf_frac * layer_density(l, wo, wi) +
-                  (1.0f - a.bsdf_frac) * mixture_pdf(lobes, to_world(fr, wi));
-            pmarg = pdf;
-            if (wi.y > 0.0f && pdf > 0.0f) {
-                bsdf = layer_f(l, wo, wi);
-                refl = layer_reflectance(l, wo, wi);
-            } else {
-                bsdf = V3{0.0f, 0.0f, 0.0f};
-                refl = V3{0.0f, 0.0f, 0.0f};
-                pdf = 1.0f;
-            }
-        } else {
-            layered_eval(m, wo, bsdf, refl, pdf, wi, r);  // pathtracer.cpp:36
+        Survivor sv;
+        bool alive = false;
+        if (j < n)
+            shade_path<MULTI, GUIDED>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& next) {
+                sv = next;
+                alive = true;
+            });
+        const uint64_t am = __ballot(alive);
+        if (__lane_id() == 0) survivors[turn][wave] = (uint32_t)__popcll(am);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t sum = 0;
+            for (uint32_t v = 0; v < kBlock / 64; ++v) sum += survivors[turn][v];
+            survivors[turn][kBlock / 64] = sum ? atomicAdd(cntB, sum) : 0u;
         }
-        const V3 wwi = to_world(fr, wi);              // pathtracer.cpp:37
-        const V3 no = pos + wwi * 1e-3f;              // pathtracer.cpp:38
-        rad.x += thr.x * m.emission[0];
-        rad.y += thr.y * m.emission[1];
-        rad.z += thr.z * m.emission[2];
-        const float kk = gmax(gmax(refl.x, refl.y), refl.z);  // pathtracer.cpp:41
-        // training weight before roulette: L_i / p (PRODUCT, radiance target)
-        // or f cos / p L_i (the product target)
-        const float rec_w = prod ? ((pmarg > 0.0f) ? 1.0f / pmarg : 0.0f) : lum(bsdf) * wi.y / pdf;
-        bool alive = true;
-        if ((jb.rr_depth >= 0) && ((int32_t)depth >= jb.rr_depth)) {  // pathtracer.cpp:43-49
-            if ((r.next() < kk) && (depth < 1000u))
-                bsdf = bsdf / kk;
-            else
-                alive = false;
-        }
-        if (r.overflow) atomicAdd(&w.cnt[2], 1u);
-        const uint32_t nd = depth + 1;
-        if (alive && (jb.max_depth >= 0) && ((int32_t)nd >= jb.max_depth)) alive = false;  // pathtracer.cpp:18
-        if (!alive) {
-            if (GUIDED && a.train) finish_records(a, A.grec[i], rad, A.key[i]);
-            finish_path<MULTI>(a, jb, jid, pix, a.per_path ? A.local[i] : 0ull, rad);
-            continue;
-        }
-        // pathtracer.cpp:52-54, forwards: throughput *= f * cos / pdf
-        const V3 wgt = (bsdf * wi.y) / pdf;
-        uint4 gr = (GUIDED && a.train) ? A.grec[i] : make_uint4(0u, 0u, 0u, 0u);
-        const bool cand = GUIDED && a.train && guided && via && gr.w < 3u && wi.y > 0.0f && bsdf.x + bsdf.y + bsdf.z > 0.0f;
-        const bool take = cand && (a.rec_stride <= 1u ||
-                                   mix64(key + (uint64_t)(depth + 1) * 0x9E3779B97F4A7C15ull) % a.rec_stride == 0u);
-        uint32_t rs = 0;
-        if (GUIDED && a.train) {
-            // one 64-bit atomic per wave adds the wave's candidates (high
-            // word) and records (low word); the record slots of the wave are
-            // consecutive from the old low word
-            const uint64_t cb = __ballot(cand), tb = __ballot(take);
-            const int leader = __ffsll((unsigned long long)cb) - 1;
-            const unsigned long long inc = ((unsigned long long)__popcll(cb) << 32) | (unsigned long long)__popcll(tb);
-            unsigned long long* rc = reinterpret_cast<unsigned long long*>(a.rec_count);
-            if (tb) {
-                unsigned long long old = 0;
-                if (__lane_id() == (unsigned)leader) old = atomicAdd(rc, inc);
-                rs = __shfl((uint32_t)old, leader) + (uint32_t)__popcll(tb & __lanemask_lt());
-            } else if (cb && __lane_id() == (unsigned)leader) {
-                atomicAdd(rc, inc);
-            }
-        }
-        if (take) {
-            if (a.rec_ring) rs %= a.rec_cap;
-            if (rs < a.rec_cap) {
-                float* rec = a.records + (size_t)rs * guide::kRecord;
-                rec[20] = __uint_as_float(rec_tag(key, gr.w));
-                const V3 wdir = to_world(fr, wi);
-                const float vals[20] = {pos.x, pos.y, pos.z, nrm.x, nrm.y, nrm.z, -d.x, -d.y, -d.z, wdir.x, wdir.y,
-                                        wdir.z, 0.0f, rec_w, rad.x, rad.y, rad.z,
-                                        thr.x * wgt.x, thr.y * wgt.y, thr.z * wgt.z};
-                for (int k = 0; k < 20; ++k) rec[k] = vals[k];
-                if (gr.w == 0) gr.x = rs;
-                else if (gr.w == 1) gr.y = rs;
-                else gr.z = rs;
-                ++gr.w;
-            }
-        }
-        const uint32_t slot = atomicAdd(cntB, 1u);
-        B.o[slot] = make_float4(no.x, no.y, no.z, __uint_as_float(pix));
-        B.d[slot] = make_float4(wwi.x, wwi.y, wwi.z, __uint_as_float(jid));
-        B.thr[slot] = make_float4(thr.x * wgt.x, thr.y * wgt.y, thr.z * wgt.z, __uint_as_float(r.k));
-        B.rad[slot] = make_float4(rad.x, rad.y, rad.z, __uint_as_float(nd));
-        B.key[slot] = key;
-        if (a.per_path) B.local[slot] = A.local[i];
-        if (GUIDED && a.train) B.grec[slot] = gr;
+        __syncthreads();
+        if (!alive) continue;
+        uint32_t slot = survivors[turn][kBlock / 64] + (uint32_t)__popcll(am & __lanemask_lt());
+        for (uint32_t v = 0; v < wave; ++v) slot += survivors[turn][v];
+        store_survivor<GUIDED>(a, B, sv, slot);
+    }
+    if (MULTI && a.n_jobs <= kDoneJobs) {
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < a.n_jobs; k += kBlock)
+            if (done[k]) count_done(a, k, done[k]);
     }
 }
-
 
 uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
@@ -1228,15 +1310,20 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
 // on its own stream, with its own queue (the capacity split between them),
 // status word, flags and stack spill buffer, taking a contiguous share of
 // the call's path numbering. One wavefront's traversal (bound by VALU issue)
-// then overlaps another's shading (bound by memory latency). Per-path results
-// do not depend on the wavefront a path runs in. Guided calls (one record
-// ring, one output buffer) and calls of fewer than 2^21 paths per wavefront
-// run as one.
+// then overlaps another's gathers. Per-path results do not depend on the
+// wavefront a path runs in. Calls of fewer than 2^21 paths per wavefront use
+// fewer.
 template <bool MULTI>
 spt_status run_fronts(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuning& tn, spt_render_stats& stats) {
     spt_tuning t1 = tn;
     uint32_t k = std::max<uint32_t>(1, std::min<uint32_t>(4, tn.wavefronts));
     if (a.rec_ring) k = 1;  // in-call training trains from one wavefront's ring
+    // a plain render of one scene runs as one wavefront unless the caller asks
+    // for more: its traversal and shading each fill the chip (800x600, 256
+    // spp: 132 ms on one, 138 on three; 1024 spp 506 and 548); guided passes
+    // and batches keep a gain of 2-6% (64-spp guided pass 66.6 against 67.8
+    // ms, 12 scenes 69.0 against 72.2 ms)
+    if (!MULTI && !a.guided && ctx->tuning.wavefronts == 0) k = 1;
     while (k > 1 && total / k < (1ull << 21)) --k;
     if (k == 1) {
         t1.wavefronts = 1;
@@ -1482,6 +1569,7 @@ spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
     a.tiles = b.d_tiles;
     a.tile_start = b.d_tile_start;
     a.n_tiles = (uint32_t)tiles.size();
+    a.n_jobs = nj;
     a.job_done = b.d_done;
     a.job_clock = b.d_clock;
     a.flags = 0;
