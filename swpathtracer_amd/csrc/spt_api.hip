@@ -32,11 +32,16 @@ spt_status stream_wait(spt_ctx* ctx, const char* what) {
     }
 }
 
-spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what) {
-    if (bytes > 4096 || !ctx->h_pin) return set_error(ctx, SPT_ERR_INVALID, "read_small: more than 4 KiB");
-    spt_status s = check_hip(ctx, hipMemcpyAsync(ctx->h_pin, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
+spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what, void* dst2,
+                      const void* d_src2, size_t bytes2) {
+    if (bytes + bytes2 > 4096 || !ctx->h_pin) return set_error(ctx, SPT_ERR_INVALID, "read_small: more than 4 KiB");
+    char* pin = static_cast<char*>(ctx->h_pin);
+    spt_status s = check_hip(ctx, hipMemcpyAsync(pin, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
+    if (s == SPT_OK && bytes2)
+        s = check_hip(ctx, hipMemcpyAsync(pin + bytes, d_src2, bytes2, hipMemcpyDeviceToHost, ctx->stream), what);
     if (s == SPT_OK) s = stream_wait(ctx, what);
-    if (s == SPT_OK) std::memcpy(dst, ctx->h_pin, bytes);
+    if (s == SPT_OK) std::memcpy(dst, pin, bytes);
+    if (s == SPT_OK && bytes2) std::memcpy(dst2, pin + bytes, bytes2);
     return s;
 }
 

@@ -444,8 +444,10 @@ spt_status check_hip(spt_ctx* ctx, hipError_t e, const char* what);
 // Waits for the context stream by polling it (no blocking wait on an
 // interrupt: those have been seen to wake up hundreds of ms late).
 spt_status stream_wait(spt_ctx* ctx, const char* what);
-// Copies up to 4 KiB from the device through pinned memory and waits.
-spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what);
+// Copies up to 4 KiB, from one or two places, from the device through pinned
+// memory and waits once.
+spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what, void* dst2 = nullptr,
+                      const void* d_src2 = nullptr, size_t bytes2 = 0);
 // grows ctx->d_spill to hold `words` entries; returns false on failure
 spt_status ensure_spill(spt_ctx* ctx, size_t words);
 // launch helpers implemented by the kernel translation units

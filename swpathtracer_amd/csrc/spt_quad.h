@@ -182,6 +182,8 @@ struct RayShares {
         groups = (fixed + chunk - 1) / chunk;
         span = (n - fixed + kRayCounters - 1) / kRayCounters;
     }
+    // all n rays to one wave
+    __device__ explicit RayShares(uint32_t n) : waves(1), chunk(kQuadPool), fixed(n), groups((n + kQuadPool - 1) / kQuadPool), span(0) {}
 };
 
 __device__ inline uint64_t ballot(bool x) { return __builtin_amdgcn_ballot_w64(x); }
@@ -193,8 +195,9 @@ __device__ inline int lanes(uint64_t mask) { return (int)__builtin_popcountll(ma
 // result: it is called by one lane per ray. `refill`: idle lanes of a wave that make it
 // take new rays. spill: this block's spill space (quad_spill_words words).
 template <bool FETCH, typename GetRay, typename PutHit>
-__device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray_counter, QuadLds& lds,
-                                   uint32_t* spill, bool& overflow, uint32_t refill, GetRay get_ray, PutHit put_hit) {
+__device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh, uint32_t first_group,
+                                    uint32_t* ray_counter, QuadLds& lds, uint32_t* spill, bool& overflow,
+                                    uint32_t refill, GetRay get_ray, PutHit put_hit) {
     const uint32_t lane = __lane_id(), q4 = lane & 3u, quad = threadIdx.x >> 2;
     float4(*pool)[kQuadPool] = lds.pool[threadIdx.x >> 6];
     lds_entry* stk = (lds_entry*)lds.stack[quad];
@@ -204,14 +207,14 @@ __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray
     const char* nodes_at = reinterpret_cast<const char*>(sc.qnodes);
     const char* prims_at = reinterpret_cast<const char*>(sc.qprims);
     const uint32_t child_ofs = 16 + 12 * q4, prim_ofs = 48 * q4;
-    RayShares sh(n, gridDim.x * (kBlock / 64));
+    sh.waves = __builtin_amdgcn_readfirstlane(sh.waves);
     sh.chunk = __builtin_amdgcn_readfirstlane(sh.chunk);  // scalar registers
     sh.fixed = __builtin_amdgcn_readfirstlane(sh.fixed);
     sh.groups = __builtin_amdgcn_readfirstlane(sh.groups);
     sh.span = __builtin_amdgcn_readfirstlane(sh.span);
     uint32_t range = 0, range_end = 0;  // rays taken and not yet in the pool
     uint32_t pool_n = 0, pool_at = 0;   // rays in the pool, next one to hand out
-    uint32_t group = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
+    uint32_t group = __builtin_amdgcn_readfirstlane(first_group);
     uint32_t tried = 0;                 // regions found empty, the block's own first
     uint32_t left = sh.span;            // rays left in the current region at this wave's last look
     bool more = true;
@@ -547,6 +550,14 @@ __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray
             pop();
         }
     }
+}
+
+// The rays of a launch, shared between all its waves.
+template <bool FETCH, typename GetRay, typename PutHit>
+__device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray_counter, QuadLds& lds,
+                                   uint32_t* spill, bool& overflow, uint32_t refill, GetRay get_ray, PutHit put_hit) {
+    trace_shares<FETCH>(sc, n, RayShares(n, gridDim.x * (kBlock / 64)), blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
+                        ray_counter, lds, spill, overflow, refill, get_ray, put_hit);
 }
 
 }  // namespace spt

@@ -24,7 +24,6 @@ namespace {
 constexpr uint32_t kLdsMats = 48;         // shading stages up to this many materials in LDS
 constexpr uint32_t kMaxSortKeys = 1024;  // materials + 1 (miss) sorted; more keys: unsorted
 constexpr uint32_t kMaxSortBlocks = 2048;  // most chunks (blocks) of the histogram / scatter passes
-constexpr uint32_t kScanThreads = 1024;
 
 // Path state of one buffer (structure of arrays, one slot per live path).
 // Two buffers alternate: shade reads buffer A and appends survivors to B.
@@ -45,7 +44,8 @@ struct Work {
     float4* hit;       // t, leaf-order triangle index (bits), u, v   (indexed like buffer A)
     uint32_t* skey;    // sort key: material of the hit, n_mats for a miss
     uint32_t* perm;    // shading order (stable counting sort by skey)
-    uint32_t* bhist;   // [key][block] histogram, then exclusive offsets
+    uint32_t* bhist;   // [key][block] histogram, then exclusive offsets within the key
+    uint32_t* btotal;  // slots per key
     uint32_t* cnt;     // [0], [1]: live counts of the two buffers; [2]: replay overflows;
                        // u64 at [10]: rays, u64 at [12]: bounces
     uint32_t* rays;    // ray counters of the extend kernel (kRayCounterWords)
@@ -246,6 +246,18 @@ __global__ __launch_bounds__(kBlock) void k_generate(RenderArgs a, PathBuf A, Wo
 // u64 [20] next path to generate; [24] first slot and [25] number of the
 // planned new paths, u64 [26] their first path index; [28] plans made;
 // u64 [30] hits evaluated by the guide network.
+// A ray counter's line (w.rays) also holds, for the blocks that share it: u64
+// [2] rays k_finish traced, [4] the segments of its longest path.
+// Live paths from which k_finish takes over once none is left to generate: a
+// lane for each in the waves that fit the chip. 2^18 against none and 2^20:
+// 800x600 mesh image, 4 samples 4.6 (6.1, 4.3) ms; 256x256 box image, 16
+// samples 1.69 (1.77, 1.51); batch of 8 scenes, two wavefronts 8.4 (9.0, 9.3):
+// with more paths than lanes the incoherent ones of a batch run longer than
+// in sorted bounces.
+constexpr uint32_t kFinishPaths = 1u << 18;
+// Live paths below which the host follows each bounce closely.
+constexpr uint32_t kNearEnd = 1u << 21;
+constexpr int kFinishRays = 2, kFinishBounces = 4;
 constexpr int kGen = 20, kPlanSlot = 24, kPlanN = 25, kPlanPath = 26, kPlanSeq = 28;
 
 // Between bounces (one wave): the consumed buffer's count and the extend
@@ -363,41 +375,41 @@ __global__ __launch_bounds__(kBlock) void k_hist(RenderArgs a, Work w, const uin
     for (uint32_t k = threadIdx.x; k < a.keys; k += kBlock) w.bhist[k * gridDim.x + blockIdx.x] = hist[k];
 }
 
-// Exclusive prefix sum of the [key][chunk] counts in place, one block:
-// tiles of kScanThreads counts read and written coalesced, each scanned by
-// wave shuffles and one pass over the wave totals, with a running carry.
-__global__ __launch_bounds__(kScanThreads) void k_scan(RenderArgs a, Work w, uint32_t nb) {
-    constexpr uint32_t kWaves = kScanThreads / 64;
-    __shared__ uint32_t wbase[kWaves];
-    __shared__ uint32_t tile_sum;
-    const uint32_t total = a.keys * nb;
+// Exclusive prefix sum over the chunks of each key in place, a block per key,
+// and the key's total; k_scatter adds the totals of the keys before. One block
+// scanning all keys in turn took 12 us with 4 keys and 90 us with the 30 of a
+// batch of scenes; this takes 6 and 6.
+__global__ __launch_bounds__(kBlock) void k_scan(RenderArgs a, Work w, uint32_t nb, const uint32_t* __restrict__ cntA) {
+    constexpr uint32_t kWaves = kBlock / 64;
+    __shared__ uint32_t wsum[2][kWaves];
+    if (*cntA == 0) return;
+    uint32_t* row = w.bhist + (size_t)blockIdx.x * nb;
     const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
-    uint32_t carry = 0;
-    for (uint32_t t0 = 0; t0 < total; t0 += kScanThreads) {
+    uint32_t carry = 0, turn = 0;
+    for (uint32_t t0 = 0; t0 < nb; t0 += kBlock, turn ^= 1u) {
         const uint32_t i = t0 + threadIdx.x;
-        const uint32_t v = i < total ? w.bhist[i] : 0u;
+        const uint32_t v = i < nb ? row[i] : 0u;
         uint32_t x = v;  // inclusive scan within the wave
         for (uint32_t off = 1; off < 64; off <<= 1) {
             const uint32_t y = __shfl_up(x, off);
             if (lane >= off) x += y;
         }
-        if (lane == 63) wbase[wave] = x;
+        if (lane == 63) wsum[turn][wave] = x;
         __syncthreads();
-        if (wave == 0) {  // exclusive scan of the wave totals
-            const uint32_t s = lane < kWaves ? wbase[lane] : 0u;
-            uint32_t t = s;
-            for (uint32_t off = 1; off < kWaves; off <<= 1) {
-                const uint32_t y = __shfl_up(t, off);
-                if (lane >= off) t += y;
-            }
-            if (lane < kWaves) wbase[lane] = t - s;
-            if (lane == kWaves - 1) tile_sum = t;
+        uint32_t below = 0, all = 0;
+        for (uint32_t k = 0; k < kWaves; ++k) {
+            below += k < wave ? wsum[turn][k] : 0u;
+            all += wsum[turn][k];
         }
-        __syncthreads();
-        if (i < total) w.bhist[i] = carry + wbase[wave] + x - v;
-        carry += tile_sum;
-        __syncthreads();  // wbase and tile_sum are rewritten by the next tile
+        if (i < nb) row[i] = carry + below + x - v;
+        carry += all;
     }
+    if (threadIdx.x != 0) return;
+    w.btotal[blockIdx.x] = carry;
+    // guided calls: the hits the guide network evaluates this bounce, those on
+    // guidable materials (the last key is the misses)
+    if (a.guided && carry && blockIdx.x + 1 < a.keys && guide_mode(a, blockIdx.x) != 0u)
+        atomicAdd(reinterpret_cast<unsigned long long*>(w.cnt + 30), (unsigned long long)carry);
 }
 
 __global__ __launch_bounds__(kBlock) void k_scatter(RenderArgs a, Work w, const uint32_t* __restrict__ cntA) {
@@ -405,13 +417,29 @@ __global__ __launch_bounds__(kBlock) void k_scatter(RenderArgs a, Work w, const 
     __shared__ uint32_t wcnt[kBlock / 64][kMaxSortKeys];
     const uint32_t n = *cntA;
     const uint32_t wave = threadIdx.x / 64;
+    uint32_t c0, c1;
+    chunk_range(n, blockIdx.x, gridDim.x, c0, c1);
+    if (c0 >= c1) return;
+    if (wave == 0) {  // exclusive scan of the keys' totals
+        uint32_t carry = 0;
+        for (uint32_t k0 = 0; k0 < a.keys; k0 += 64) {
+            const uint32_t k = k0 + threadIdx.x;
+            const uint32_t v = k < a.keys ? w.btotal[k] : 0u;
+            uint32_t x = v;
+            for (uint32_t off = 1; off < 64; off <<= 1) {
+                const uint32_t y = __shfl_up(x, off);
+                if (threadIdx.x >= off) x += y;
+            }
+            if (k < a.keys) base[k] = carry + x - v;
+            carry += __shfl(x, 63);
+        }
+    }
+    __syncthreads();
     for (uint32_t k = threadIdx.x; k < a.keys; k += kBlock) {
-        base[k] = w.bhist[k * gridDim.x + blockIdx.x];
+        base[k] += w.bhist[k * gridDim.x + blockIdx.x];
         for (uint32_t v = 0; v < kBlock / 64; ++v) wcnt[v][k] = 0;
     }
     __syncthreads();
-    uint32_t c0, c1;
-    chunk_range(n, blockIdx.x, gridDim.x, c0, c1);
     const uint64_t lt = __lanemask_lt();
     for (uint32_t r0 = c0; r0 < c1; r0 += kBlock) {
         const uint32_t e = r0 + threadIdx.x;
@@ -447,18 +475,6 @@ __global__ __launch_bounds__(kBlock) void k_scatter(RenderArgs a, Work w, const 
         }
         __syncthreads();
     }
-}
-
-// Guided calls: the hits the guide network evaluates this bounce (those on
-// guidable materials), read off the sort's exclusive offsets ([key][chunk]:
-// the count of key m is the first offset of m + 1 minus that of m), added to
-// the u64 at work word 30. One thread.
-__global__ void k_count_guided(RenderArgs a, Work w, uint32_t nb) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    unsigned long long q = 0;
-    for (uint32_t m = 0; m + 1 < a.keys; ++m)  // the last key is the misses
-        if (guide_mode(a, m) != 0u) q += w.bhist[(m + 1) * nb] - w.bhist[m * nb];
-    if (q) atomicAdd(reinterpret_cast<unsigned long long*>(w.cnt + 30), q);
 }
 
 // Guide inference for the live hits of buffer A whose material is guidable,
@@ -906,6 +922,106 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
 }
 
+// Every path of buffer A (count *cntA) run to its end in one launch: a wave
+// owns a contiguous share of the paths, up to 64 at a time in its lanes, and
+// alternates between tracing their rays with its 16 quads and shading them in
+// place, at its own pace. For the last paths of a call, and all paths of a
+// small one, whose bounces would each take seven launches and wait for the
+// longest ray (up to 100 us) and the longest layered walk (500 steps, 110 us)
+// of any path: here a path waits for those of its own wave. Bound by the
+// latency of those chains; the path state and hits stay in the queue's arrays,
+// read back from the caches. 128 VGPRs and 36 KB of LDS: four blocks a CU.
+// 97x61 box image, 1 sample: 590 -> 150 us; 800x600 mesh image, 4 samples,
+// where it takes the bounces from the eighth on: 6.1 -> 4.4 ms.
+template <bool MULTI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_finish(
+    RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA, uint32_t* __restrict__ spill,
+    uint32_t* __restrict__ flags) {
+    __shared__ QuadLds lds;
+    __shared__ spt_material smats[kLdsMats];
+    __shared__ uint32_t slots[kBlock / 64][64];
+    __shared__ uint32_t done[MULTI ? kDoneJobs : 1];
+    const bool lds_mats = a.sc.n_mats <= kLdsMats;
+    if (lds_mats) {
+        const uint32_t words = a.sc.n_mats * (uint32_t)(sizeof(spt_material) / 4);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(a.sc.mats);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(smats);
+        for (uint32_t k = threadIdx.x; k < words; k += kBlock) dst[k] = src[k];
+    }
+    if (MULTI)
+        for (uint32_t k = threadIdx.x; k < kDoneJobs; k += kBlock) done[k] = 0;
+    __syncthreads();
+    a.keys = 0;  // slots are shaded in place, not in material order
+    const uint32_t n = *cntA;
+    const uint32_t waves = gridDim.x * (kBlock / 64);
+    const uint32_t share = (n + waves - 1) / waves;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
+    uint32_t next = min(n, wave * share);
+    const uint32_t end = min(n, next + share);
+    uint32_t* mine = slots[threadIdx.x >> 6];
+    const uint64_t lt = __lanemask_lt();
+    bool overflow = false;
+    uint32_t slot = kDone, segments = 0, longest = 0;
+    uint32_t rays = 0;
+    while (true) {
+        const uint64_t need = ballot(slot == kDone);
+        if (slot == kDone) {
+            const uint32_t k = next + (uint32_t)lanes(need & lt);
+            if (k < end) {
+                slot = k;
+                segments = 0;
+            }
+        }
+        next = min(end, next + (uint32_t)lanes(need));
+        const uint64_t live = ballot(slot != kDone);
+        if (!live) break;
+        const uint32_t m = (uint32_t)lanes(live);
+        rays += m;
+        if (slot != kDone) mine[lanes(live & lt)] = slot;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        trace_shares<false>(
+            a.sc, m, RayShares(m), 0u, w.rays, lds, spill + (size_t)blockIdx.x * quad_spill_words(a.sc.stack_cap4), overflow,
+            a.refill,
+            [&](uint32_t i, V3& o, V3& d, Root& root) {
+                const uint32_t s = mine[i];
+                const float4 o4 = A.o[s], d4 = A.d[s];
+                o = V3{o4.x, o4.y, o4.z};
+                d = V3{d4.x, d4.y, d4.z};
+                if (MULTI) {
+                    const Job& jb = a.jobs[__float_as_uint(d4.w)];
+                    root = Root{V3{jb.rmin[0], jb.rmin[1], jb.rmin[2]}, V3{jb.rmax[0], jb.rmax[1], jb.rmax[2]}, jb.node0};
+                }
+            },
+            [&](uint32_t i, const Hit& h, V3, V3, uint32_t, uint32_t) {
+                const uint32_t s = mine[i];
+                w.hit[s] = make_float4(h.t, __uint_as_float(h.idx), h.u, h.v);
+                w.skey[s] = h.mat;
+            });
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        if (slot != kDone) {
+            bool alive = false;
+            longest = max(longest, ++segments);
+            shade_path<MULTI, false>(a, A, w, smats, lds_mats, slot, done, [&](const Survivor& sv) {
+                store_survivor<false>(a, A, sv, slot);
+                alive = true;
+            });
+            if (!alive) slot = kDone;
+        }
+    }
+    if (overflow) atomicOr(flags, 1u);
+    for (int k = 32; k > 0; k >>= 1) longest = max(longest, (uint32_t)__shfl_xor(longest, k));
+    if (__lane_id() == 0 && rays) {
+        uint32_t* c = w.rays + (blockIdx.x % kRayCounters) * kRayCounterStride;
+        atomicAdd(reinterpret_cast<unsigned long long*>(c + kFinishRays), (unsigned long long)rays);
+        atomicMax(c + kFinishBounces, longest);
+    }
+    if (MULTI && a.n_jobs <= kDoneJobs) {
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < a.n_jobs; k += kBlock)
+            if (done[k]) count_done(a, k, done[k]);
+    }
+}
+
 uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
 size_t guide_paths_lds_bytes() {
@@ -1016,7 +1132,7 @@ template <bool MULTI>
 spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuning& tn, spt_render_stats& stats) {
     uint64_t cap = std::min<uint64_t>(total, tn.path_capacity);
     auto state_bytes = [](uint64_t c) {
-        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + (size_t)kMaxSortKeys * kMaxSortBlocks * 4 + 8192;
+        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + (size_t)kMaxSortKeys * (kMaxSortBlocks + 1) * 4 + 8192;
     };
     if (state_bytes(cap) > ctx->paths_bytes) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -1056,8 +1172,9 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     w.skey = (uint32_t*)take(cap * 4);
     w.perm = (uint32_t*)take(cap * 4);
     w.bhist = (uint32_t*)take((size_t)kMaxSortKeys * kMaxSortBlocks * 4);
-    w.cnt = (uint32_t*)take(256);
-    w.rays = (uint32_t*)take(kRayCounterWords * 4);
+    w.btotal = (uint32_t*)take((size_t)kMaxSortKeys * 4);
+    w.cnt = (uint32_t*)take((64 + kRayCounterWords) * 4);
+    w.rays = w.cnt + 64;
     if ((size_t)(base - reinterpret_cast<char*>(ctx->d_paths)) > ctx->paths_bytes)
         return set_error(ctx, SPT_ERR_NOMEM, "path state layout exceeds its allocation");
     a.rec_count = a.rec_shared ? a.rec_shared : w.cnt + 16;
@@ -1092,12 +1209,15 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     // sort chunks: many (latency hiding) unless many keys would make the scan long
     const uint32_t sort_blocks =
         a.keys ? std::max<uint32_t>(1024, std::min<uint32_t>(kMaxSortBlocks, 16384 / a.keys)) : 256;
-    spt_status s = ensure_spill(ctx, std::max<size_t>(1, (size_t)ext_grid * quad_spill_words(a.sc.stack_cap4)));
-    if (s != SPT_OK) return s;
     hipStream_t st = ctx->stream;
     const bool timed = (a.flags & SPT_RENDER_TIME_KERNELS) != 0;
     const bool fetch_stats = (a.flags & SPT_RENDER_FETCH_STATS) != 0;
-    s = check_hip(ctx, hipMemsetAsync(w.cnt, 0, 256, st), "counters");  // the ray counters: k_plan
+    const uint64_t finish_at = (a.guided || timed || fetch_stats) ? 0 : kFinishPaths;
+    const uint32_t finish_grid = std::min<uint32_t>(blocks_for(std::min<uint64_t>(cap, finish_at) * 64), (uint32_t)ctx->num_cus * 4);
+    spt_status s = ensure_spill(
+        ctx, std::max<size_t>(1, (size_t)std::max(ext_grid, finish_grid) * quad_spill_words(a.sc.stack_cap4)));
+    if (s != SPT_OK) return s;
+    s = check_hip(ctx, hipMemsetAsync(w.cnt, 0, (64 + kRayCounterWords) * 4, st), "counters");
     if (s != SPT_OK) return s;
     if (a.train && !a.rec_shared) {  // records continue after those collected since the last training step
         s = check_hip(ctx,
@@ -1114,6 +1234,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         if (s != SPT_OK) return s;
     }
     std::vector<hipEvent_t> gev;  // guide inference launches (TIME_KERNELS)
+    bool generated = total <= cap;  // no bounce plans new paths any more, as far as the host has seen
     // One bounce over buffer (b & 1) into the other buffer.
     auto bounce = [&](uint32_t b) -> spt_status {
         PathBuf& A = buf[b & 1];
@@ -1141,9 +1262,8 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         }
         if (a.keys) {
             hipLaunchKernelGGL(k_hist, dim3(sort_blocks), dim3(kBlock), 0, st, a, w, cntA);
-            hipLaunchKernelGGL(k_scan, dim3(1), dim3(kScanThreads), 0, st, a, w, sort_blocks);
+            hipLaunchKernelGGL(k_scan, dim3(a.keys), dim3(kBlock), 0, st, a, w, sort_blocks, cntA);
             hipLaunchKernelGGL(k_scatter, dim3(sort_blocks), dim3(kBlock), 0, st, a, w, cntA);
-            if (a.guided) hipLaunchKernelGGL(k_count_guided, dim3(1), dim3(64), 0, st, a, w, sort_blocks);
         }
         if (a.guided) {
             if (timed) {
@@ -1165,7 +1285,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         // regeneration: the survivors' buffer is topped up with new camera paths
         hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, cntA, cntB, w.cnt, w.rays, (uint32_t)cap, total, ctx->d_status,
                            a.job_clock);
-        hipLaunchKernelGGL((k_refill<MULTI>), dim3(refill_grid), dim3(kBlock), 0, st, a, B, w);
+        if (!generated) hipLaunchKernelGGL((k_refill<MULTI>), dim3(refill_grid), dim3(kBlock), 0, st, a, B, w);
         return check_hip(ctx, hipGetLastError(), "bounce launch");
     };
     // Graph mode: two bounces (one per buffer parity) captured once and
@@ -1199,7 +1319,9 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     }
     // The host stays at most `lag` bounces ahead of the device and stops once
     // a plan reports every path generated and none live; the bounces issued
-    // after that one find empty queues (a few empty launches each).
+    // after that one find empty queues (a few empty launches each: 30 us).
+    // Once few paths are left it stays one bounce ahead, so that it sees the
+    // end, or the point for k_finish, sooner.
     const uint32_t lag = std::max<uint32_t>(2, graph_on ? (tn.check_every + 1) & ~1u : tn.check_every);
     if (!MULTI && a.job.max_depth == 0) {  // every path finishes at generation
         for (uint64_t done = 0; done < total && s == SPT_OK; done += cap) {
@@ -1217,7 +1339,16 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         // in-call training (ring of records): train aligned batches of the
         // records counted one round earlier; skip what is about to be reused
         uint32_t next_train = ctx->guide.train_every, prev_count = 0, trained = 0;
-        while (s == SPT_OK) {
+        auto finish = [&]() {  // reads its count on the device: may be queued behind a bounce still running
+            hipLaunchKernelGGL((k_finish<MULTI>), dim3(finish_grid), dim3(kBlock), 0, st, a, buf[b & 1], w, w.cnt + (b & 1),
+                               ctx->d_spill, ctx->d_flags);
+            return check_hip(ctx, hipGetLastError(), "finish launch");
+        };
+        auto few = [&](uint64_t live) { return live <= kNearEnd && !a.rec_ring; };
+        bool near_end = generated && few(total);
+        const bool at_once = generated && total <= finish_at;
+        if (s == SPT_OK && at_once) s = finish();
+        while (s == SPT_OK && !at_once) {
             if (graph_on) {
                 s = check_hip(ctx, hipGraphLaunch(exec, st), "graph launch");
                 b += 2;
@@ -1225,9 +1356,10 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
                 s = bounce(b);
                 ++b;
             }
-            if (s != SPT_OK || b <= lag) continue;
+            const uint32_t behind = near_end ? (graph_on ? 2u : 1u) : lag;
+            if (s != SPT_OK || b <= behind) continue;
             // plan number 1 is the initial one; bounce j's plan is number j + 2
-            const uint32_t want = b - lag + 1;
+            const uint32_t want = b - behind + 1;
             bool idle = false;
             while (ctx->h_status[0] < want && !idle) {
                 const hipError_t q = hipStreamQuery(st);
@@ -1236,7 +1368,16 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
                 if (s != SPT_OK) break;
                 __builtin_ia32_pause();
             }
-            if (s == SPT_OK && ctx->h_status[2] && ctx->h_status[1] == 0) break;
+            if (s == SPT_OK && ctx->h_status[2]) {
+                generated = true;
+                const uint32_t live = ctx->h_status[1];
+                if (live == 0) break;
+                if (live <= finish_at) {
+                    s = finish();
+                    break;
+                }
+                near_end = few(live);
+            }
             if (idle && ctx->h_status[0] < want) {
                 s = set_error(ctx, SPT_ERR_DEVICE, "bounce status did not advance");
                 break;
@@ -1259,8 +1400,9 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         drop_graph();
         return s;
     }
-    uint32_t cnt[32];  // the work words above
-    s = read_small(ctx, cnt, w.cnt, sizeof(cnt), "render");
+    uint32_t cnt[64 + kRayCounterWords];  // the work words and the ray counters' lines
+    uint32_t flags = 0;
+    s = read_small(ctx, cnt, w.cnt, sizeof(cnt), "render", &flags, ctx->d_flags, sizeof(flags));
     drop_graph();
     if (s != SPT_OK) return s;
     stats.stream_overflows = cnt[2];
@@ -1281,6 +1423,13 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     stats.rays = (uint64_t)cnt[10] | ((uint64_t)cnt[11] << 32);
     if (a.train && !a.rec_shared && total) ctx->guide.rays_per_path = std::max(1.0, (double)stats.rays / (double)total);
     stats.bounces = (uint64_t)cnt[12] | ((uint64_t)cnt[13] << 32);
+    uint32_t longest = 0;
+    for (uint32_t k = 0; k < kRayCounters; ++k) {
+        const uint32_t* c = cnt + 64 + k * kRayCounterStride;
+        stats.rays += (uint64_t)c[kFinishRays] | ((uint64_t)c[kFinishRays + 1] << 32);
+        longest = std::max(longest, c[kFinishBounces]);
+    }
+    stats.bounces += longest;
     stats.guide_queries = (uint64_t)cnt[30] | ((uint64_t)cnt[31] << 32);
     if (timed) {
         for (uint64_t i = 0; i < stats.extend_launches; ++i) {
@@ -1288,9 +1437,6 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
             if (hipEventElapsedTime(&ms, ctx->tev[2 * i], ctx->tev[2 * i + 1]) == hipSuccess) stats.extend_ms += ms;
         }
     }
-    uint32_t flags = 0;
-    s = read_small(ctx, &flags, ctx->d_flags, 4, "flags");
-    if (s != SPT_OK) return s;
     if (fetch_stats) {
         unsigned long long f[2] = {0, 0};
         s = read_small(ctx, f, ctx->d_flags + 4, 16, "fetch counters");
