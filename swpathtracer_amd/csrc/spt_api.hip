@@ -622,6 +622,7 @@ spt_status spt_upload_scene(spt_ctx* ctx, const spt_node64* nodes, uint32_t n_no
     ctx->stack_cap4 = cap4;
     ctx->small_coords = quad_small_coords(tris, n_tris);
     ctx->small_tree = qt.small();
+    ctx->one_block = qt.prims.size() == 4;
     ctx->max_mat = 0;
     ctx->has_spheres = false;
     for (uint32_t i = 0; i < n_tris; ++i) {

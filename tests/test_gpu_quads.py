@@ -99,3 +99,22 @@ def test_axis_aligned_rays(device):
     r[np.arange(len(r)), 4 + axis] = rng.choice([-1.0, 1.0], len(r))
     r[::3, 1] = -1.0
     _check(device, sc.verts, r)
+
+
+@pytest.mark.parametrize("spheres,triangles", [(1, 0), (2, 0), (4, 0), (1, 3), (0, 4), (2, 3)])
+@pytest.mark.parametrize("distance", [3.0, 5000.0])
+def test_scenes_of_one_block(device, spheres, triangles, distance):
+    """Up to four primitives are tested without a tree (five with one)."""
+    rng = np.random.default_rng(10 * spheres + triangles)
+    n = spheres + triangles
+    v = _soup(rng, n, 0.6)
+    kinds = np.zeros(n, np.uint32)
+    kinds[:spheres] = L.SPT_PRIM_SPHERE
+    v[:spheres, 3:] = 0.0
+    v[:spheres, 3] = rng.uniform(0.3, 0.9, spheres)
+    for n_rays in (1, 255, 257, 70_001):
+        r = _rays(rng, n_rays, -1, 1)
+        r[:, 0:3] -= np.float32(distance) * r[:, 4:7]
+        r[::9, 0:3] = rng.uniform(-0.3, 0.3, r[::9, 0:3].shape)
+        r[::101, 5] = np.nan
+        _check(device, v, r, kinds=kinds)
