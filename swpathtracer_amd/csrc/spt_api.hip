@@ -45,6 +45,28 @@ spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, 
     return s;
 }
 
+spt_material prepare_material(const spt_material& m) {
+    spt_material r = m;
+    for (uint32_t i = 0; i < std::min<uint32_t>(m.n_layers, SPT_MAX_LAYERS); ++i) {
+        spt_layer& l = r.layers[i];
+        if (l.type == SPT_BSDF_LAMBERTIAN) {
+            for (int c = 0; c < 3; ++c) l.r0[c] = l.kd[c] / kPi;
+        } else if (l.type == SPT_BSDF_SMOOTH_DIELECTRIC) {
+            const float root = (1.0f - l.ior) / (1.0f + l.ior);
+            l.r0[0] = root * root;
+            l.r0[1] = 1.0f / l.ior;
+            l.r0[2] = 1.0f / (l.ior * l.ior);
+        } else if (l.type == SPT_BSDF_GGX_CONDUCTOR) {
+            for (int c = 0; c < 3; ++c) {
+                const float e2 = l.eta[c] * l.eta[c], k2 = l.k[c] * l.k[c];
+                l.eta[c] = e2 - k2;
+                l.k[c] = 4.0f * e2 * k2;
+            }
+        }
+    }
+    return r;
+}
+
 spt_status ensure_spill(spt_ctx* ctx, size_t words) {
     if (words <= ctx->spill_words) return SPT_OK;
     if (ctx->d_spill) {
@@ -656,7 +678,9 @@ spt_status spt_set_materials(spt_ctx* ctx, const spt_material* mats, uint32_t n_
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->d_mats) (void)hipFree(ctx->d_mats);
     ctx->d_mats = nullptr;
-    spt_status s = upload(ctx, &ctx->d_mats, mats, (size_t)n_mats * sizeof(spt_material), "materials");
+    std::vector<spt_material> prepared(n_mats);
+    std::transform(mats, mats + n_mats, prepared.begin(), prepare_material);
+    spt_status s = upload(ctx, &ctx->d_mats, prepared.data(), (size_t)n_mats * sizeof(spt_material), "materials");
     if (s != SPT_OK) return s;
     ctx->n_mats = n_mats;
     ctx->h_mats.assign(mats, mats + n_mats);

@@ -227,7 +227,7 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
             std::memcpy(&o[9], &m, 4);
         }
         sh.insert(sh.end(), bs.begin(), bs.end());
-        mats.insert(mats.end(), sc.mats, sc.mats + sc.n_mats);
+        std::transform(sc.mats, sc.mats + sc.n_mats, std::back_inserter(mats), prepare_material);
         for (int k = 0; k < 3; ++k) {
             jb.rmin[k] = rb[k];
             jb.rmax[k] = rb[3 + k];

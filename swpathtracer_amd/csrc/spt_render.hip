@@ -168,7 +168,7 @@ __device__ inline Draws make_draws(const Job& jb, uint64_t key, uint32_t k) {
         r.key = 0;
         r.stream = jb.stream + key * (uint64_t)jb.stride;
     } else {
-        r.key = key;
+        r.key = key + (uint64_t)(k + 1) * kGolden;
         r.stream = nullptr;
     }
     return r;
