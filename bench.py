@@ -409,7 +409,7 @@ def main():
                     help="samples per pixel of one step (one render call); 1 step = the 1024-spp image")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-closest-hit", action="store_true")
-    ap.add_argument("--no-sort", action="store_true", help="skip the material sort between stages")
+    ap.add_argument("--no-sort", action="store_true", help="accepted; paths are shaded in queue order")
     ap.add_argument("--rings", type=int, default=512)
     ap.add_argument("--segments", type=int, default=1024)
     ap.add_argument("--no-guide", action="store_true", help="skip the guided vs plain equal-RMSE experiment")

@@ -158,7 +158,7 @@ enum {
     SPT_RENDER_FILM32 = 1u << 0,    /* accumulate FP32 film into d_rgb32 */
     SPT_RENDER_FILM64 = 1u << 1,    /* accumulate FP64 film into d_rgb64 (oracle film) */
     SPT_RENDER_PER_PATH = 1u << 2,  /* write each path's radiance into d_path_rgb */
-    SPT_RENDER_NO_SORT = 1u << 3,   /* skip the material sort between stages */
+    SPT_RENDER_NO_SORT = 1u << 3,   /* accepted; paths are shaded in queue order */
     SPT_RENDER_GUIDED = 1u << 4,    /* sample with the learned guide (spt_guide_*) */
     SPT_RENDER_FETCH_STATS = 1u << 5, /* count tree data in 32-B units (a 64-B node is 2,
                                          a 32-B leaf record 1) and 48-B triangle records

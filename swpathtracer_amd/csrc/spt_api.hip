@@ -683,6 +683,7 @@ spt_status spt_set_materials(spt_ctx* ctx, const spt_material* mats, uint32_t n_
     spt_status s = upload(ctx, &ctx->d_mats, prepared.data(), (size_t)n_mats * sizeof(spt_material), "materials");
     if (s != SPT_OK) return s;
     ctx->n_mats = n_mats;
+    ctx->layered = std::any_of(mats, mats + n_mats, [](const spt_material& m) { return m.n_layers > 1; });
     ctx->h_mats.assign(mats, mats + n_mats);
     // vertices the learned guide may sample: a layer with an evaluable
     // density, alone or under one smooth dielectric coat

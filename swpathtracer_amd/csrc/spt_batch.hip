@@ -250,6 +250,7 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
     if (s == SPT_OK) s = check_hip(ctx, hipMalloc(&d.d_clock, (n + 1) * sizeof(uint64_t)), "batch clocks");
     if (s != SPT_OK) return fail(s);
     d.small_tree = qt.small();
+    d.layered = std::any_of(mats.begin(), mats.end(), [](const spt_material& m) { return m.n_layers > 1; });
     d.n_nodes = (uint32_t)nodes.size();
     d.n_tris = (uint32_t)tris.size();
     d.n_mats = (uint32_t)mats.size();

@@ -270,17 +270,24 @@ __device__ inline void layer_eval(const spt_layer& l, V3 wo, V3 wi, V3& f, V3& r
 
 // LayeredBSDF::evalBSDF (materials/layered_bsdf.cpp:10-74): a random walk
 // through the stack, at most 500 inner steps.
-__device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& refl, float& pdf, V3& wi,
-                                    Draws& r) {
-    const int n = (int)m.n_layers;
-    V3 fb{1.0f, 1.0f, 1.0f}, fr{1.0f, 1.0f, 1.0f};
-    float fp = 1.0f;
-    V3 nwo = wo;
-    bool reached_inf = false;
-    int bounce = 0;
-    int id = (nwo.y > 0.0f) ? 0 : n - 1;
-    const float inf = __builtin_inff();
-    while ((id > -1) && (id < n) && (fp > 0.0f) && (!reached_inf) && (bounce < 500)) {
+struct Walk {
+    V3 nwo, wi, fb, fr;
+    float fp;
+    int id, bounce;
+    bool reached_inf;
+    __device__ void start(const spt_material& m, V3 wo) {
+        nwo = wo;
+        fb = fr = V3{1.0f, 1.0f, 1.0f};
+        fp = 1.0f;
+        reached_inf = false;
+        bounce = 0;
+        id = (nwo.y > 0.0f) ? 0 : (int)m.n_layers - 1;
+    }
+    __device__ bool running(const spt_material& m) const {
+        return (id > -1) && (id < (int)m.n_layers) && (fp > 0.0f) && (!reached_inf) && (bounce < 500);
+    }
+    __device__ void step(const spt_material& m, Draws& r) {
+        const float inf = __builtin_inff();
         const spt_layer& l = m.layers[id];
         const BSample s = layer_sample(l, nwo, r);
         wi = s.wi;
@@ -294,7 +301,7 @@ __device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& 
             --id;
         } else if ((wi.y < 0.0f) && !layer_opaque(l)) {  // through a dielectric
             const V3 f = layer_f(l, nwo, wi);
-            fb = (id == n - 1) ? fb * f : fb * (f * wi.y);
+            fb = (id == (int)m.n_layers - 1) ? fb * f : fb * (f * wi.y);
             ++id;
         } else {
             fp = 0.0f;
@@ -303,15 +310,27 @@ __device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& 
         nwo = -wi;
         ++bounce;
     }
-    if ((bounce < 500) && !reached_inf && (fp > 0.0f)) {
-        pdf = fp;
-        bsdf = fb;
-        refl = fr;
-    } else {
-        pdf = 1.0f;
-        bsdf = V3{0.0f, 0.0f, 0.0f};
-        refl = V3{0.0f, 0.0f, 0.0f};
+    __device__ void result(V3& bsdf, V3& refl, float& pdf) const {
+        if ((bounce < 500) && !reached_inf && (fp > 0.0f)) {
+            pdf = fp;
+            bsdf = fb;
+            refl = fr;
+        } else {
+            pdf = 1.0f;
+            bsdf = V3{0.0f, 0.0f, 0.0f};
+            refl = V3{0.0f, 0.0f, 0.0f};
+        }
     }
+};
+
+__device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& refl, float& pdf, V3& wi,
+                                    Draws& r) {
+    Walk k;
+    k.wi = wi;
+    k.start(m, wo);
+    while (k.running(m)) k.step(m, r);
+    wi = k.wi;
+    k.result(bsdf, refl, pdf);
 }
 
 // Pixel-sampler offset of sample s (pixel_samplers/*.cpp). getSample() is

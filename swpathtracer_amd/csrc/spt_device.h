@@ -260,6 +260,7 @@ struct BatchData {
     float4* d_tris = nullptr;
     float4* d_shading = nullptr;
     spt_material* d_mats = nullptr;
+    bool layered = false;  // some material has several layers
     uint32_t n_nodes = 0, n_tris = 0, n_mats = 0, stack_cap = 0, stack_cap4 = 0;
     bool has_spheres = false, small_coords = true, small_tree = false;
     std::vector<Job> jobs;  // host copy: sampling, outputs, roots
@@ -376,6 +377,7 @@ struct spt_ctx {
     float4* d_tris = nullptr;
     float4* d_shading = nullptr;
     spt_material* d_mats = nullptr;
+    bool layered = false;  // some material has several layers
     uint32_t n_nodes = 0, n_tris = 0, n_mats = 0;
     float root_box[6] = {0, 0, 0, 0, 0, 0};
     uint32_t root_leaf = 0;

@@ -3,9 +3,10 @@
 //
 // Pipeline per bounce, each a separate kernel over a queue of live paths:
 //   generate (camera sample + primary ray) -> extend (closest hit) ->
-//   [material histogram -> scatter: paths sorted by hit material] ->
-//   shade (emission, layered BSDF walk, Russian roulette, next ray; finished
-//   paths write the film) -> the survivors form the next queue.
+//   [walk: the random walks through layered materials] -> shade (emission,
+//   BSDF sample, Russian roulette, next ray; finished paths write the film) ->
+//   the survivors form the next queue.
+// The last paths of a call run to their end in one kernel (k_finish).
 // The recursion L = Le + f * L' * cos / pdf is evaluated forwards with a
 // throughput: L = sum_d (prod_{j<d} f_j cos_j / pdf_j) * Le_d.
 #include <algorithm>
@@ -22,8 +23,7 @@ namespace spt {
 namespace {
 
 constexpr uint32_t kLdsMats = 48;         // shading stages up to this many materials in LDS
-constexpr uint32_t kMaxSortKeys = 1024;  // materials + 1 (miss) sorted; more keys: unsorted
-constexpr uint32_t kMaxSortBlocks = 2048;  // most chunks (blocks) of the histogram / scatter passes
+constexpr int kWalkRefill = 32;           // lanes of a wave without a walk that make it take new ones
 
 // Path state of one buffer (structure of arrays, one slot per live path).
 // Two buffers alternate: shade reads buffer A and appends survivors to B.
@@ -42,15 +42,13 @@ constexpr uint32_t kNoRec = 0xFFFFFFFFu;
 // Per-bounce scratch shared by both buffers.
 struct Work {
     float4* hit;       // t, leaf-order triangle index (bits), u, v   (indexed like buffer A)
-    uint32_t* skey;    // sort key: material of the hit, n_mats for a miss
-    uint32_t* perm;    // shading order (stable counting sort by skey)
-    uint32_t* bhist;   // [key][block] histogram, then exclusive offsets within the key
-    uint32_t* btotal;  // slots per key
+    uint32_t* skey;    // material of the hit, n_mats for a miss
+    float2* walk;      // layered walks: cosine and density of the sampled direction
     uint32_t* cnt;     // [0], [1]: live counts of the two buffers; [2]: replay overflows;
                        // u64 at [10]: rays, u64 at [12]: bounces
     uint32_t* rays;    // ray counters of the extend kernel (kRayCounterWords)
 };
-constexpr size_t kWorkBytes = 16 + 4 + 4;
+constexpr size_t kWorkBytes = 16 + 4 + 8;
 
 struct RenderArgs {
     DevScene sc;
@@ -65,7 +63,7 @@ struct RenderArgs {
     uint32_t flags;
     uint32_t per_path;  // some job writes per-path radiance: paths carry their output index
     uint32_t refill;  // idle lanes that trigger a ray refill in the traversal
-    uint32_t keys;  // sort keys (n_mats + 1), 0 = no sort
+    uint32_t walk;  // k_walk runs the walks of materials of several layers
     uint64_t gen_base;  // number of this wavefront's first path in the call's numbering
     // learned guide
     uint32_t guided, train;
@@ -141,15 +139,17 @@ __device__ inline void finish_path(const RenderArgs& a, const Job& jb, uint32_t 
     }
     if (jb.film32) {
         float* f = jb.film32 + 3 * (size_t)pix;
-        unsafeAtomicAdd(f + 0, L.x);
-        unsafeAtomicAdd(f + 1, L.y);
-        unsafeAtomicAdd(f + 2, L.z);
+        // adding 0 changes nothing, and most paths end without light: 28M paths
+        // shaded in 1.37 ms instead of 1.65
+        if (L.x != 0.0f) unsafeAtomicAdd(f + 0, L.x);
+        if (L.y != 0.0f) unsafeAtomicAdd(f + 1, L.y);
+        if (L.z != 0.0f) unsafeAtomicAdd(f + 2, L.z);
     }
     if (jb.film64) {
         double* f = jb.film64 + 3 * (size_t)pix;
-        unsafeAtomicAdd(f + 0, (double)L.x);
-        unsafeAtomicAdd(f + 1, (double)L.y);
-        unsafeAtomicAdd(f + 2, (double)L.z);
+        if (L.x != 0.0f) unsafeAtomicAdd(f + 0, (double)L.x);
+        if (L.y != 0.0f) unsafeAtomicAdd(f + 1, (double)L.y);
+        if (L.z != 0.0f) unsafeAtomicAdd(f + 2, (double)L.z);
     }
     if (jb.path_rgb) {
         float* o = jb.path_rgb + 3 * (size_t)local;
@@ -244,20 +244,18 @@ __global__ __launch_bounds__(kBlock) void k_generate(RenderArgs a, PathBuf A, Wo
 // Work-word layout (w.cnt, 64 words): [0], [1] live counts of the two
 // buffers; [2] replay overflows; u64 [10] rays, u64 [12] bounces; [16] guide records, [17] candidates;
 // u64 [20] next path to generate; [24] first slot and [25] number of the
-// planned new paths, u64 [26] their first path index; [28] plans made;
-// u64 [30] hits evaluated by the guide network.
+// planned new paths, u64 [26] their first path index; [28] plans made.
 // A ray counter's line (w.rays) also holds, for the blocks that share it: u64
-// [2] rays k_finish traced, [4] the segments of its longest path.
-// Live paths from which k_finish takes over once none is left to generate: a
-// lane for each in the waves that fit the chip. 2^18 against none and 2^20:
-// 800x600 mesh image, 4 samples 4.6 (6.1, 4.3) ms; 256x256 box image, 16
-// samples 1.69 (1.77, 1.51); batch of 8 scenes, two wavefronts 8.4 (9.0, 9.3):
-// with more paths than lanes the incoherent ones of a batch run longer than
-// in sorted bounces.
-constexpr uint32_t kFinishPaths = 1u << 18;
+// [2] rays k_finish traced, [4] the segments of its longest path, u64 [6]
+// hits evaluated by the guide network.
+// Live paths from which k_finish takes over once none is left to generate: two
+// for each lane of the waves that fit the chip. 2^17, 2^18, 2^19, 2^20: 800x600
+// mesh image, 4 samples 4.28, 4.06, 3.94, 3.83 ms; 256x256 box image, 16
+// samples 1.35, 1.35, 1.35, 1.46 ms; batch of 8 scenes 7.11, 7.06, 7.03, 7.02.
+constexpr uint32_t kFinishPaths = 1u << 19;
 // Live paths below which the host follows each bounce closely.
 constexpr uint32_t kNearEnd = 1u << 21;
-constexpr int kFinishRays = 2, kFinishBounces = 4;
+constexpr int kFinishRays = 2, kFinishBounces = 4, kGuideQueries = 6;
 constexpr int kGen = 20, kPlanSlot = 24, kPlanN = 25, kPlanPath = 26, kPlanSeq = 28;
 
 // Between bounces (one wave): the consumed buffer's count and the extend
@@ -305,7 +303,7 @@ __global__ __launch_bounds__(kBlock) void k_refill(RenderArgs a, PathBuf B, Work
 }
 
 // Closest hit of every live path of buffer A (count *cntA). Persistent
-// traversal; hit record and sort key written at the path's slot. FETCH adds
+// traversal; hit record and material written at the path's slot. FETCH adds
 // node / triangle record fetch counts to the two 64-bit counters at flags + 4.
 template <bool FETCH, bool MULTI>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_extend(RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA,
@@ -353,132 +351,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWav
     }
 }
 
-// Stable counting sort of the live slots by material, in three passes over
-// contiguous chunks (one per block): per-chunk histogram (LDS), one exclusive scan
-// over [key][chunk], then a scatter that ranks equal keys in slot order. No
-// global atomics: many lanes with one material would serialise on them.
-__device__ inline void chunk_range(uint32_t n, uint32_t b, uint32_t nb, uint32_t& c0, uint32_t& c1) {
-    const uint32_t per = (n + nb - 1) / nb;
-    c0 = min(n, b * per);
-    c1 = min(n, c0 + per);
-}
-
-__global__ __launch_bounds__(kBlock) void k_hist(RenderArgs a, Work w, const uint32_t* __restrict__ cntA) {
-    __shared__ uint32_t hist[kMaxSortKeys];
-    const uint32_t n = *cntA;
-    for (uint32_t k = threadIdx.x; k < a.keys; k += kBlock) hist[k] = 0;
-    __syncthreads();
-    uint32_t c0, c1;
-    chunk_range(n, blockIdx.x, gridDim.x, c0, c1);
-    for (uint32_t e = c0 + threadIdx.x; e < c1; e += kBlock) atomicAdd(&hist[w.skey[e]], 1u);
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < a.keys; k += kBlock) w.bhist[k * gridDim.x + blockIdx.x] = hist[k];
-}
-
-// Exclusive prefix sum over the chunks of each key in place, a block per key,
-// and the key's total; k_scatter adds the totals of the keys before. One block
-// scanning all keys in turn took 12 us with 4 keys and 90 us with the 30 of a
-// batch of scenes; this takes 6 and 6.
-__global__ __launch_bounds__(kBlock) void k_scan(RenderArgs a, Work w, uint32_t nb, const uint32_t* __restrict__ cntA) {
-    constexpr uint32_t kWaves = kBlock / 64;
-    __shared__ uint32_t wsum[2][kWaves];
-    if (*cntA == 0) return;
-    uint32_t* row = w.bhist + (size_t)blockIdx.x * nb;
-    const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
-    uint32_t carry = 0, turn = 0;
-    for (uint32_t t0 = 0; t0 < nb; t0 += kBlock, turn ^= 1u) {
-        const uint32_t i = t0 + threadIdx.x;
-        const uint32_t v = i < nb ? row[i] : 0u;
-        uint32_t x = v;  // inclusive scan within the wave
-        for (uint32_t off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off);
-            if (lane >= off) x += y;
-        }
-        if (lane == 63) wsum[turn][wave] = x;
-        __syncthreads();
-        uint32_t below = 0, all = 0;
-        for (uint32_t k = 0; k < kWaves; ++k) {
-            below += k < wave ? wsum[turn][k] : 0u;
-            all += wsum[turn][k];
-        }
-        if (i < nb) row[i] = carry + below + x - v;
-        carry += all;
-    }
-    if (threadIdx.x != 0) return;
-    w.btotal[blockIdx.x] = carry;
-    // guided calls: the hits the guide network evaluates this bounce, those on
-    // guidable materials (the last key is the misses)
-    if (a.guided && carry && blockIdx.x + 1 < a.keys && guide_mode(a, blockIdx.x) != 0u)
-        atomicAdd(reinterpret_cast<unsigned long long*>(w.cnt + 30), (unsigned long long)carry);
-}
-
-__global__ __launch_bounds__(kBlock) void k_scatter(RenderArgs a, Work w, const uint32_t* __restrict__ cntA) {
-    __shared__ uint32_t base[kMaxSortKeys];
-    __shared__ uint32_t wcnt[kBlock / 64][kMaxSortKeys];
-    const uint32_t n = *cntA;
-    const uint32_t wave = threadIdx.x / 64;
-    uint32_t c0, c1;
-    chunk_range(n, blockIdx.x, gridDim.x, c0, c1);
-    if (c0 >= c1) return;
-    if (wave == 0) {  // exclusive scan of the keys' totals
-        uint32_t carry = 0;
-        for (uint32_t k0 = 0; k0 < a.keys; k0 += 64) {
-            const uint32_t k = k0 + threadIdx.x;
-            const uint32_t v = k < a.keys ? w.btotal[k] : 0u;
-            uint32_t x = v;
-            for (uint32_t off = 1; off < 64; off <<= 1) {
-                const uint32_t y = __shfl_up(x, off);
-                if (threadIdx.x >= off) x += y;
-            }
-            if (k < a.keys) base[k] = carry + x - v;
-            carry += __shfl(x, 63);
-        }
-    }
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < a.keys; k += kBlock) {
-        base[k] += w.bhist[k * gridDim.x + blockIdx.x];
-        for (uint32_t v = 0; v < kBlock / 64; ++v) wcnt[v][k] = 0;
-    }
-    __syncthreads();
-    const uint64_t lt = __lanemask_lt();
-    for (uint32_t r0 = c0; r0 < c1; r0 += kBlock) {
-        const uint32_t e = r0 + threadIdx.x;
-        const bool valid = e < c1;
-        const uint32_t key = valid ? w.skey[e] : 0u;
-        uint32_t rank = 0;
-        uint64_t todo = __ballot(valid);
-        while (todo) {  // rank among equal keys of this wave, count per key
-            const int leader = __ffsll((unsigned long long)todo) - 1;
-            const uint32_t lkey = __shfl(key, leader);
-            const uint64_t group = __ballot(valid && key == lkey) & todo;
-            if (__lane_id() == (unsigned)leader) wcnt[wave][lkey] = (uint32_t)__popcll(group);
-            if (valid && key == lkey) rank = (uint32_t)__popcll(group & lt);
-            todo &= ~group;
-        }
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = base[key] + rank;
-            for (uint32_t v = 0; v < wave; ++v) pos += wcnt[v][key];
-            w.perm[pos] = e;
-        }
-        __syncthreads();
-        todo = __ballot(valid);
-        while (todo) {  // advance the running bases, clear this wave's counts
-            const int leader = __ffsll((unsigned long long)todo) - 1;
-            const uint32_t lkey = __shfl(key, leader);
-            const uint64_t group = __ballot(valid && key == lkey) & todo;
-            if (__lane_id() == (unsigned)leader) {
-                atomicAdd(&base[lkey], wcnt[wave][lkey]);
-                wcnt[wave][lkey] = 0;
-            }
-            todo &= ~group;
-        }
-        __syncthreads();
-    }
-}
-
-// Guide inference for the live hits of buffer A whose material is guidable,
-// in shading order: each wave encodes 64 hits (one per lane) and runs the
+// Guide inference for the live hits of buffer A whose material is guidable:
+// each wave encodes 64 hits (one per lane) and runs the
 // register-resident MLP; raw outputs go to gout[slot] as half floats.
 __global__ __launch_bounds__(kBlock) void k_guide_paths(RenderArgs a, PathBuf A, Work w,
                                                         const uint32_t* __restrict__ cntA,
@@ -494,13 +368,12 @@ __global__ __launch_bounds__(kBlock) void k_guide_paths(RenderArgs a, PathBuf A,
     __syncthreads();
     const int wave = threadIdx.x >> 6, l = __lane_id(), r = l & 15;
     WaveStage& st = stages[wave];
+    uint32_t queries = 0;
     for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
-        const uint32_t j = base + threadIdx.x;
+        const uint32_t slot = base + threadIdx.x;
         bool mine = false;
-        uint32_t slot = 0;
         float f[kEnc];
-        if (j < n) {
-            slot = a.keys ? w.perm[j] : j;
+        if (slot < n) {
             const float4 hv = w.hit[slot];
             const uint32_t idx = __float_as_uint(hv.y);
             mine = (idx != kNoHit) && guide_mode(a, w.skey[slot]) != 0u;
@@ -519,6 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_guide_paths(RenderArgs a, PathBuf A,
         if (!mine)
             for (int i = 0; i < kEnc; ++i) f[i] = 0.0f;
         const uint64_t any = __ballot(mine);
+        queries += (uint32_t)__popcll(any);
         stage_row(st, f);
         __syncthreads();
         if (any)
@@ -529,6 +403,9 @@ __global__ __launch_bounds__(kBlock) void k_guide_paths(RenderArgs a, PathBuf A,
             });
         __syncthreads();
     }
+    if (l == 0 && queries)
+        atomicAdd(reinterpret_cast<unsigned long long*>(w.rays + (blockIdx.x % kRayCounters) * kRayCounterStride + kGuideQueries),
+                  (unsigned long long)queries);
 }
 
 // Density of a single BSDF layer's own sampler (guidable layers only).
@@ -680,12 +557,25 @@ __device__ inline void store_survivor(const RenderArgs& a, const PathBuf& B, con
     if (GUIDED && a.train) B.grec[slot] = sv.gr;
 }
 
+// A path's vertex at its hit: position, shading normal, local frame and
+// outgoing direction in it.
+__device__ inline void path_vertex(const RenderArgs& a, V3 o, V3 d, float4 hv, V3& pos, V3& nrm, Frame& fr, V3& wo) {
+    Hit h;
+    h.t = hv.x;
+    h.idx = __float_as_uint(hv.y);
+    h.u = hv.z;
+    h.v = hv.w;
+    pos = o + d * h.t;  // triangle.cpp:69
+    nrm = shading_normal(a.sc, h, pos);
+    fr = frame_from_up(nrm);          // pathtracer.cpp:28
+    wo = normalize(to_local(fr, -d));    // pathtracer.cpp:30
+}
+
 // Shading of one vertex (integrators/pathtracer.cpp:21-54) of path j in
 // shading order; go_on(survivor) is called for a path that does not end here.
-template <bool MULTI, bool GUIDED, typename GoOn>
+template <bool MULTI, bool GUIDED, bool WALKS, typename GoOn>
 __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const Work& w, const spt_material* smats,
-                                  bool lds_mats, uint32_t j, uint32_t* done, GoOn go_on) {
-    const uint32_t i = a.keys ? w.perm[j] : j;
+                                  bool lds_mats, uint32_t i, uint32_t* done, GoOn go_on) {
     const float4 hv = w.hit[i];
     float4 rad = A.rad[i];
     const float4 thr = A.thr[i];
@@ -694,7 +584,10 @@ __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const W
     const Job& jb = job_of<MULTI>(a, jid);
     const uint32_t depth = __float_as_uint(rad.w);
     const uint32_t idx = __float_as_uint(hv.y);
-    if (idx == kNoHit) {  // miss: background at depth 0, else 0 (pathtracer.cpp:21-26)
+    const uint32_t mid = w.skey[i];
+    // the path's walk is done: hit, o and d hold its results
+    const bool walked = !WALKS && mid < a.sc.n_mats && (lds_mats ? smats[mid] : a.sc.mats[mid]).n_layers > 1;
+    if (!walked && idx == kNoHit) {  // miss: background at depth 0, else 0 (pathtracer.cpp:21-26)
         if (depth == 0) {
             rad.x += thr.x * jb.bg[0];
             rad.y += thr.y * jb.bg[1];
@@ -704,18 +597,11 @@ __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const W
         finish_path<MULTI>(a, jb, jid, pix, a.per_path ? A.local[i] : 0ull, rad, done);
         return;
     }
-    const V3 o{o4.x, o4.y, o4.z}, d{d4.x, d4.y, d4.z};
-    Hit h;
-    h.t = hv.x;
-    h.idx = idx;
-    h.u = hv.z;
-    h.v = hv.w;
-    const V3 pos = o + d * h.t;  // triangle.cpp:69
-    const V3 nrm = shading_normal(a.sc, h, pos);
-    const uint32_t mid = w.skey[i];
     const spt_material& m = lds_mats ? smats[mid] : a.sc.mats[mid];
-    const Frame fr = frame_from_up(nrm);          // pathtracer.cpp:28
-    const V3 wo = normalize(to_local(fr, -d));    // pathtracer.cpp:30
+    const V3 o{o4.x, o4.y, o4.z}, d{d4.x, d4.y, d4.z};
+    V3 pos{}, nrm{}, wo{};
+    Frame fr{};
+    if (!walked) path_vertex(a, o, d, hv, pos, nrm, fr, wo);
     const uint64_t key = A.key[i];
     Draws r = make_draws(jb, key, __float_as_uint(thr.w));
     V3 bsdf, refl, wi;
@@ -774,15 +660,33 @@ __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const W
             refl = V3{0.0f, 0.0f, 0.0f};
             pdf = 1.0f;
         }
-    } else {
+    } else if (WALKS) {
         layered_eval(m, wo, bsdf, refl, pdf, wi, r);  // pathtracer.cpp:36
+    } else if (!walked) {  // one layer: the walk is one step
+        Walk k;
+        k.start(m, wo);
+        k.step(m, r);
+        wi = k.wi;
+        k.result(bsdf, refl, pdf);
     }
-    const V3 wwi = to_world(fr, wi);              // pathtracer.cpp:37
-    const V3 no = pos + wwi * 1e-3f;              // pathtracer.cpp:38
+    V3 wwi, no;
+    float kk;
+    if (walked) {
+        const float2 cp = w.walk[i];
+        wi.y = cp.x;
+        pdf = cp.y;
+        bsdf = V3{hv.x, hv.y, hv.z};
+        kk = hv.w;
+        wwi = d;
+        no = o;
+    } else {
+        wwi = to_world(fr, wi);              // pathtracer.cpp:37
+        no = pos + wwi * 1e-3f;              // pathtracer.cpp:38
+        kk = gmax(gmax(refl.x, refl.y), refl.z);  // pathtracer.cpp:41
+    }
     rad.x += thr.x * m.emission[0];
     rad.y += thr.y * m.emission[1];
     rad.z += thr.z * m.emission[2];
-    const float kk = gmax(gmax(refl.x, refl.y), refl.z);  // pathtracer.cpp:41
     // training weight before roulette: L_i / p (PRODUCT, radiance target)
     // or f cos / p L_i (the product target)
     const float rec_w = prod ? ((pmarg > 0.0f) ? 1.0f / pmarg : 0.0f) : lum(bsdf) * wi.y / pdf;
@@ -851,15 +755,128 @@ __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const W
     go_on(sv);
 }
 
+// The walks through materials of several layers (pathtracer.cpp:28-38) of
+// the live paths of A, before k_shade, which only weighs and appends these
+// paths: new origin and direction, BSDF value, largest reflectance component,
+// cosine and density replace ray and hit in the path's slot.
+//
+// Walks of coated metal take 4 steps on average, the longest of 64 lanes 23;
+// walked inside k_shade they left 16 lanes active, unless the paths were
+// sorted by material first, which then cost the sort and the gathers of every
+// array in that order (3 TB/s of partly used lines). Here a wave looks its
+// share of the queue through for such paths (one word each) and takes new
+// ones once half of its lanes have finished; each round it steps the lanes at
+// a dielectric or the others, whichever are more, so that lanes line up.
+// 123M-path mesh image (28M live paths a launch): sort, walks and shading 2.5
+// -> 0.88 (walks) + 1.37 ms (k_shade), the rays of the unsorted queue 5% faster
+// as well. Bound by VALU issue at 20 lanes.
+template <bool MULTI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(RenderArgs a, PathBuf A, Work w,
+                                                                                           const uint32_t* __restrict__ cntA) {
+    __shared__ spt_material smats[kLdsMats];
+    __shared__ uint32_t lists[kBlock / 64][128];  // slots found and not yet taken
+    __shared__ float park[6][kBlock];  // position and normal of a lane's vertex
+    if (*cntA == 0) return;
+    const bool lds_mats = a.sc.n_mats <= kLdsMats;
+    if (lds_mats) {
+        const uint32_t words = a.sc.n_mats * (uint32_t)(sizeof(spt_material) / 4);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(a.sc.mats);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(smats);
+        for (uint32_t k = threadIdx.x; k < words; k += kBlock) dst[k] = src[k];
+    }
+    __syncthreads();
+    const uint64_t lt = __lanemask_lt();
+    const uint32_t n = *cntA, waves = gridDim.x * (kBlock / 64);
+    const uint32_t share = ((n + waves - 1) / waves + 63u) & ~63u;
+    uint32_t* list = lists[threadIdx.x / 64];
+    uint32_t next = min(n, (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * share), found = 0;
+    const uint32_t end = min(n, next + share);
+    uint32_t slot = kDone, mid = 0;
+    bool walking = false;
+    Walk wk{};
+    Draws r{};
+    while (true) {
+        const uint64_t idle = __ballot(!walking);
+        if (idle == ~0ull || ((next < end || found) && __popcll(idle) >= kWalkRefill)) {
+            if (!walking && slot != kDone) {
+                V3 bsdf, refl;
+                float pdf;
+                wk.result(bsdf, refl, pdf);
+                const V3 pos{park[0][threadIdx.x], park[1][threadIdx.x], park[2][threadIdx.x]};
+                const Frame fr = frame_from_up(V3{park[3][threadIdx.x], park[4][threadIdx.x], park[5][threadIdx.x]});
+                const V3 wwi = to_world(fr, wk.wi);  // pathtracer.cpp:37
+                const V3 no = pos + wwi * 1e-3f;     // pathtracer.cpp:38
+                float* p = reinterpret_cast<float*>(A.o + slot);
+                p[0] = no.x;
+                p[1] = no.y;
+                p[2] = no.z;
+                p = reinterpret_cast<float*>(A.d + slot);
+                p[0] = wwi.x;
+                p[1] = wwi.y;
+                p[2] = wwi.z;
+                A.thr[slot].w = __uint_as_float(r.k);
+                w.hit[slot] = make_float4(bsdf.x, bsdf.y, bsdf.z, gmax(gmax(refl.x, refl.y), refl.z));
+                w.walk[slot] = make_float2(wk.wi.y, pdf);
+                if (r.overflow) atomicAdd(&w.cnt[2], 1u);
+                slot = kDone;
+            }
+            while (found < (uint32_t)__popcll(idle) && next < end) {
+                const uint32_t e = next + __lane_id();
+                const uint32_t k = e < end ? w.skey[e] : a.sc.n_mats;
+                const bool layered = k < a.sc.n_mats && (lds_mats ? smats[k] : a.sc.mats[k]).n_layers > 1;
+                const uint64_t lm = __ballot(layered);
+                if (layered) list[found + (uint32_t)__popcll(lm & lt)] = e;
+                found += (uint32_t)__popcll(lm);
+                next += 64;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (!walking) {
+                const uint32_t q = (uint32_t)__popcll(idle & lt);
+                if (q < found) {
+                    slot = list[found - 1 - q];
+                    mid = w.skey[slot];
+                    const float4 hv = w.hit[slot], o4 = A.o[slot], d4 = A.d[slot];
+                    const uint32_t k = __float_as_uint(A.thr[slot].w);
+                    r = make_draws(job_of<MULTI>(a, __float_as_uint(d4.w)), A.key[slot], k);
+                    V3 pos, nrm, wo;
+                    Frame fr;
+                    path_vertex(a, V3{o4.x, o4.y, o4.z}, V3{d4.x, d4.y, d4.z}, hv, pos, nrm, fr, wo);
+                    park[0][threadIdx.x] = pos.x;
+                    park[1][threadIdx.x] = pos.y;
+                    park[2][threadIdx.x] = pos.z;
+                    park[3][threadIdx.x] = nrm.x;
+                    park[4][threadIdx.x] = nrm.y;
+                    park[5][threadIdx.x] = nrm.z;
+                    const spt_material& mm = lds_mats ? smats[mid] : a.sc.mats[mid];
+                    wk.start(mm, wo);
+                    walking = wk.running(mm);
+                }
+            }
+            found -= min(found, (uint32_t)__popcll(idle));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (!__ballot(slot != kDone)) break;
+        }
+        const spt_material& m = lds_mats ? smats[mid] : a.sc.mats[mid];
+        const bool coat = walking && m.layers[wk.id].type == SPT_BSDF_SMOOTH_DIELECTRIC;
+        const bool coats = 2 * __popcll(__ballot(coat)) >= __popcll(__ballot(walking));
+        if (walking && coat == coats) {
+            wk.step(m, r);
+            walking = wk.running(m);
+        }
+    }
+}
+
 // Shading of one bounce (integrators/pathtracer.cpp:21-54) for every live
-// path of A, in material order when sorted; survivors are appended to B, with
-// one atomic on B's count per block and 256 paths: one per wave (the
-// compiler's aggregation) made that address the limit, about 10 ns per atomic
-// that all XCDs share (61M paths: 950k atomics in a 10.2-ms launch).
-// GUIDED instantiates the guide's sampling and record capture; the plain
-// instantiation carries none of their registers. Four waves per SIMD (128
-// VGPRs, a few spills) measured 2% faster than the two the register count
-// allows: the kernel waits on gathers from a path queue no cache holds.
+// path of A, in the queue's order; survivors are appended to B, with one atomic
+// on B's count per block and 256 paths: one per wave (the compiler's
+// aggregation) made that address the limit, about 10 ns per atomic that all
+// XCDs share (61M paths: 950k atomics in a 10.2-ms launch).
+// GUIDED instantiates the guide's sampling and record capture and walks in
+// place (a bounce's launches are shorter there, and a launch more costs the
+// length of its longest walk, 60 us); the plain instantiation carries none of
+// their registers and leaves layered materials to k_walk. Bound by the queue's
+// traffic, about 210 B a path (28M paths 1.37 ms, 4.4 TB/s); five or six waves
+// per SIMD instead of four do not change that (1.40, 1.56 ms).
 template <bool MULTI, bool GUIDED>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_shade(RenderArgs a, PathBuf A, PathBuf B, Work w,
                                                   const uint32_t* __restrict__ cntA, uint32_t* __restrict__ cntB) {
@@ -889,7 +906,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                        // across the barriers would spill 72 VGPRs instead of 22, which costs guided
                        // passes as much as the shared address
             if (j < n)
-                shade_path<MULTI, GUIDED>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& sv) {
+                shade_path<MULTI, true, true>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& sv) {
                     store_survivor<GUIDED>(a, B, sv, atomicAdd(cntB, 1u));
                 });
             continue;
@@ -897,7 +914,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         Survivor sv;
         bool alive = false;
         if (j < n)
-            shade_path<MULTI, GUIDED>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& next) {
+            shade_path<MULTI, false, false>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& next) {
                 sv = next;
                 alive = true;
             });
@@ -932,7 +949,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // latency of those chains; the path state and hits stay in the queue's arrays,
 // read back from the caches. 128 VGPRs and 36 KB of LDS: four blocks a CU.
 // 97x61 box image, 1 sample: 590 -> 150 us; 800x600 mesh image, 4 samples,
-// where it takes the bounces from the eighth on: 6.1 -> 4.4 ms.
+// where it takes the bounces from the seventh on: 6.1 -> 4.4 ms.
 template <bool MULTI>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_finish(
     RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA, uint32_t* __restrict__ spill,
@@ -951,7 +968,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     if (MULTI)
         for (uint32_t k = threadIdx.x; k < kDoneJobs; k += kBlock) done[k] = 0;
     __syncthreads();
-    a.keys = 0;  // slots are shaded in place, not in material order
     const uint32_t n = *cntA;
     const uint32_t waves = gridDim.x * (kBlock / 64);
     const uint32_t share = (n + waves - 1) / waves;
@@ -1001,7 +1017,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         if (slot != kDone) {
             bool alive = false;
             longest = max(longest, ++segments);
-            shade_path<MULTI, false>(a, A, w, smats, lds_mats, slot, done, [&](const Survivor& sv) {
+            shade_path<MULTI, false, true>(a, A, w, smats, lds_mats, slot, done, [&](const Survivor& sv) {
                 store_survivor<false>(a, A, sv, slot);
                 alive = true;
             });
@@ -1132,7 +1148,7 @@ template <bool MULTI>
 spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuning& tn, spt_render_stats& stats) {
     uint64_t cap = std::min<uint64_t>(total, tn.path_capacity);
     auto state_bytes = [](uint64_t c) {
-        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + (size_t)kMaxSortKeys * (kMaxSortBlocks + 1) * 4 + 8192;
+        return (size_t)c * (2 * kBufBytes + kWorkBytes + 4 * 8) + 8192;
     };
     if (state_bytes(cap) > ctx->paths_bytes) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -1170,9 +1186,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     Work w;
     w.hit = (float4*)take(cap * 16);
     w.skey = (uint32_t*)take(cap * 4);
-    w.perm = (uint32_t*)take(cap * 4);
-    w.bhist = (uint32_t*)take((size_t)kMaxSortKeys * kMaxSortBlocks * 4);
-    w.btotal = (uint32_t*)take((size_t)kMaxSortKeys * 4);
+    w.walk = (float2*)take(cap * 8);
     w.cnt = (uint32_t*)take((64 + kRayCounterWords) * 4);
     w.rays = w.cnt + 64;
     if ((size_t)(base - reinterpret_cast<char*>(ctx->d_paths)) > ctx->paths_bytes)
@@ -1205,10 +1219,8 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         per_cu = std::min<int>(per_cu, tn.wavefronts == 2 ? 5 : 4);
     const uint32_t ext_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)(per_cu * ctx->num_cus));
     const uint32_t shade_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * tn.shade_blocks_per_cu);
+    const uint32_t walk_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * 4);
     const uint32_t refill_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * 8);
-    // sort chunks: many (latency hiding) unless many keys would make the scan long
-    const uint32_t sort_blocks =
-        a.keys ? std::max<uint32_t>(1024, std::min<uint32_t>(kMaxSortBlocks, 16384 / a.keys)) : 256;
     hipStream_t st = ctx->stream;
     const bool timed = (a.flags & SPT_RENDER_TIME_KERNELS) != 0;
     const bool fetch_stats = (a.flags & SPT_RENDER_FETCH_STATS) != 0;
@@ -1260,11 +1272,6 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
             (void)hipEventRecord(ctx->tev[2 * stats.extend_launches + 1], st);
             ++stats.extend_launches;
         }
-        if (a.keys) {
-            hipLaunchKernelGGL(k_hist, dim3(sort_blocks), dim3(kBlock), 0, st, a, w, cntA);
-            hipLaunchKernelGGL(k_scan, dim3(a.keys), dim3(kBlock), 0, st, a, w, sort_blocks, cntA);
-            hipLaunchKernelGGL(k_scatter, dim3(sort_blocks), dim3(kBlock), 0, st, a, w, cntA);
-        }
         if (a.guided) {
             if (timed) {
                 hipEvent_t e0, e1;
@@ -1278,10 +1285,8 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
                                st, a, A, w, cntA, a.theta, a.wbf, a.gbox);
             if (timed && !gev.empty()) (void)hipEventRecord(gev.back(), st);
         }
-        if (a.guided)
-            hipLaunchKernelGGL((k_shade<MULTI, true>), dim3(shade_grid), dim3(kBlock), 0, st, a, A, B, w, cntA, cntB);
-        else
-            hipLaunchKernelGGL((k_shade<MULTI, false>), dim3(shade_grid), dim3(kBlock), 0, st, a, A, B, w, cntA, cntB);
+        if (a.walk) hipLaunchKernelGGL((k_walk<MULTI>), dim3(walk_grid), dim3(kBlock), 0, st, a, A, w, cntA);
+        hipLaunchKernelGGL((a.guided ? k_shade<MULTI, true> : k_shade<MULTI, false>), dim3(shade_grid), dim3(kBlock), 0, st, a, A, B, w, cntA, cntB);
         // regeneration: the survivors' buffer is topped up with new camera paths
         hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, cntA, cntB, w.cnt, w.rays, (uint32_t)cap, total, ctx->d_status,
                            a.job_clock);
@@ -1428,9 +1433,9 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         const uint32_t* c = cnt + 64 + k * kRayCounterStride;
         stats.rays += (uint64_t)c[kFinishRays] | ((uint64_t)c[kFinishRays + 1] << 32);
         longest = std::max(longest, c[kFinishBounces]);
+        stats.guide_queries += (uint64_t)c[kGuideQueries] | ((uint64_t)c[kGuideQueries + 1] << 32);
     }
     stats.bounces += longest;
-    stats.guide_queries = (uint64_t)cnt[30] | ((uint64_t)cnt[31] << 32);
     if (timed) {
         for (uint64_t i = 0; i < stats.extend_launches; ++i) {
             float ms = 0.0f;
@@ -1464,12 +1469,11 @@ spt_status run_fronts(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tun
     spt_tuning t1 = tn;
     uint32_t k = std::max<uint32_t>(1, std::min<uint32_t>(4, tn.wavefronts));
     if (a.rec_ring) k = 1;  // in-call training trains from one wavefront's ring
-    // a plain render of one scene runs as one wavefront unless the caller asks
-    // for more: its traversal and shading each fill the chip (800x600, 256
-    // spp: 132 ms on one, 138 on three; 1024 spp 506 and 548); guided passes
-    // and batches keep a gain of 2-6% (64-spp guided pass 66.6 against 67.8
-    // ms, 12 scenes 69.0 against 72.2 ms)
-    if (!MULTI && !a.guided && ctx->tuning.wavefronts == 0) k = 1;
+    // one wavefront unless the caller asks for more: its traversal and shading
+    // each fill the chip, and with other streams in the process several lose
+    // (1, 2, 3 of them: guided 800x600, 64 spp 63.9, 74.7, 72.5 ms, 400x300,
+    // 36 spp 11.5, 11.4, 11.6; batch of 12 scenes 59.3, 64.5, 66.3)
+    if (ctx->tuning.wavefronts == 0) k = 1;
     while (k > 1 && total / k < (1ull << 21)) --k;
     if (k == 1) {
         t1.wavefronts = 1;
@@ -1612,8 +1616,7 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
             (uint32_t)std::min<double>(1 << 30, std::max(1.0, std::ceil(want / ctx->guide.records_cap)));
     }
     a.rec_stride = ctx->guide.rec_stride;
-    const uint32_t keys = ctx->n_mats + 1;
-    a.keys = (!(prm->flags & SPT_RENDER_NO_SORT) && keys <= kMaxSortKeys) ? keys : 0u;
+    a.walk = ctx->layered && !a.guided;
     spt_render_stats stats{};
     stats.paths = total;
     s = run_fronts<false>(ctx, a, total, resolve_tuning(ctx->tuning), stats);
@@ -1720,8 +1723,7 @@ spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
     a.job_clock = b.d_clock;
     a.flags = 0;
     for (const Job& jb : jobs) a.per_path |= jb.path_rgb ? 1u : 0u;
-    const uint32_t keys = b.n_mats + 1;
-    a.keys = keys <= kMaxSortKeys ? keys : 0u;
+    a.walk = b.layered;
     spt_render_stats stats{};
     stats.paths = total;
     s = run_fronts<true>(ctx, a, total, tn, stats);

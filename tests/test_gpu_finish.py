@@ -91,3 +91,32 @@ def test_batches(device):
         _, paths0, _ = _render(device, sc, L.SPT_RENDER_TIME_KERNELS)
         assert _same_bits(b.path_radiance(i), paths0)
     b.close()
+
+
+def test_batch_of_layered_scenes(device):
+    scs = [scenes.mesh_in_box(rings=16 + 4 * k, segments=32 + 8 * k, width=500 + 30 * k, height=300, spp=4, seed=k)
+           for k in range(3)]
+    b = api.Batch(device, scs, per_path=True)
+    b.render()
+    for i, sc in enumerate(scs):
+        _, paths0, _ = _render(device, sc, L.SPT_RENDER_TIME_KERNELS)
+        assert _same_bits(b.path_radiance(i), paths0)
+    b.close()
+
+
+def test_layered_materials_outside_the_table(device):
+    """60 materials (read from memory, not LDS), all layered, in calls of bounces."""
+    sc = scenes.mesh_in_box(rings=24, segments=48, width=400, height=400, spp=9)
+    n0 = len(sc.materials)
+    rng = np.random.default_rng(3)
+    layered = next(m for m in sc.materials if m.n_layers > 1)
+    sc.materials = list(sc.materials) + [layered] * (60 - n0)
+    ids = np.array(sc.mat_ids)
+    k = next(i for i, m in enumerate(sc.materials) if m.n_layers > 1)
+    ids[ids == k] = rng.choice([k] + list(range(n0, 60)), size=int((ids == k).sum()))
+    ref = scenes.mesh_in_box(rings=24, segments=48, width=400, height=400, spp=9)
+    _, want, _ = _render(device, ref, 0)
+    sc.mat_ids = ids.astype(sc.mat_ids.dtype)
+    for flags in (0, L.SPT_RENDER_TIME_KERNELS):
+        _, paths, _ = _render(device, sc, flags)
+        assert _same_bits(paths, want)
