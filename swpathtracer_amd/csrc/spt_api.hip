@@ -34,7 +34,7 @@ spt_status stream_wait(spt_ctx* ctx, const char* what) {
 
 spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what, void* dst2,
                       const void* d_src2, size_t bytes2) {
-    if (bytes + bytes2 > 4096 || !ctx->h_pin) return set_error(ctx, SPT_ERR_INVALID, "read_small: more than 4 KiB");
+    if (bytes + bytes2 > kPinBytes || !ctx->h_pin) return set_error(ctx, SPT_ERR_INVALID, "read_small: more than 64 KiB");
     char* pin = static_cast<char*>(ctx->h_pin);
     spt_status s = check_hip(ctx, hipMemcpyAsync(pin, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
     if (s == SPT_OK && bytes2)
@@ -462,7 +462,7 @@ spt_status spt_create(int device, spt_ctx** out) {
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
         ctx->wall_clock_khz = khz;
-    if (hipHostMalloc(&ctx->h_pin, 4096, hipHostMallocDefault) != hipSuccess) ctx->h_pin = nullptr;
+    if (hipHostMalloc(&ctx->h_pin, kPinBytes, hipHostMallocDefault) != hipSuccess) ctx->h_pin = nullptr;
     if (!ctx->h_pin || hipMalloc(&ctx->d_flags, 64) != hipSuccess || hipMemset(ctx->d_flags, 0, 64) != hipSuccess) {
         if (ctx->h_pin) (void)hipHostFree(ctx->h_pin);
         (void)hipStreamDestroy(ctx->stream);

@@ -320,12 +320,9 @@ struct GuideState {
     double cand_per_path = 0.0;   // candidate vertices per path of the last training render
     uint64_t candidates = 0;      // candidate vertices of the last training render
     double kernel_ms = 0.0;       // device time of the training kernels (settled steps)
-    // training scratch, feature-major (feature f of sample s at f * rows + s):
-    // x^T bf16 [32], h1..h3^T bf16 [64] each, dy^T f32 [48], dz3..dz1^T bf16
-    // [64] each, then per-split partial gradients f32 [splits][params]
+    // training scratch: the partial gradients of the training kernel's blocks, f32 [blocks][params]
     char* d_scratch = nullptr;
     size_t scratch_bytes = 0;
-    uint32_t scratch_rows = 0;
     std::vector<hipEvent_t> ev_free, ev_pending;  // event pairs around training kernels
 
     GuideCtl* ctl() const { return reinterpret_cast<GuideCtl*>(d_acc); }
@@ -407,7 +404,7 @@ struct spt_ctx {
     spt::GuideState guide;
     spt_tuning tuning{};  // zero fields: defaults
     int wall_clock_khz = 100000;
-    void* h_pin = nullptr;  // 4 KiB of pinned host memory for small read-backs
+    void* h_pin = nullptr;  // kPinBytes of pinned host memory for small read-backs
     // mapped host memory the bounce loop reports its progress to (see k_plan)
     volatile uint32_t* h_status = nullptr;
     uint32_t* d_status = nullptr;
@@ -454,8 +451,9 @@ spt_material prepare_material(const spt_material& m);
 // Waits for the context stream by polling it (no blocking wait on an
 // interrupt: those have been seen to wake up hundreds of ms late).
 spt_status stream_wait(spt_ctx* ctx, const char* what);
-// Copies up to 4 KiB, from one or two places, from the device through pinned
+// Copies up to 64 KiB, from one or two places, from the device through pinned
 // memory and waits once.
+constexpr size_t kPinBytes = 64 * 1024;
 spt_status read_small(spt_ctx* ctx, void* dst, const void* d_src, size_t bytes, const char* what, void* dst2 = nullptr,
                       const void* d_src2 = nullptr, size_t bytes2 = 0);
 // grows ctx->d_spill to hold `words` entries; returns false on failure

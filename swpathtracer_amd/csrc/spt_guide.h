@@ -29,13 +29,12 @@ typedef short bf16x8s __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// round-to-nearest-even float -> bfloat16 bits, and back
+// round-to-nearest-even float -> bfloat16 bits
 __device__ inline unsigned short f2bf(float x) {
     uint32_t u = __float_as_uint(x);
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (unsigned short)(u >> 16);
 }
-__device__ inline float bf2f(unsigned short b) { return __uint_as_float((uint32_t)b << 16); }
 
 // Input encoding (32): x = (p - bmin) / bext clamped to [0,1]; sin/cos of
 // 2 pi 2^k x_c for k = 0..2; n; wo; one-blob (4 Gaussian bins, sigma 1/4) of
@@ -70,30 +69,6 @@ __device__ inline void encode(V3 p, V3 n, V3 wo, const float* bmin, const float*
     f[31] = 1.0f;
 }
 
-// Block-shared weights: bf16 copies of W1..W4 and fp32 biases.
-struct SharedWeights {
-    unsigned short w1[kHid * kEnc];
-    unsigned short w2[kHid * kHid];
-    unsigned short w3[kHid * kHid];
-    unsigned short w4[kOutP * kHid];
-    float b1[kHid], b2[kHid], b3[kHid], b4[kOutP];
-};
-
-__device__ inline void load_weights(SharedWeights& s, const unsigned short* wbf, const float* theta) {
-    for (int i = threadIdx.x; i < kHid * kEnc; i += blockDim.x) s.w1[i] = wbf[kW1 + i];
-    for (int i = threadIdx.x; i < kHid * kHid; i += blockDim.x) {
-        s.w2[i] = wbf[kW2 + i];
-        s.w3[i] = wbf[kW3 + i];
-    }
-    for (int i = threadIdx.x; i < kOutP * kHid; i += blockDim.x) s.w4[i] = wbf[kW4 + i];
-    for (int i = threadIdx.x; i < kHid; i += blockDim.x) {
-        s.b1[i] = theta[kB1 + i];
-        s.b2[i] = theta[kB2 + i];
-        s.b3[i] = theta[kB3 + i];
-    }
-    for (int i = threadIdx.x; i < kOutP; i += blockDim.x) s.b4[i] = theta[kB4 + i];
-}
-
 // 4 consecutive bf16 of an LDS row as an MFMA operand
 __device__ inline bf16x4 ld4(const unsigned short* p) {
     const uint2 v = *reinterpret_cast<const uint2*>(p);
@@ -104,16 +79,6 @@ __device__ inline bf16x4 ld4(const unsigned short* p) {
     r[3] = (short)(v.y >> 16);
     return r;
 }
-// 4 bf16 with a stride
-__device__ inline bf16x4 ld4s(const unsigned short* p, int stride) {
-    bf16x4 r;
-    r[0] = (short)p[0];
-    r[1] = (short)p[stride];
-    r[2] = (short)p[2 * stride];
-    r[3] = (short)p[3 * stride];
-    return r;
-}
-
 // Operand layout of the data (wave64), lane l, r = l % 16, g = l / 16, per
 // 16-wide k-tile:
 //   A (16 rows x 16 k):  A[r][4g + j]         j = 0..3
@@ -123,7 +88,7 @@ __device__ inline bf16x4 ld4s(const unsigned short* p, int stride) {
 // lane (r, g) multiplies element e of lane (c, g) for every e, and all 32
 // products per (row, col) are summed. k is only a summation index, so two
 // k-tiles are fed as one by concatenating the lane's 4 values of tile k and
-// of tile k + 1 in A and in B alike (mfma_k32).
+// of tile k + 1 in A and in B alike (mfma_w).
 // ---------------------------------------------------------------------------
 // Register-resident forward pass ("column" form): the layer is computed as
 // out^T = W * in^T, weights as the MFMA A operand (from LDS) and 16 samples as
@@ -154,18 +119,6 @@ __device__ inline bf16x4 pack_relu(f32x4 v) {
 }
 
 __device__ inline f32x4 bias4(const float* b) { return f32x4{b[0], b[1], b[2], b[3]}; }
-
-// D += A B over two 16-wide k-tiles (a0, b0: tile k; a1, b1: tile k + 1).
-__device__ inline f32x4 mfma_k32(bf16x4 a0, bf16x4 a1, bf16x4 b0, bf16x4 b1, f32x4 c) {
-    const bf16x8s a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-    const bf16x8s b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-}
-// D += A B over one 16-wide k-tile (the odd tile of a 48-wide reduction).
-__device__ inline f32x4 mfma_k16(bf16x4 a, bf16x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
 
 // Inference weights in MFMA A-operand order. For a layer of IN inputs, output
 // tile t and k-tile pair p (tiles 2p and 2p + 1) one 1-KB block holds, for
@@ -406,37 +359,6 @@ __device__ inline V3 mixture_sample(const Lobe L[kLobes], float u0, float u1, fl
     V3 t, b;
     basis(L[k].mu, t, b);
     return t * (st * cosf(ph)) + b * (st * sinf(ph)) + L[k].mu * w;
-}
-
-// Gradient of -W log q(d) w.r.t. the 40 raw outputs (dy[40..47] = 0).
-__device__ inline float loss_grad(const float* y, V3 d, float W, float* dy) {
-    Lobe L[kLobes];
-    mixture_params(y, L);
-    float lv[kLobes];
-    float m = -3.0e38f;
-    for (int i = 0; i < kLobes; ++i) {
-        lv[i] = L[i].logw + log_vmf(L[i], d);
-        m = fmaxf(m, lv[i]);
-    }
-    float sum = 0.0f;
-    for (int i = 0; i < kLobes; ++i) sum += expf(lv[i] - m);
-    const float logq = m + logf(sum);
-    for (int i = 0; i < kLobes; ++i) {
-        const float r = expf(lv[i] - logq);
-        const float w = expf(L[i].logw);
-        const float c = dot(L[i].mu, d);
-        dy[5 * i + 4] = -W * (r - w);
-        const float kap = L[i].kappa;
-        const float dlv = 1.0f - 2.0f * kap / expm1f(2.0f * kap) + kap * (c - 1.0f);
-        dy[5 * i + 3] = L[i].inside ? -W * r * dlv : 0.0f;
-        const V3 gmu = d * (-W * r * kap);
-        const V3 proj = (gmu - L[i].mu * dot(gmu, L[i].mu)) * (1.0f / L[i].norm);
-        dy[5 * i + 0] = proj.x;
-        dy[5 * i + 1] = proj.y;
-        dy[5 * i + 2] = proj.z;
-    }
-    for (int i = kOut; i < kOutP; ++i) dy[i] = 0.0f;
-    return -W * logq;
 }
 
 }  // namespace guide

@@ -47,284 +47,370 @@ __global__ __launch_bounds__(kBlock) void k_guide_eval(const float* __restrict__
     }
 }
 
-// Sum of the record weights (for the batch-mean normalisation).
+// Sum of the record weights (for the batch-mean normalisation), one atomic
+// per block.
 __global__ __launch_bounds__(kBlock) void k_guide_wsum(const float* __restrict__ rec, uint32_t n, uint32_t rs,
                                                        float* __restrict__ acc) {
+    __shared__ float part[kBlock / 64];
     float s = 0.0f;
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
         s += rec[(size_t)i * rs * kRecord + 12];
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (__lane_id() == 0) atomicAdd(acc, s);
+    if (__lane_id() == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(acc, (part[0] + part[1]) + (part[2] + part[3]));
 }
 
 // ---------------------------------------------------------------------------
-// Training step in four stages over a feature-major scratch (feature f of
-// sample s at f * rows + s): forward + loss gradient, backward through the
-// activations, weight gradients as split-K MFMA products, reduction.
+// The gradient of a training batch in one kernel: a block takes tiles of 128
+// records through encoding, forward pass, loss gradient and backward pass and
+// adds the weight gradients up in its accumulators, which it writes once.
+// Nothing but the records is read and nothing but a partial gradient written:
+// activations and their gradients as bf16 lie in LDS, feature-major, so that
+// a weight gradient dW[o][k] = sum_s dz[o][s] in[k][s] reads both of its MFMA
+// operands as 16-B rows of samples. LDS (150 KB of 160) allows one block of
+// eight waves a CU: a wave owns 16 samples of a tile in the passes (column
+// form, as in inference) and one or two 16 x 16 tiles of each layer's gradient.
+// The loss gradient of a record takes four lanes, two lobes each.
+//
+// 262,144 records: 75 us; as three kernels with all of that in global memory
+// (0.5 GB written and read again) 342 us. Bound by the chain of a tile's
+// stages at two waves a SIMD.
 // ---------------------------------------------------------------------------
-struct TrainScratch {
-    unsigned short* xT;   // [32][rows]
-    unsigned short* h1T;  // [64][rows]
-    unsigned short* h2T;
-    unsigned short* h3T;
-    float* dyT;           // [48][rows], rows 40..47 stay zero
-    unsigned short* dz3T; // [64][rows]
-    unsigned short* dz2T;
-    unsigned short* dz1T;
-    float* partial;       // [splits][kParams]
-    uint32_t rows;
+constexpr int kTrainTile = 128, kTrainBlock = 512, kTrainRow = kTrainTile + 8;  // 272 B: 16 rows on distinct banks
+
+struct TrainLds {
+    FwdWeights fw;
+    // W2^T, W3^T, W4^T as MFMA operands of the backward pass (as in FwdWeights,
+    // rows = inputs; W4 with 16 more outputs of weight 0: a v_mfma 16x16x16
+    // issued right behind the 16x16x32 whose result it adds to gave wrong rows)
+    uint4 w2t[4 * 2 * 64], w3t[4 * 2 * 64], w4t[4 * 2 * 64];
+    unsigned short x[2][kEnc][kTrainRow];  // two tiles in turn
+    unsigned short h1[kHid][kTrainRow], h2[kHid][kTrainRow], h3[kHid][kTrainRow];
+    unsigned short dy[kOutP][kTrainRow];   // rows 40..47 stay zero
+    union {
+        float y[kTrainTile][kOut + 1];
+        unsigned short dz[kHid][kTrainRow];
+    };
 };
 
-__device__ inline bf16x4 cvt4(float a, float b, float c, float d) {
-    bf16x4 r;
-    r[0] = (short)f2bf(a);
-    r[1] = (short)f2bf(b);
-    r[2] = (short)f2bf(c);
-    r[3] = (short)f2bf(d);
-    return r;
+__device__ inline bf16x8 bf8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+// D += A B, 32 samples from s0 on as the reduction axis: rows o0 + r of T and
+// rows k0 + r of U.
+__device__ inline f32x4 mfma_rows(const unsigned short (*T)[kTrainRow], int o0, const unsigned short (*U)[kTrainRow],
+                                  int k0, int s0, f32x4 c) {
+    const int r = __lane_id() & 15, g = __lane_id() >> 4;
+    const uint4 a = *reinterpret_cast<const uint4*>(&T[o0 + r][s0 + 8 * g]);
+    const uint4 b = *reinterpret_cast<const uint4*>(&U[k0 + r][s0 + 8 * g]);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(a), bf8(b), c, 0, 0, 0);
+}
+// The same with B = 1: every column of D gets the sums of the rows of T.
+__device__ inline f32x4 mfma_row_sums(const unsigned short (*T)[kTrainRow], int o0, int s0, f32x4 c) {
+    const int r = __lane_id() & 15, g = __lane_id() >> 4;
+    const uint4 a = *reinterpret_cast<const uint4*>(&T[o0 + r][s0 + 8 * g]);
+    const uint32_t ones = 0x3F803F80u;
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(a), bf8(make_uint4(ones, ones, ones, ones)), c, 0, 0, 0);
 }
 
-// feature-major bf16 column: features f0 + i (i = 0..3) of sample s
-__device__ inline bf16x4 ld_col4(const unsigned short* T, uint32_t rows, uint32_t f0, uint32_t s) {
-    bf16x4 r;
-    r[0] = (short)T[(size_t)f0 * rows + s];
-    r[1] = (short)T[(size_t)(f0 + 1) * rows + s];
-    r[2] = (short)T[(size_t)(f0 + 2) * rows + s];
-    r[3] = (short)T[(size_t)(f0 + 3) * rows + s];
-    return r;
+// Features f0 + 0..3 of sample s.
+__device__ inline bf16x4 ld_col4(const unsigned short (*T)[kTrainRow], int f0, int s) {
+    return bf16x4{(short)T[f0][s], (short)T[f0 + 1][s], (short)T[f0 + 2][s], (short)T[f0 + 3][s]};
+}
+__device__ inline void st_col4(unsigned short (*T)[kTrainRow], int f0, int s, bf16x4 v) {
+    T[f0][s] = (unsigned short)v[0];
+    T[f0 + 1][s] = (unsigned short)v[1];
+    T[f0 + 2][s] = (unsigned short)v[2];
+    T[f0 + 3][s] = (unsigned short)v[3];
+}
+// Gradients through the ReLU whose outputs are h, as bf16.
+__device__ inline bf16x4 relu_grad(f32x4 v, bf16x4 h) {
+    for (int i = 0; i < 4; ++i)
+        if (h[i] <= 0) v[i] = 0.0f;  // the sign of a bf16 is that of its bits
+    return __builtin_bit_cast(bf16x4, (u32x2){pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])});
 }
 
-__device__ inline void st_col4(unsigned short* T, uint32_t rows, uint32_t f0, uint32_t s, bf16x4 v) {
-    T[(size_t)f0 * rows + s] = (unsigned short)v[0];
-    T[(size_t)(f0 + 1) * rows + s] = (unsigned short)v[1];
-    T[(size_t)(f0 + 2) * rows + s] = (unsigned short)v[2];
-    T[(size_t)(f0 + 3) * rows + s] = (unsigned short)v[3];
+// W^T of a row-major layer of 64 inputs as MFMA operands: block (t, p) holds
+// for lane r + 16 g W[32 p + 4 g + 0..3][16 t + r] and W[32 p + 16 + 4 g + 0..3][16 t + r].
+// Rows from `rows` on count as 0.
+__device__ inline void transpose_layer(uint4* dst, const unsigned short* w, int rows) {
+    for (int i = threadIdx.x; i < 4 * 2 * 64; i += blockDim.x) {
+        const int l = i & 63, p = (i >> 6) & 1, t = i >> 7;
+        uint32_t v[4];
+        for (int k = 0; k < 4; ++k) {
+            const int row = 32 * p + 4 * (l >> 4) + (k >> 1) * 16 + (k & 1) * 2;
+            const unsigned short* c = w + row * kHid + 16 * t + (l & 15);
+            v[k] = row < rows ? (uint32_t)c[0] | ((uint32_t)c[kHid] << 16) : 0u;
+        }
+        dst[i] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
 }
 
-// A operand of W^T for the backward pass: A[r][4g + j] = W[16 ot + 4g + j][16 kt + r]
-__device__ inline bf16x4 ld_wT(const unsigned short* W, int K, int ot, int kt) {
-    const int l = __lane_id(), r = l & 15, g = l >> 4;
-    return ld4s(W + (16 * ot + 4 * g) * K + 16 * kt + r, K);
+// Sum and maximum over the four lanes of a quad.
+template <int CTRL>
+__device__ inline float quad_swap_f(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xF, 0xF, true));
+}
+__device__ inline float quad_sum(float v) {
+    v += quad_swap_f<0xB1>(v);
+    return v + quad_swap_f<0x4E>(v);
+}
+__device__ inline float quad_max(float v) {
+    v = fmaxf(v, quad_swap_f<0xB1>(v));
+    return fmaxf(v, quad_swap_f<0x4E>(v));
 }
 
-// Stage 1: encode, forward (activations stored feature-major), and each
-// record's loss gradient w.r.t. the 48 raw outputs, scaled by loss_scale / n
-// (rows n..rows16: zero gradient). One block = 256 records, lane = record.
-__global__ __launch_bounds__(kBlock) void k_train_fwd(const float* __restrict__ theta,
-                                                      const unsigned short* __restrict__ wbf,
-                                                      const float* __restrict__ rec, uint32_t n, uint32_t rs,
-                                                      uint32_t n16, GuideCtl* __restrict__ ctl, GuideBox box,
-                                                      TrainScratch ts) {
+// Gradient of -W log q(d) w.r.t. the 40 raw outputs, by the four lanes of a
+// quad: y and dy are the lane's two lobes (10 outputs); every lane returns the
+// loss.
+__device__ inline float loss_grad_quad(const float y[10], V3 d, float W, float dy[10]) {
+    const float amax = quad_max(fmaxf(y[4], y[9]));
+    const float lse = amax + logf(quad_sum(expf(y[4] - amax) + expf(y[9] - amax)));
+    Lobe L[2];
+    float lv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const V3 raw{y[5 * i], y[5 * i + 1], y[5 * i + 2]};
+        const float nr = sqrtf(dot(raw, raw) + 1e-12f);
+        L[i].mu = raw * (1.0f / nr);
+        L[i].norm = nr;
+        const float s = y[5 * i + 3];
+        const float sc = fminf(fmaxf(s, logf(kKappaMin)), logf(kKappaMax));
+        L[i].inside = (s == sc);
+        L[i].kappa = expf(sc);
+        L[i].logw = y[5 * i + 4] - lse;
+        lv[i] = L[i].logw + log_vmf(L[i], d);
+    }
+    const float m = quad_max(fmaxf(lv[0], lv[1]));
+    const float logq = m + logf(quad_sum(expf(lv[0] - m) + expf(lv[1] - m)));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float r = expf(lv[i] - logq);
+        const float w = expf(L[i].logw);
+        const float c = dot(L[i].mu, d);
+        dy[5 * i + 4] = -W * (r - w);
+        const float kap = L[i].kappa;
+        const float dlv = 1.0f - 2.0f * kap / expm1f(2.0f * kap) + kap * (c - 1.0f);
+        dy[5 * i + 3] = L[i].inside ? -W * r * dlv : 0.0f;
+        const V3 gmu = d * (-W * r * kap);
+        const V3 proj = (gmu - L[i].mu * dot(gmu, L[i].mu)) * (1.0f / L[i].norm);
+        dy[5 * i + 0] = proj.x;
+        dy[5 * i + 1] = proj.y;
+        dy[5 * i + 2] = proj.z;
+    }
+    return -W * logq;
+}
+
+// Gradients of the records' loss, scaled by loss_scale / n, as one partial
+// gradient per block; the loss goes to ctl->loss. Tiles past n count zero.
+__global__ __launch_bounds__(kTrainBlock) void k_train_grad(const float* __restrict__ theta,
+                                                            const unsigned short* __restrict__ wbf,
+                                                            const float* __restrict__ rec, uint32_t n, uint32_t rs,
+                                                            GuideCtl* __restrict__ ctl, GuideBox box,
+                                                            float* __restrict__ partial) {
     extern __shared__ float dyn[];
-    FwdWeights& sw = *reinterpret_cast<FwdWeights*>(dyn);
-    WaveStage* stages = reinterpret_cast<WaveStage*>(reinterpret_cast<char*>(dyn) + sizeof(FwdWeights));
-    float* ystage = reinterpret_cast<float*>(stages + kBlock / 64);  // [4 waves][64][kOut]
-    load_weights(sw, wbf, theta);
+    TrainLds& t = *reinterpret_cast<TrainLds*>(dyn);
+    load_weights(t.fw, wbf, theta);
+    transpose_layer(t.w2t, wbf + kW2, kHid);
+    transpose_layer(t.w3t, wbf + kW3, kHid);
+    transpose_layer(t.w4t, wbf + kW4, kOutP);
+    for (int i = threadIdx.x; i < (kOutP - kOut) * kTrainRow; i += kTrainBlock) t.dy[kOut + i / kTrainRow][i % kTrainRow] = 0;
     const int wave = threadIdx.x >> 6, l = __lane_id(), r = l & 15, g = l >> 4;
-    WaveStage& st = stages[wave];
-    float* ys = ystage + wave * 64 * kOut;
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t wbase = blockIdx.x * kBlock + wave * 64;
-    float f[kEnc];
-    if (s < n) {
-        const float* p = rec + (size_t)s * rs * kRecord;
-        encode(V3{p[0], p[1], p[2]}, V3{p[3], p[4], p[5]}, V3{p[6], p[7], p[8]}, box.bmin, box.bext, f);
-    } else {
-        for (int i = 0; i < kEnc; ++i) f[i] = 0.0f;
-    }
-    stage_row(st, f);
-    if (s < n16)
-        for (int i = 0; i < kEnc; ++i) ts.xT[(size_t)i * ts.rows + s] = f2bf(f[i]);
-    __syncthreads();
-    // forward, column form, 16 records at a time; activations out to scratch
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t sq = wbase + 16 * q + r;
-        const bool keep = sq < n16;
-        const unsigned short* row = st.x + (16 * q + r) * kStageRow;
-        const bf16x4 x[2] = {ld4(row + 4 * g), ld4(row + 16 + 4 * g)};
-        bf16x4 ha[4], hb[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            ha[t] = pack_relu(mfma_w(sw.w1 + 64 * t, x[0], x[1], bias4(sw.b1 + 16 * t + 4 * g)));
-            if (keep) st_col4(ts.h1T, ts.rows, 16 * t + 4 * g, sq, ha[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            f32x4 acc = bias4(sw.b2 + 16 * t + 4 * g);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) acc = mfma_w(sw.w2 + 64 * (2 * t + p), ha[2 * p], ha[2 * p + 1], acc);
-            hb[t] = pack_relu(acc);
-            if (keep) st_col4(ts.h2T, ts.rows, 16 * t + 4 * g, sq, hb[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            f32x4 acc = bias4(sw.b3 + 16 * t + 4 * g);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) acc = mfma_w(sw.w3 + 64 * (2 * t + p), hb[2 * p], hb[2 * p + 1], acc);
-            ha[t] = pack_relu(acc);
-            if (keep) st_col4(ts.h3T, ts.rows, 16 * t + 4 * g, sq, ha[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            f32x4 acc = bias4(sw.b4 + 16 * t + 4 * g);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) acc = mfma_w(sw.w4 + 64 * (2 * t + p), ha[2 * p], ha[2 * p + 1], acc);
-            if (16 * t + 4 * g < kOut)
-                for (int i = 0; i < 4; ++i) ys[(16 * q + r) * kOut + 16 * t + 4 * g + i] = acc[i];
-        }
-    }
-    __syncthreads();
-    // loss gradient of this lane's record
+    const int col = 16 * wave + r;              // this lane's sample of the tile in the passes
+    const int lrec = 16 * wave + (l >> 2), part = l & 3;  // its record and lobe pair in the loss
+    const int ot = wave & 3, half = wave >> 2;  // its tiles of the weight gradients
     const float wmean = fmaxf(ctl->wsum / (float)n, 1e-30f);
     const float scale = ctl->scale / (float)n;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 g4[2] = {zero, zero}, g3[2] = {zero, zero}, g2[2] = {zero, zero}, g1 = zero, b3 = zero, b2 = zero, b1 = zero;
+    float b4[10] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     float loss = 0.0f;
-    if (s < n16) {
-        float dy[kOutP];
-        if (s < n) {
-            const float* p = rec + (size_t)s * rs * kRecord;
-            loss = loss_grad(ys + l * kOut, V3{p[9], p[10], p[11]}, p[12] / wmean, dy);
-        } else {
-            for (int i = 0; i < kOutP; ++i) dy[i] = 0.0f;
+    uint32_t turn = 0;
+    for (uint32_t base = blockIdx.x * kTrainTile; base < n; base += gridDim.x * kTrainTile, turn ^= 1u) {
+        unsigned short(*x)[kTrainRow] = t.x[turn];
+        if (threadIdx.x < kTrainTile) {
+            const uint32_t s = base + threadIdx.x;
+            float f[kEnc];
+            if (s < n) {
+                const float* p = rec + (size_t)s * rs * kRecord;
+                encode(V3{p[0], p[1], p[2]}, V3{p[3], p[4], p[5]}, V3{p[6], p[7], p[8]}, box.bmin, box.bext, f);
+            } else {
+                for (int i = 0; i < kEnc; ++i) f[i] = 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < kEnc; i += 2) {
+                const uint32_t v = pack_bf2(f[i], f[i + 1]);
+                x[i][threadIdx.x] = (unsigned short)v;
+                x[i + 1][threadIdx.x] = (unsigned short)(v >> 16);
+            }
         }
-        for (int o = 0; o < kOut; ++o) ts.dyT[(size_t)o * ts.rows + s] = dy[o] * scale;
+        __syncthreads();  // encoded; the tile before has been read
+        bf16x4 h1[4], h2[4], h3[4];
+        {
+            const bf16x4 x0 = ld_col4(x, 4 * g, col), x1 = ld_col4(x, 16 + 4 * g, col);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                h1[k] = pack_relu(mfma_w(t.fw.w1 + 64 * k, x0, x1, bias4(t.fw.b1 + 16 * k + 4 * g)));
+                st_col4(t.h1, 16 * k + 4 * g, col, h1[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f32x4 acc = bias4(t.fw.b2 + 16 * k + 4 * g);
+#pragma unroll
+                for (int p = 0; p < 2; ++p) acc = mfma_w(t.fw.w2 + 64 * (2 * k + p), h1[2 * p], h1[2 * p + 1], acc);
+                h2[k] = pack_relu(acc);
+                st_col4(t.h2, 16 * k + 4 * g, col, h2[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f32x4 acc = bias4(t.fw.b3 + 16 * k + 4 * g);
+#pragma unroll
+                for (int p = 0; p < 2; ++p) acc = mfma_w(t.fw.w3 + 64 * (2 * k + p), h2[2 * p], h2[2 * p + 1], acc);
+                h3[k] = pack_relu(acc);
+                st_col4(t.h3, 16 * k + 4 * g, col, h3[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                f32x4 acc = bias4(t.fw.b4 + 16 * k + 4 * g);
+#pragma unroll
+                for (int p = 0; p < 2; ++p) acc = mfma_w(t.fw.w4 + 64 * (2 * k + p), h3[2 * p], h3[2 * p + 1], acc);
+                if (16 * k + 4 * g < kOut)
+                    for (int i = 0; i < 4; ++i) t.y[col][16 * k + 4 * g + i] = acc[i];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // a wave reads its own samples' outputs
+        {
+            float y[10], dy[10];
+#pragma unroll
+            for (int i = 0; i < 10; ++i) y[i] = t.y[lrec][10 * part + i];
+            const uint32_t s = base + (uint32_t)lrec;
+            if (s < n) {
+                const float* p = rec + (size_t)s * rs * kRecord;
+                const float v = loss_grad_quad(y, V3{p[9], p[10], p[11]}, p[12] / wmean, dy);
+                loss += part == 0 ? v : 0.0f;
+#pragma unroll
+                for (int i = 0; i < 10; ++i) dy[i] *= scale;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 10; ++i) dy[i] = 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 10; i += 2) {
+                b4[i] += dy[i];
+                b4[i + 1] += dy[i + 1];
+                const uint32_t v = pack_bf2(dy[i], dy[i + 1]);
+                t.dy[10 * part + i][lrec] = (unsigned short)v;
+                t.dy[10 * part + i + 1][lrec] = (unsigned short)(v >> 16);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        bf16x4 z3[4], z2[4], z1[4];  // gradients of the hidden pre-activations
+        {
+            const bf16x4 d0 = ld_col4(t.dy, 4 * g, col), d1 = ld_col4(t.dy, 16 + 4 * g, col),
+                         d2 = ld_col4(t.dy, 32 + 4 * g, col);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f32x4 acc = mfma_w(t.w4t + 64 * (2 * k), d0, d1, zero);
+                acc = mfma_w(t.w4t + 64 * (2 * k + 1), d2, bf16x4{0, 0, 0, 0}, acc);
+                z3[k] = relu_grad(acc, h3[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f32x4 acc = zero;
+#pragma unroll
+                for (int p = 0; p < 2; ++p) acc = mfma_w(t.w3t + 64 * (2 * k + p), z3[2 * p], z3[2 * p + 1], acc);
+                z2[k] = relu_grad(acc, h2[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f32x4 acc = zero;
+#pragma unroll
+                for (int p = 0; p < 2; ++p) acc = mfma_w(t.w2t + 64 * (2 * k + p), z2[2 * p], z2[2 * p + 1], acc);
+                z1[k] = relu_grad(acc, h1[k]);
+            }
+        }
+        __syncthreads();  // activations and dy of the whole tile lie in LDS; y has been read
+#pragma unroll
+        for (int k = 0; k < 4; ++k) st_col4(t.dz, 16 * k + 4 * g, col, z3[k]);
+        if (ot < 3)
+            for (int s0 = 0; s0 < kTrainTile; s0 += 32)
+                for (int k = 0; k < 2; ++k) g4[k] = mfma_rows(t.dy, 16 * ot, t.h3, 16 * (2 * half + k), s0, g4[k]);
+        __syncthreads();  // dz3 is there, h3 has been read
+#pragma unroll
+        for (int k = 0; k < 4; ++k) st_col4(t.h3, 16 * k + 4 * g, col, z2[k]);
+        for (int s0 = 0; s0 < kTrainTile; s0 += 32) {
+            for (int k = 0; k < 2; ++k) g3[k] = mfma_rows(t.dz, 16 * ot, t.h2, 16 * (2 * half + k), s0, g3[k]);
+            if (half == 0) b3 = mfma_row_sums(t.dz, 16 * ot, s0, b3);
+        }
+        __syncthreads();  // dz2 is there (in h3), h2 has been read
+#pragma unroll
+        for (int k = 0; k < 4; ++k) st_col4(t.h2, 16 * k + 4 * g, col, z1[k]);
+        for (int s0 = 0; s0 < kTrainTile; s0 += 32) {
+            for (int k = 0; k < 2; ++k) g2[k] = mfma_rows(t.h3, 16 * ot, t.h1, 16 * (2 * half + k), s0, g2[k]);
+            if (half == 0) b2 = mfma_row_sums(t.h3, 16 * ot, s0, b2);
+        }
+        __syncthreads();  // dz1 is there (in h2)
+        for (int s0 = 0; s0 < kTrainTile; s0 += 32) {
+            g1 = mfma_rows(t.h2, 16 * ot, x, 16 * half, s0, g1);
+            if (half == 0) b1 = mfma_row_sums(t.h2, 16 * ot, s0, b1);
+        }
     }
-    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
-    if (l == 0) atomicAdd(&ctl->loss, loss / (float)n);
-}
-
-// Stage 2: gradients w.r.t. the hidden pre-activations, dz3 = (W4^T dy) . [h3 > 0],
-// dz2 = (W3^T dz3) . [h2 > 0], dz1 = (W2^T dz2) . [h1 > 0], column form, 16
-// records per wave per iteration; stored feature-major as bf16.
-__global__ __launch_bounds__(kBlock) void k_train_bwd(const float* __restrict__ theta,
-                                                      const unsigned short* __restrict__ wbf, uint32_t n16,
-                                                      TrainScratch ts) {
-    extern __shared__ float dyn[];
-    SharedWeights& sw = *reinterpret_cast<SharedWeights*>(dyn);
-    load_weights(sw, wbf, theta);
-    __syncthreads();
-    const int l = __lane_id(), r = l & 15, g = l >> 4;
-    const uint32_t wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), nw = gridDim.x * (kBlock / 64);
-    for (uint32_t base = wave * 16; base < n16; base += nw * 16) {
-        const uint32_t s = base + r;
-        bf16x4 dy[3];
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const float* c = ts.dyT + (size_t)(16 * t + 4 * g) * ts.rows + s;
-            dy[t] = cvt4(c[0], c[ts.rows], c[2 * (size_t)ts.rows], c[3 * (size_t)ts.rows]);
-        }
-        bf16x4 za[4], zb[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {  // dz3: K = 48 outputs
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mfma_k32(ld_wT(sw.w4, kHid, 0, t), ld_wT(sw.w4, kHid, 1, t), dy[0], dy[1], acc);
-            acc = mfma_k16(ld_wT(sw.w4, kHid, 2, t), dy[2], acc);
-            const bf16x4 h = ld_col4(ts.h3T, ts.rows, 16 * t + 4 * g, s);
-            for (int i = 0; i < 4; ++i)
-                if (bf2f((unsigned short)h[i]) <= 0.0f) acc[i] = 0.0f;
-            za[t] = cvt4(acc[0], acc[1], acc[2], acc[3]);
-            st_col4(ts.dz3T, ts.rows, 16 * t + 4 * g, s, za[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {  // dz2
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int k = 0; k < 4; k += 2)
-                acc = mfma_k32(ld_wT(sw.w3, kHid, k, t), ld_wT(sw.w3, kHid, k + 1, t), za[k], za[k + 1], acc);
-            const bf16x4 h = ld_col4(ts.h2T, ts.rows, 16 * t + 4 * g, s);
-            for (int i = 0; i < 4; ++i)
-                if (bf2f((unsigned short)h[i]) <= 0.0f) acc[i] = 0.0f;
-            zb[t] = cvt4(acc[0], acc[1], acc[2], acc[3]);
-            st_col4(ts.dz2T, ts.rows, 16 * t + 4 * g, s, zb[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {  // dz1
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int k = 0; k < 4; k += 2)
-                acc = mfma_k32(ld_wT(sw.w2, kHid, k, t), ld_wT(sw.w2, kHid, k + 1, t), zb[k], zb[k + 1], acc);
-            const bf16x4 h = ld_col4(ts.h1T, ts.rows, 16 * t + 4 * g, s);
-            for (int i = 0; i < 4; ++i)
-                if (bf2f((unsigned short)h[i]) <= 0.0f) acc[i] = 0.0f;
-            st_col4(ts.dz1T, ts.rows, 16 * t + 4 * g, s, cvt4(acc[0], acc[1], acc[2], acc[3]));
-        }
-    }
-}
-
-// 4 consecutive samples s0 .. s0 + 3 of feature f (feature-major bf16 / f32)
-__device__ inline bf16x4 ld_row4(const unsigned short* T, uint32_t rows, uint32_t f, uint32_t s0) {
-    const uint2 v = *reinterpret_cast<const uint2*>(T + (size_t)f * rows + s0);
-    bf16x4 r;
-    r[0] = (short)(v.x & 0xFFFFu);
-    r[1] = (short)(v.x >> 16);
-    r[2] = (short)(v.y & 0xFFFFu);
-    r[3] = (short)(v.y >> 16);
-    return r;
-}
-
-// Stage 3: weight and bias gradients of one layer over one slice of samples:
-// dW[o][k] = sum_s dz[o][s] in[k][s] as MFMA with the samples as the
-// reduction axis (K), db[o] = sum_s dz[o][s]; written to partial[split].
-// Block = (layer, split); wave w takes output tile w.
-__global__ __launch_bounds__(kBlock) void k_train_wgrad(TrainScratch ts, uint32_t n16, uint32_t span) {
-    const int layer = blockIdx.x & 3;  // 0: W1, 1: W2, 2: W3, 3: W4
-    const uint32_t split = blockIdx.x >> 2;
-    const int ot = threadIdx.x >> 6, l = __lane_id(), r = l & 15, g = l >> 4;
-    const int n_ot = layer == 3 ? 3 : 4, n_kt = layer == 0 ? 2 : 4, K = layer == 0 ? kEnc : kHid;
-    if (ot >= n_ot) return;
-    const unsigned short* dz = layer == 0 ? ts.dz1T : layer == 1 ? ts.dz2T : ts.dz3T;
-    const unsigned short* in = layer == 0 ? ts.xT : layer == 1 ? ts.h1T : layer == 2 ? ts.h2T : ts.h3T;
-    const uint32_t s_begin = split * span, s_end = min(n16, s_begin + span);
-    f32x4 acc[4];
-    for (int k = 0; k < 4; ++k) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;
-    // dz of 4 samples s0 + 4 g .. + 3 for output row 16 ot + r (and their bias sum)
-    auto dz4 = [&](uint32_t s0) {
-        bf16x4 a;
-        if (layer == 3) {
-            const float4 v = *reinterpret_cast<const float4*>(ts.dyT + (size_t)(16 * ot + r) * ts.rows + s0 + 4 * g);
-            a = cvt4(v.x, v.y, v.z, v.w);
-            bsum += (v.x + v.y) + (v.z + v.w);
-        } else {
-            a = ld_row4(dz, ts.rows, 16 * ot + r, s0 + 4 * g);
-            bsum += (bf2f((unsigned short)a[0]) + bf2f((unsigned short)a[1])) +
-                    (bf2f((unsigned short)a[2]) + bf2f((unsigned short)a[3]));
-        }
-        return a;
+    // the block's partial gradient
+    float* out = partial + (size_t)blockIdx.x * kParams;
+    auto put = [&](int wofs, int K, int kt, f32x4 v) {
+        for (int i = 0; i < 4; ++i) out[wofs + (16 * ot + 4 * g + i) * K + 16 * kt + r] = v[i];
     };
-    // samples are the reduction axis: 32 per MFMA, a last odd 16 alone
-    uint32_t s0 = s_begin;
-    for (; s0 + 32 <= s_end; s0 += 32) {
-        const bf16x4 a0 = dz4(s0), a1 = dz4(s0 + 16);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k < n_kt)
-                acc[k] = mfma_k32(a0, a1, ld_row4(in, ts.rows, 16 * k + r, s0 + 4 * g),
-                                  ld_row4(in, ts.rows, 16 * k + r, s0 + 16 + 4 * g), acc[k]);
+    for (int k = 0; k < 2; ++k) {
+        if (ot < 3) put(kW4, kHid, 2 * half + k, g4[k]);
+        put(kW3, kHid, 2 * half + k, g3[k]);
+        put(kW2, kHid, 2 * half + k, g2[k]);
     }
-    if (s0 < s_end) {
-        const bf16x4 a = dz4(s0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k < n_kt) acc[k] = mfma_k16(a, ld_row4(in, ts.rows, 16 * k + r, s0 + 4 * g), acc[k]);
+    put(kW1, kEnc, half, g1);
+    if (half == 0 && r == 0)
+        for (int i = 0; i < 4; ++i) {
+            out[kB3 + 16 * ot + 4 * g + i] = b3[i];
+            out[kB2 + 16 * ot + 4 * g + i] = b2[i];
+            out[kB1 + 16 * ot + 4 * g + i] = b1[i];
+        }
+    // output biases and loss: sums over the lanes of one lobe pair, then the waves
+    for (int o = 4; o < 64; o <<= 1) {
+        for (int i = 0; i < 10; ++i) b4[i] += __shfl_xor(b4[i], o);
+        loss += __shfl_xor(loss, o);
     }
-    float* out = ts.partial + (size_t)split * kParams;
-    const int wofs = layer == 0 ? kW1 : layer == 1 ? kW2 : layer == 2 ? kW3 : kW4;
-    const int bofs = layer == 0 ? kB1 : layer == 1 ? kB2 : layer == 2 ? kB3 : kB4;
-    for (int k = 0; k < n_kt; ++k)
-        for (int i = 0; i < 4; ++i) out[wofs + (16 * ot + 4 * g + i) * K + 16 * k + r] = acc[k][i];
-    bsum += __shfl_xor(bsum, 16);
-    bsum += __shfl_xor(bsum, 32);
-    if (g == 0) out[bofs + 16 * ot + r] = bsum;
+    __syncthreads();  // y lies where dz was read
+    if (l < 4) {
+        for (int i = 0; i < 10; ++i) t.y[wave][10 * part + i] = b4[i];
+        if (l == 0) t.y[wave][kOut] = loss;
+    }
+    __syncthreads();
+    if (threadIdx.x <= kOut) {
+        float v = 0.0f;
+        for (int w = 0; w < kTrainBlock / 64; ++w) v += t.y[w][threadIdx.x];
+        if (threadIdx.x < kOut)
+            out[kB4 + threadIdx.x] = v;
+        else
+            atomicAdd(&ctl->loss, v / (float)n);
+    } else if (threadIdx.x < kOutP + 1) {
+        out[kB4 + threadIdx.x - 1] = 0.0f;  // the padding outputs'
+    }
 }
 
-// Stage 4: grad = sum of the split partials (grad holds the scaled gradient).
+// grad = sum of the blocks' partial gradients (grad holds the scaled
+// gradient): 64 parameters a block, four threads each, so that 256 partials
+// are 64 loads deep instead of 256 (5 instead of 64 us).
 __global__ __launch_bounds__(kBlock) void k_train_reduce(const float* __restrict__ partial, uint32_t splits,
                                                          float* __restrict__ grad) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= (uint32_t)kParams) return;
+    __shared__ float part[kBlock / 64][64];
+    const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
     float acc = 0.0f;
-    for (uint32_t sp = 0; sp < splits; ++sp) acc += partial[(size_t)sp * kParams + i];
-    grad[i] = acc;
+    if (i < (uint32_t)kParams) {
+#pragma unroll 8
+        for (uint32_t sp = w; sp < splits; sp += kBlock / 64) acc += partial[(size_t)sp * kParams + i];
+    }
+    part[w][threadIdx.x & 63] = acc;
+    __syncthreads();
+    if (w == 0 && i < (uint32_t)kParams)
+        grad[i] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
 }
 
 // Start of a step: clears the per-step fields of the control block.
@@ -384,19 +470,16 @@ __global__ void k_guide_tobf16(const float* __restrict__ theta, unsigned short* 
 }
 
 size_t eval_lds_bytes() { return sizeof(FwdWeights) + sizeof(WaveStage) * (kBlock / 64); }
-size_t fwd_lds_bytes() {
-    return sizeof(FwdWeights) + sizeof(WaveStage) * (kBlock / 64) + sizeof(float) * 64 * kOut * (kBlock / 64);
-}
 
-// The inference and forward kernels use more than the default 64 KiB of
+// The inference and training kernels use more than the default 64 KiB of
 // dynamic LDS (gfx950 has 160 KiB per CU).
 spt_status allow_lds(spt_ctx* ctx) {
     static bool done = false;
     if (done) return SPT_OK;
     spt_status s = check_hip(ctx,
-                             hipFuncSetAttribute(reinterpret_cast<const void*>(&k_train_fwd),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)fwd_lds_bytes()),
-                             "forward LDS size");
+                             hipFuncSetAttribute(reinterpret_cast<const void*>(&k_train_grad),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(TrainLds)),
+                             "training LDS size");
     if (s == SPT_OK)
         s = check_hip(ctx,
                       hipFuncSetAttribute(reinterpret_cast<const void*>(&k_guide_eval),
@@ -406,68 +489,31 @@ spt_status allow_lds(spt_ctx* ctx) {
     return s;
 }
 
-// Scratch for n16 records (grown on demand; the dy rows 40..47 stay zero).
-spt_status train_scratch(spt_ctx* ctx, uint32_t n16, uint32_t splits, TrainScratch& ts) {
-    GuideState& gs = ctx->guide;
-    const uint32_t rows = (n16 + 63) & ~63u;
-    const size_t per_row = 2 * kEnc + 3 * 2 * kHid + 4 * kOutP + 3 * 2 * kHid;
-    const size_t need = (size_t)rows * per_row + (size_t)splits * kParams * sizeof(float) + 1024;
-    if (rows > gs.scratch_rows || need > gs.scratch_bytes) {
-        spt_status s = stream_wait(ctx, "guide scratch");
-        if (s != SPT_OK) return s;
-        if (gs.d_scratch) (void)hipFree(gs.d_scratch);
-        gs.d_scratch = nullptr;
-        gs.scratch_bytes = 0;
-        gs.scratch_rows = 0;
-        s = check_hip(ctx, hipMalloc(&gs.d_scratch, need), "guide scratch");
-        if (s != SPT_OK) return s;
-        s = check_hip(ctx, hipMemsetAsync(gs.d_scratch, 0, need, ctx->stream), "guide scratch clear");
-        if (s != SPT_OK) return s;
-        gs.scratch_bytes = need;
-        gs.scratch_rows = rows;
-    }
-    const uint32_t R = gs.scratch_rows;
-    char* p = gs.d_scratch;
-    auto take = [&](size_t bytes) {
-        char* q = p;
-        p += (bytes + 255) & ~size_t(255);
-        return q;
-    };
-    ts.xT = reinterpret_cast<unsigned short*>(take((size_t)R * kEnc * 2));
-    ts.h1T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.h2T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.h3T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.dyT = reinterpret_cast<float*>(take((size_t)R * kOutP * 4));
-    ts.dz3T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.dz2T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.dz1T = reinterpret_cast<unsigned short*>(take((size_t)R * kHid * 2));
-    ts.partial = reinterpret_cast<float*>(take((size_t)splits * kParams * 4));
-    ts.rows = R;
-    if ((size_t)(p - gs.d_scratch) > gs.scratch_bytes) return set_error(ctx, SPT_ERR_NOMEM, "guide scratch layout");
-    return SPT_OK;
-}
-
 // Queues the gradient of one step (ctl->wsum and ctl->loss, grad = scaled
 // gradient) on the context stream.
 spt_status queue_gradient(spt_ctx* ctx, const float* d_rec, uint32_t n, uint32_t rs, hipEvent_t e0, hipEvent_t e1) {
     GuideState& gs = ctx->guide;
     hipStream_t st = ctx->stream;
     GuideCtl* ctl = gs.ctl();
-    const uint32_t n16 = (n + 15) & ~15u;
-    const uint32_t span = std::max<uint32_t>(1024, (((n16 + 511) / 512) + 15) & ~15u);
-    const uint32_t splits = (n16 + span - 1) / span;
-    TrainScratch ts;
-    spt_status s = train_scratch(ctx, n16, splits, ts);
-    if (s != SPT_OK) return s;
-    hipLaunchKernelGGL(k_guide_wsum, dim3(256), dim3(kBlock), 0, st, d_rec, n, rs, &ctl->wsum);
+    const uint32_t blocks = std::min<uint32_t>((n + kTrainTile - 1) / kTrainTile, (uint32_t)ctx->num_cus);
+    const size_t need = (size_t)blocks * kParams * sizeof(float);  // the blocks' partial gradients
+    if (need > gs.scratch_bytes) {
+        spt_status s = stream_wait(ctx, "guide scratch");
+        if (s != SPT_OK) return s;
+        if (gs.d_scratch) (void)hipFree(gs.d_scratch);
+        gs.d_scratch = nullptr;
+        gs.scratch_bytes = 0;
+        s = check_hip(ctx, hipMalloc(&gs.d_scratch, need), "guide scratch");
+        if (s != SPT_OK) return s;
+        gs.scratch_bytes = need;
+    }
+    float* partial = reinterpret_cast<float*>(gs.d_scratch);
+    hipLaunchKernelGGL(k_guide_wsum, dim3(std::min<uint32_t>((n + kBlock - 1) / kBlock, 256)), dim3(kBlock), 0, st, d_rec, n,
+                       rs, &ctl->wsum);
     if (e0) (void)hipEventRecord(e0, st);
-    hipLaunchKernelGGL(k_train_fwd, dim3((n16 + kBlock - 1) / kBlock), dim3(kBlock), fwd_lds_bytes(), st, gs.d_theta,
-                       gs.d_wbf, d_rec, n, rs, n16, ctl, guide_box(ctx), ts);
-    hipLaunchKernelGGL(k_train_bwd, dim3(std::min<uint32_t>((n16 + 63) / 64, (uint32_t)ctx->num_cus * 4)), dim3(kBlock),
-                       sizeof(SharedWeights), st, gs.d_theta, gs.d_wbf, n16, ts);
-    hipLaunchKernelGGL(k_train_wgrad, dim3(4 * splits), dim3(kBlock), 0, st, ts, n16, span);
-    hipLaunchKernelGGL(k_train_reduce, dim3((kParams + kBlock - 1) / kBlock), dim3(kBlock), 0, st, ts.partial, splits,
-                       gs.d_grad);
+    hipLaunchKernelGGL(k_train_grad, dim3(blocks), dim3(kTrainBlock), sizeof(TrainLds), st, gs.d_theta, gs.d_wbf, d_rec,
+                       n, rs, ctl, guide_box(ctx), partial);
+    hipLaunchKernelGGL(k_train_reduce, dim3((kParams + 63) / 64), dim3(kBlock), 0, st, partial, blocks, gs.d_grad);
     if (e1) (void)hipEventRecord(e1, st);
     return check_hip(ctx, hipGetLastError(), "guide gradient launch");
 }
@@ -528,10 +574,8 @@ spt_status guide_grad_launch(spt_ctx* ctx, const float* d_rec, uint32_t n, float
     hipLaunchKernelGGL(k_guide_begin, dim3(1), dim3(64), 0, st, ctl);
     spt_status s = queue_gradient(ctx, d_rec, n, 1u, nullptr, nullptr);
     if (s != SPT_OK) return s;
-    s = check_hip(ctx, hipMemcpyAsync(grad_out, gs.d_grad, kParams * sizeof(float), hipMemcpyDeviceToHost, st),
-                  "guide grad read");
     GuideCtl h;
-    if (s == SPT_OK) s = read_small(ctx, &h, ctl, sizeof(h), "guide grad");
+    s = read_small(ctx, grad_out, gs.d_grad, kParams * sizeof(float), "guide grad", &h, ctl, sizeof(h));
     if (s != SPT_OK) return s;
     for (int i = 0; i < kParams; ++i) grad_out[i] /= h.scale;
     if (loss_out) *loss_out = h.loss;
