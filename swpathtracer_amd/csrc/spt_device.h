@@ -303,7 +303,7 @@ struct GuideState {
     float* d_v = nullptr;
     float* d_grad = nullptr;
     float* d_acc = nullptr;
-    unsigned short* d_wbf = nullptr;  // bf16 copy of the parameters
+    unsigned short* d_wbf = nullptr;  // bf16 copy of the parameters, in the order of guide::FwdWeights
     float* d_records = nullptr;
     uint32_t records_cap = 0;    // batch x steps_per_pass
     uint32_t records_alloc = 0;  // allocated record slots

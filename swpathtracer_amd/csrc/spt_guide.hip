@@ -14,7 +14,10 @@ namespace {
 
 // Raw outputs for queries (p, n, wo) as 9 floats with a stride: each wave
 // encodes 64 queries (one per lane) into its stage, then runs the
-// register-resident MLP on 4 groups of 16.
+// register-resident MLP on 4 groups of 16. Three blocks a CU, as many as their
+// LDS lets in at once (a million queries 51.7 us, with four 56.7, six 52.0,
+// sixteen 55.5), and no block-wide waits. Bound by the 196 B a query moves: a
+// million queries 48 us (before: 59), 41 at the rate of a large copy.
 __global__ __launch_bounds__(kBlock) void k_guide_eval(const float* __restrict__ theta,
                                                        const unsigned short* __restrict__ wbf,
                                                        const float* __restrict__ q, uint32_t stride, uint32_t n,
@@ -36,14 +39,14 @@ __global__ __launch_bounds__(kBlock) void k_guide_eval(const float* __restrict__
             for (int i = 0; i < kEnc; ++i) f[i] = 0.0f;
         }
         stage_row(st, f);
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a stage belongs to one wave
         const uint32_t wbase = base + (uint32_t)wave * 64;
         if (wbase < n)
             mlp_stage_fwd(sw, st, [&](int g16, const f32x4 y[3]) {
                 const uint32_t smp = wbase + 16 * g16 + r;
                 if (smp < n) store_outputs(out + (size_t)smp * kOut, y);
             });
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
 
@@ -130,7 +133,7 @@ __device__ inline bf16x4 relu_grad(f32x4 v, bf16x4 h) {
     return __builtin_bit_cast(bf16x4, (u32x2){pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])});
 }
 
-// W^T of a row-major layer of 64 inputs as MFMA operands: block (t, p) holds
+// W^T of a layer of 64 inputs as MFMA operands: block (t, p) holds
 // for lane r + 16 g W[32 p + 4 g + 0..3][16 t + r] and W[32 p + 16 + 4 g + 0..3][16 t + r].
 // Rows from `rows` on count as 0.
 __device__ inline void transpose_layer(uint4* dst, const unsigned short* w, int rows) {
@@ -139,8 +142,8 @@ __device__ inline void transpose_layer(uint4* dst, const unsigned short* w, int 
         uint32_t v[4];
         for (int k = 0; k < 4; ++k) {
             const int row = 32 * p + 4 * (l >> 4) + (k >> 1) * 16 + (k & 1) * 2;
-            const unsigned short* c = w + row * kHid + 16 * t + (l & 15);
-            v[k] = row < rows ? (uint32_t)c[0] | ((uint32_t)c[kHid] << 16) : 0u;
+            const int col = 16 * t + (l & 15);
+            v[k] = row < rows ? (uint32_t)w[bf_at(kHid, row, col)] | ((uint32_t)w[bf_at(kHid, row + 1, col)] << 16) : 0u;
         }
         dst[i] = make_uint4(v[0], v[1], v[2], v[3]);
     }
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(kBlock) void k_guide_adam(float* __restrict__ theta
         v[i] = vi;
         theta[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
     }
-    wbf[i] = f2bf(theta[i]);
+    wbf[bf_at((int)i)] = f2bf(theta[i]);
     grad[i] = 0.0f;
 }
 
@@ -466,7 +469,7 @@ __global__ void k_guide_post(GuideCtl* ctl, uint32_t n) {
 
 __global__ void k_guide_tobf16(const float* __restrict__ theta, unsigned short* __restrict__ wbf) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < (uint32_t)kParams) wbf[i] = f2bf(theta[i]);
+    if (i < (uint32_t)kParams) wbf[bf_at((int)i)] = f2bf(theta[i]);
 }
 
 size_t eval_lds_bytes() { return sizeof(FwdWeights) + sizeof(WaveStage) * (kBlock / 64); }
@@ -533,7 +536,7 @@ spt_status guide_eval_launch(spt_ctx* ctx, const float* d_q, uint32_t stride, ui
     GuideState& gs = ctx->guide;
     spt_status ls = allow_lds(ctx);
     if (ls != SPT_OK) return ls;
-    const uint32_t grid = std::min<uint32_t>((n + kBlock - 1) / kBlock, (uint32_t)ctx->num_cus * 4);
+    const uint32_t grid = std::min<uint32_t>((n + kBlock - 1) / kBlock, (uint32_t)ctx->num_cus * 3);
     hipLaunchKernelGGL(k_guide_eval, dim3(grid), dim3(kBlock), eval_lds_bytes(), ctx->stream, gs.d_theta, gs.d_wbf,
                        d_q, stride, n, d_out, guide_box(ctx));
     return check_hip(ctx, hipGetLastError(), "guide eval launch");

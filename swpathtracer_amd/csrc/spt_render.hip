@@ -394,14 +394,14 @@ __global__ __launch_bounds__(kBlock) void k_guide_paths(RenderArgs a, PathBuf A,
         const uint64_t any = __ballot(mine);
         queries += (uint32_t)__popcll(any);
         stage_row(st, f);
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a stage belongs to one wave
         if (any)
             mlp_stage_fwd(sw, st, [&](int g16, const f32x4 y[3]) {
                 const int src = 16 * g16 + r;
                 const uint32_t s = __shfl(slot, src);
                 if ((any >> src) & 1ull) store_outputs_h(a.gout + (size_t)s * kOut, y);
             });
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     if (l == 0 && queries)
         atomicAdd(reinterpret_cast<unsigned long long*>(w.rays + (blockIdx.x % kRayCounters) * kRayCounterStride + kGuideQueries),
