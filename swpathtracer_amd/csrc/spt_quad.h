@@ -194,7 +194,7 @@ __device__ inline int lanes(uint64_t mask) { return (int)__builtin_popcountll(ma
 // as the single scene's); PutHit(i, h, o, d, nodes, tris) stores a
 // result: it is called by one lane per ray. `refill`: idle lanes of a wave that make it
 // take new rays. spill: this block's spill space (quad_spill_words words).
-template <bool FETCH, typename GetRay, typename PutHit>
+template <bool FETCH, bool SMALL, typename GetRay, typename PutHit>
 __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh, uint32_t first_group,
                                     uint32_t* ray_counter, QuadLds& lds, uint32_t* spill, bool& overflow,
                                     uint32_t refill, GetRay get_ray, PutHit put_hit) {
@@ -240,27 +240,26 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
         sel_far = sel_near ^ 0x00010001u;
         sel_z = inv.z >= 0.0f ? 0x0C010C00u : 0x0C000C01u;
     };
-    // Next entry of the rays that took a step; entries beyond the best hit are dropped.
-    auto pop = [&]() {
-        bool again = true;
-        const bool any_deep = ballot(sp > kQuadStack + 1) != 0;
-        while (true) {
-            if (again) {
-                --sp;
-                QuadEntry e;
-                if (any_deep) {
-                    if (sp <= kQuadStack)
-                        e = stk[sp];
-                    else
-                        e = deep[(size_t)(sp - kQuadStack - 1) * kQuadsPerBlock];
-                } else {
-                    e = stk[sp];
-                }
-                cur = (uint32_t)e;
-                again = __uint_as_float((uint32_t)(e >> 32)) > best;
-            }
-            if (!ballot(again)) break;
+    // Next entry of the rays that took a step; entries beyond the best hit are
+    // dropped. any_deep: some of their stacks reach beyond the part in LDS.
+    auto take = [&](bool any_deep) {
+        --sp;
+        QuadEntry e;
+        if (any_deep) {
+            if (sp <= kQuadStack)
+                e = stk[sp];
+            else
+                e = deep[(size_t)(sp - kQuadStack - 1) * kQuadsPerBlock];
+        } else {
+            e = stk[sp];
         }
+        cur = (uint32_t)e;
+        return __uint_as_float((uint32_t)(e >> 32)) > best;
+    };
+    auto pop = [&](bool any_deep) {
+        bool again = take(any_deep);
+        while (ballot(again))
+            if (again) again = take(any_deep);
     };
 
     while (true) {
@@ -439,9 +438,11 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
             if (at_node) {
                 uint4 g;
                 uint3 c;
-                if (sc.small_tree) {
+                if (SMALL) {
                     g = *reinterpret_cast<const uint4*>(nodes_at + (cur << 6));
-                    c = *reinterpret_cast<const uint3*>(nodes_at + ((cur << 6) + child_ofs));
+                    uint32_t at;  // in one instruction, and as a 32-bit offset beside a scalar base
+                    asm("v_lshl_or_b32 %0, %1, 6, %2" : "=v"(at) : "v"(cur), "v"(child_ofs));
+                    c = *reinterpret_cast<const uint3*>(nodes_at + at);
                 } else {
                     g = *reinterpret_cast<const uint4*>(nodes_at + (uint64_t)cur * 64);
                     c = *reinterpret_cast<const uint3*>(nodes_at + (uint64_t)cur * 64 + child_ofs);
@@ -463,8 +464,9 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                 const uint32_t zz = __builtin_amdgcn_perm(c.y, c.y, sel_z);
                 const float tn = fmaxf(fmaxf(fma_half(nxy, 0, ax, nx), fma_half(nxy, 1, ay, ny)),
                                        fmaxf(fma_half(zz, 0, az, nz), 0.0f));
-                const float tf = fminf(fminf(fma_half(fxy, 0, ax, fx), fma_half(fxy, 1, ay, fy)),
-                                       fminf(fma_half(zz, 1, az, fz), best));
+                float tf = fminf(fma_half(fxy, 0, ax, fx), fma_half(fxy, 1, ay, fy));
+                // (fminf would canonicalise best, which is never a NaN, first)
+                asm("v_min3_f32 %0, %1, %2, %3" : "=v"(tf) : "v"(tf), "v"(fma_half(zz, 1, az, fz)), "v"(best));
                 const bool hit = (tn <= tf) && c.z != kQuadNone;
                 // order among the quad's hits: entry distance, its low bits replaced by the
                 // lane; before = -(hits nearer than this lane's), the differences' sign bits
@@ -472,12 +474,12 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                 const int before = (((int)quad_swap<kSwap1>((uint32_t)key) - key) >> 31) +
                                    (((int)quad_swap<kSwap2>((uint32_t)key) - key) >> 31) +
                                    (((int)quad_swap<kSwap3>((uint32_t)key) - key) >> 31);
-                uint32_t hits = hit ? 1u : 0u;  // of the quad
-                hits += quad_swap<kSwap1>(hits);
-                hits += quad_swap<kSwap2>(hits);
-                sp += (int)hits;
+                // hits of the quad, from the wave's mask
+                const uint64_t hit_mask = ballot(tn <= tf) & ballot(c.z != kQuadNone);
+                sp += __builtin_popcount((uint32_t)(hit_mask >> (lane & 60u)) & 15u);
                 const int at = sp - 1 + before;
-                if (ballot(sp > kQuadStack + 1)) {
+                const bool any_deep = ballot(sp > kQuadStack + 1) != 0;
+                if (any_deep) {
                     if (sp > cap + 1) {  // more entries than the tree can need: reported, the ray ends
                         overflow = true;
                         sp = 1;
@@ -491,12 +493,12 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                     stk[at] = quad_entry(c.z, tn);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                pop();
+                pop(any_deep);
             }
         } else if (!at_node && cur != kQuadNone) {
             // ---- block step: one triangle (or sphere) per lane
             float4 a, b, c;
-            if (sc.small_tree) {
+            if (SMALL) {
                 const uint32_t at = ((cur + (cur << 1)) << 6) + prim_ofs;  // 192 B a block; the leaf bit shifts out
                 const float4* tp = reinterpret_cast<const float4*>(prims_at + at);
                 a = tp[0];
@@ -547,16 +549,16 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                     my.v = v;
                 }
             }
-            pop();
+            pop(ballot(sp > kQuadStack + 1) != 0);
         }
     }
 }
 
 // The rays of a launch, shared between all its waves.
-template <bool FETCH, typename GetRay, typename PutHit>
+template <bool FETCH, bool SMALL, typename GetRay, typename PutHit>
 __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray_counter, QuadLds& lds,
                                    uint32_t* spill, bool& overflow, uint32_t refill, GetRay get_ray, PutHit put_hit) {
-    trace_shares<FETCH>(sc, n, RayShares(n, gridDim.x * (kBlock / 64)), blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
+    trace_shares<FETCH, SMALL>(sc, n, RayShares(n, gridDim.x * (kBlock / 64)), blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
                         ray_counter, lds, spill, overflow, refill, get_ray, put_hit);
 }
 

@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kBlock) void k_refill(RenderArgs a, PathBuf B, Work
 // Closest hit of every live path of buffer A (count *cntA). Persistent
 // traversal; hit record and material written at the path's slot. FETCH adds
 // node / triangle record fetch counts to the two 64-bit counters at flags + 4.
-template <bool FETCH, bool MULTI>
+template <bool FETCH, bool MULTI, bool SMALL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_extend(RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA,
                                                    uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
     __shared__ QuadLds lds;
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWav
         if (threadIdx.x < 2) fetched[threadIdx.x] = 0;
         __syncthreads();
     }
-    trace_quads<FETCH>(
+    trace_quads<FETCH, SMALL>(
         a.sc, n, w.rays, lds, spill + (size_t)blockIdx.x * quad_spill_words(a.sc.stack_cap4), overflow, a.refill,
         [&](uint32_t i, V3& o, V3& d, Root& root) {
             const float4 o4 = A.o[i], d4 = A.d[i];
@@ -950,7 +950,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // read back from the caches. 128 VGPRs and 36 KB of LDS: four blocks a CU.
 // 97x61 box image, 1 sample: 590 -> 150 us; 800x600 mesh image, 4 samples,
 // where it takes the bounces from the seventh on: 6.1 -> 4.4 ms.
-template <bool MULTI>
+template <bool MULTI, bool SMALL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_finish(
     RenderArgs a, PathBuf A, Work w, const uint32_t* __restrict__ cntA, uint32_t* __restrict__ spill,
     uint32_t* __restrict__ flags) {
@@ -995,7 +995,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         rays += m;
         if (slot != kDone) mine[lanes(live & lt)] = slot;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        trace_shares<false>(
+        trace_shares<false, SMALL>(
             a.sc, m, RayShares(m), 0u, w.rays, lds, spill + (size_t)blockIdx.x * quad_spill_words(a.sc.stack_cap4), overflow,
             a.refill,
             [&](uint32_t i, V3& o, V3& d, Root& root) {
@@ -1208,7 +1208,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
     }
 
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&k_extend<true, MULTI>),
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&k_extend<true, MULTI, false>),
                                                      kBlock, 0) != hipSuccess ||
         per_cu <= 0)
         per_cu = 4;
@@ -1262,12 +1262,10 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
             }
             (void)hipEventRecord(ctx->tev[2 * stats.extend_launches], st);
         }
-        if (fetch_stats)
-            hipLaunchKernelGGL((k_extend<true, MULTI>), dim3(ext_grid), dim3(kBlock), 0, st, a, A, w, cntA,
-                               ctx->d_spill, ctx->d_flags);
-        else
-            hipLaunchKernelGGL((k_extend<false, MULTI>), dim3(ext_grid), dim3(kBlock), 0, st, a, A, w, cntA,
-                               ctx->d_spill, ctx->d_flags);
+        hipLaunchKernelGGL((fetch_stats       ? k_extend<true, MULTI, false>
+                            : a.sc.small_tree ? k_extend<false, MULTI, true>
+                                              : k_extend<false, MULTI, false>),
+                           dim3(ext_grid), dim3(kBlock), 0, st, a, A, w, cntA, ctx->d_spill, ctx->d_flags);
         if (timed) {
             (void)hipEventRecord(ctx->tev[2 * stats.extend_launches + 1], st);
             ++stats.extend_launches;
@@ -1345,7 +1343,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
         // records counted one round earlier; skip what is about to be reused
         uint32_t next_train = ctx->guide.train_every, prev_count = 0, trained = 0;
         auto finish = [&]() {  // reads its count on the device: may be queued behind a bounce still running
-            hipLaunchKernelGGL((k_finish<MULTI>), dim3(finish_grid), dim3(kBlock), 0, st, a, buf[b & 1], w, w.cnt + (b & 1),
+            hipLaunchKernelGGL((a.sc.small_tree ? k_finish<MULTI, true> : k_finish<MULTI, false>), dim3(finish_grid), dim3(kBlock), 0, st, a, buf[b & 1], w, w.cnt + (b & 1),
                                ctx->d_spill, ctx->d_flags);
             return check_hip(ctx, hipGetLastError(), "finish launch");
         };

@@ -41,7 +41,7 @@ __device__ inline uint32_t prim_of(const DevScene& sc, uint32_t idx) {
 
 // Closest-hit kernel: rays[i] -> hits[i] (FETCH: per-ray node and triangle
 // record counts into nodes_out / tris_out).
-template <bool FETCH>
+template <bool FETCH, bool SMALL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_trace_q(DevScene sc, const float4* __restrict__ rays, uint32_t n,
                                                     uint2* __restrict__ hits, uint32_t* __restrict__ nodes_out,
                                                     uint32_t* __restrict__ tris_out, uint32_t* __restrict__ spill,
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWav
                                                     uint32_t refill) {
     __shared__ QuadLds lds;
     bool overflow = false;
-    trace_quads<FETCH>(
+    trace_quads<FETCH, SMALL>(
         sc, n, rays_taken, lds, spill + (size_t)blockIdx.x * quad_spill_words(sc.stack_cap4), overflow, refill,
         [&](uint32_t i, V3& o, V3& d, Root&) {
             const float4 ro = rays[2 * (size_t)i], rd = rays[2 * (size_t)i + 1];
@@ -96,14 +96,14 @@ __device__ inline void put_pixel(const DevScene& sc, float* __restrict__ out, ui
 
 // Normal (normal_raycaster.cpp:19-31) and depth (depth_raycaster.cpp:36-48)
 // ray casters over pixels [base, base + n).
-template <int KIND>
+template <int KIND, bool SMALL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQuadWaves))) void k_raycast(DevScene sc, DevCamera cam, uint64_t base, uint32_t n,
                                                     float* __restrict__ out, uint32_t* __restrict__ spill,
                                                     uint32_t* __restrict__ flags, uint32_t* __restrict__ rays_taken,
                                                     uint32_t refill) {
     __shared__ QuadLds lds;
     bool overflow = false;
-    trace_quads<false>(
+    trace_quads<false, SMALL>(
         sc, n, rays_taken, lds, spill + (size_t)blockIdx.x * quad_spill_words(sc.stack_cap4), overflow, refill,
         [&](uint32_t i, V3& o, V3& d, Root&) { pixel_ray(cam, base + i, o, d); },
         [&](uint32_t i, const Hit& h, V3 o, V3 d, uint32_t, uint32_t) { put_pixel<KIND>(sc, out, base + i, h, o, d); });
@@ -254,17 +254,18 @@ spt_status launch_trace(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t n, spt_h
             "trace launch");
     if (mode == SPT_TRACE_CLOSEST)
         return quad_launches(
-            ctx, reinterpret_cast<const void*>(&k_trace_q<false>), n,
+            ctx, reinterpret_cast<const void*>(&k_trace_q<false, true>), n,
             [&](uint64_t base, uint32_t cnt, uint32_t grid) {
-                hipLaunchKernelGGL(k_trace_q<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
+                hipLaunchKernelGGL((sc.small_tree ? k_trace_q<false, true> : k_trace_q<false, false>), dim3(grid),
+                                   dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
                                    hits + base, nullptr, nullptr, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
             },
             "trace launch");
     if (mode == SPT_TRACE_FETCH)
         return quad_launches(
-            ctx, reinterpret_cast<const void*>(&k_trace_q<true>), n,
+            ctx, reinterpret_cast<const void*>(&k_trace_q<true, false>), n,
             [&](uint64_t base, uint32_t cnt, uint32_t grid) {
-                hipLaunchKernelGGL(k_trace_q<true>, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
+                hipLaunchKernelGGL((k_trace_q<true, false>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, rays + 2 * base, cnt,
                                    hits + base, d_tests + base, d_isects + base, ctx->d_spill, ctx->d_flags,
                                    ctx->d_rays, refill_of(ctx));
             },
@@ -314,7 +315,7 @@ spt_status launch_trace_noalloc(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t 
         return set_error(ctx, SPT_ERR_INVALID, "spt_trace_noalloc: more than SPT_NOALLOC_MAX_RAYS rays");
     if (!ctx->scratch) return set_error(ctx, SPT_ERR_STATE, "spt_trace_noalloc: no static scratch on this device");
     if (n == 0) return SPT_OK;
-    const void* kern = reinterpret_cast<const void*>(&k_trace_q<false>);
+    const void* kern = reinterpret_cast<const void*>(&k_trace_q<false, true>);
     // blocks whose stack entries beyond the LDS part fit the scratch
     const uint64_t per_block = quad_spill_words(ctx->stack_cap4);
     const uint64_t room = (uint64_t)SPT_NOALLOC_SCRATCH_WORDS - kScratchSpill;
@@ -330,7 +331,8 @@ spt_status launch_trace_noalloc(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t 
         const uint32_t grid = (uint32_t)std::min<uint64_t>(quad_grid(ctx, kern, cnt), max_blocks);
         // a fill kernel, not a memset node: callers may capture this in a graph
         hipLaunchKernelGGL(k_scratch_reset, dim3(1), dim3(kScratchSpill), 0, ctx->stream, ctl);
-        hipLaunchKernelGGL(k_trace_q<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->scene(), rays + 2 * base,
+        hipLaunchKernelGGL((ctx->small_tree ? k_trace_q<false, true> : k_trace_q<false, false>), dim3(grid), dim3(kBlock),
+                           0, ctx->stream, ctx->scene(), rays + 2 * base,
                            cnt, hits + base, nullptr, nullptr, spill, ctl, ctl + kScratchRays, refill_of(ctx));
         // a stack overflow is reported by spt_sync, as for spt_trace
         hipLaunchKernelGGL(k_scratch_fold_overflow, dim3(1), dim3(64), 0, ctx->stream, ctl, ctx->d_flags);
@@ -363,17 +365,19 @@ spt_status launch_raycast(spt_ctx* ctx, const spt_camera* cam, uint32_t kind, vo
             "raycast launch");
     if (kind == SPT_RAYCAST_NORMAL)
         return quad_launches(
-            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_NORMAL>), n,
+            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_NORMAL, true>), n,
             [&](uint64_t base, uint32_t cnt, uint32_t grid) {
-                hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_NORMAL>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
+                hipLaunchKernelGGL((sc.small_tree ? k_raycast<SPT_RAYCAST_NORMAL, true> : k_raycast<SPT_RAYCAST_NORMAL, false>),
+                                   dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
                                    base, cnt, out, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
             },
             "raycast launch");
     if (kind == SPT_RAYCAST_DEPTH)
         return quad_launches(
-            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_DEPTH>), n,
+            ctx, reinterpret_cast<const void*>(&k_raycast<SPT_RAYCAST_DEPTH, true>), n,
             [&](uint64_t base, uint32_t cnt, uint32_t grid) {
-                hipLaunchKernelGGL((k_raycast<SPT_RAYCAST_DEPTH>), dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
+                hipLaunchKernelGGL((sc.small_tree ? k_raycast<SPT_RAYCAST_DEPTH, true> : k_raycast<SPT_RAYCAST_DEPTH, false>),
+                                   dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
                                    base, cnt, out, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
             },
             "raycast launch");
