@@ -16,7 +16,7 @@ struct Draws {
     uint32_t stride;
     uint32_t k;
     bool overflow;
-    __device__ float next() {
+    __device__ __forceinline__ float next() {
         if (stream) {
             if (k >= stride) {
                 overflow = true;
@@ -37,7 +37,7 @@ struct BSample {
 };
 
 // FresnelSchlick with reflectance at normal incidence (fresnel_schlick.cpp:11-18)
-__device__ inline V3 schlick_r0(const float* r0, float c) {
+__device__ __forceinline__ V3 schlick_r0(const float* r0, float c) {
     float c5 = 1.0f - c;
     c5 = c5 * c5 * c5 * c5 * c5;
     return V3{r0[0] + (1.0f - r0[0]) * c5, r0[1] + (1.0f - r0[1]) * c5, r0[2] + (1.0f - r0[2]) * c5};
@@ -46,7 +46,7 @@ __device__ inline V3 schlick_r0(const float* r0, float c) {
 // Exact conductor Fresnel for complex IOR eta + i k from a medium of IOR 1
 // (textbook form, Pharr/Jakob/Humphreys PBR 3rd ed. sec. 8.2.1), with
 // dek = eta^2 - k^2 and fek = 4 eta^2 k^2 (prepare_layer).
-__device__ inline float fresnel_conductor(float ci, float dek, float fek) {
+__device__ __forceinline__ float fresnel_conductor(float ci, float dek, float fek) {
     ci = gmin(gmax(ci, -1.0f), 1.0f);
     const float c2 = ci * ci, s2 = 1.0f - c2;
     const float t0 = dek - s2;
@@ -60,27 +60,27 @@ __device__ inline float fresnel_conductor(float ci, float dek, float fek) {
     const float rp = rs * (t3 - t4) / (t3 + t4);
     return 0.5f * (rp + rs);
 }
-__device__ inline V3 fresnel_conductor3(float ci, const spt_layer& l) {
+__device__ __forceinline__ V3 fresnel_conductor3(float ci, const spt_layer& l) {
     return V3{fresnel_conductor(ci, l.eta[0], l.k[0]), fresnel_conductor(ci, l.eta[1], l.k[1]),
               fresnel_conductor(ci, l.eta[2], l.k[2])};
 }
 
 // GGX D and Smith G1 (Walter, Marschner, Li, Torrance 2007)
-__device__ inline float ggx_d(float ch, float alpha) {
+__device__ __forceinline__ float ggx_d(float ch, float alpha) {
     if (ch <= 0.0f) return 0.0f;
     const float a2 = alpha * alpha, c2 = ch * ch;
     const float den = c2 * (a2 - 1.0f) + 1.0f;
     return a2 / (kPi * den * den);
 }
-__device__ inline float ggx_g1(float cv, float alpha) {
+__device__ __forceinline__ float ggx_g1(float cv, float alpha) {
     if (cv <= 0.0f) return 0.0f;
     const float a2 = alpha * alpha, c2 = cv * cv;
     return 2.0f * cv / (cv + sqrt_rn(a2 + (1.0f - a2) * c2));
 }
 
-__device__ inline bool layer_opaque(const spt_layer& l) { return l.type != SPT_BSDF_SMOOTH_DIELECTRIC; }
+__device__ __forceinline__ bool layer_opaque(const spt_layer& l) { return l.type != SPT_BSDF_SMOOTH_DIELECTRIC; }
 
-__device__ inline V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
+__device__ __forceinline__ V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
     switch (l.type) {
         case SPT_BSDF_LAMBERTIAN: {  // lambertian.cpp:9-16 (brdf_ = kd / pi: prepare_layer)
             if (wi.y > 0.0f) return V3{l.r0[0], l.r0[1], l.r0[2]};
@@ -122,7 +122,7 @@ __device__ inline V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
     return V3{0.0f, 0.0f, 0.0f};
 }
 
-__device__ inline V3 layer_reflectance(const spt_layer& l, V3 wo, V3 wi) {
+__device__ __forceinline__ V3 layer_reflectance(const spt_layer& l, V3 wo, V3 wi) {
     switch (l.type) {
         case SPT_BSDF_LAMBERTIAN:
             return V3{l.kd[0], l.kd[1], l.kd[2]};
@@ -143,7 +143,7 @@ __device__ inline V3 layer_reflectance(const spt_layer& l, V3 wo, V3 wi) {
 }
 
 // UniformBSDFSampler (uniform_bsdf_sampler.cpp:5-14)
-__device__ inline BSample sample_uniform(Draws& r) {
+__device__ __forceinline__ BSample sample_uniform(Draws& r) {
     const float r1 = r.next();
     const float r2 = r.next();
     const float phi = 2.0f * kPi * r2;
@@ -154,7 +154,7 @@ __device__ inline BSample sample_uniform(Draws& r) {
 }
 
 // CookTorranceBSDFSampler::getProbability (cook_torrance_bsdf_sampler.cpp:22-42)
-__device__ inline float beckmann_pdf(const spt_layer& l, V3 wo, V3 wi) {
+__device__ __forceinline__ float beckmann_pdf(const spt_layer& l, V3 wo, V3 wi) {
     if (wi.y <= 0.0f) return 1.0f;
     const V3 h = normalize(wo + wi);
     const float nh = gmax(0.0f, h.y);
@@ -168,7 +168,7 @@ __device__ inline float beckmann_pdf(const spt_layer& l, V3 wo, V3 wi) {
     return (d1 * f_exp(d2) * nh) / (4.0f * om);
 }
 
-__device__ inline float ggx_pdf(const spt_layer& l, V3 wo, V3 wi) {
+__device__ __forceinline__ float ggx_pdf(const spt_layer& l, V3 wo, V3 wi) {
     if (wi.y <= 0.0f || wo.y <= 0.0f) return 0.0f;
     const V3 h = normalize(wo + wi);
     const float om = dot(wi, h);
@@ -176,7 +176,7 @@ __device__ inline float ggx_pdf(const spt_layer& l, V3 wo, V3 wi) {
     return ggx_d(h.y, l.roughness) * h.y / (4.0f * om);
 }
 
-__device__ inline BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
+__device__ __forceinline__ BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
     switch (l.type) {
         case SPT_BSDF_LAMBERTIAN: {
             if (l.sampler == SPT_SAMPLER_UNIFORM) return sample_uniform(r);
@@ -250,7 +250,7 @@ __device__ inline BSample layer_sample(const spt_layer& l, V3 wo, Draws& r) {
 
 // layer_f and layer_reflectance of one direction (GGX: one half vector and,
 // in front of the microfacet, one Fresnel term for both).
-__device__ inline void layer_eval(const spt_layer& l, V3 wo, V3 wi, V3& f, V3& refl) {
+__device__ __forceinline__ void layer_eval(const spt_layer& l, V3 wo, V3 wi, V3& f, V3& refl) {
     if (l.type != SPT_BSDF_GGX_CONDUCTOR) {
         f = layer_f(l, wo, wi);
         refl = layer_reflectance(l, wo, wi);
@@ -275,7 +275,7 @@ struct Walk {
     float fp;
     int id, bounce;
     bool reached_inf;
-    __device__ void start(const spt_material& m, V3 wo) {
+    __device__ __forceinline__ void start(const spt_material& m, V3 wo) {
         nwo = wo;
         fb = fr = V3{1.0f, 1.0f, 1.0f};
         fp = 1.0f;
@@ -283,10 +283,10 @@ struct Walk {
         bounce = 0;
         id = (nwo.y > 0.0f) ? 0 : (int)m.n_layers - 1;
     }
-    __device__ bool running(const spt_material& m) const {
+    __device__ __forceinline__ bool running(const spt_material& m) const {
         return (id > -1) && (id < (int)m.n_layers) && (fp > 0.0f) && (!reached_inf) && (bounce < 500);
     }
-    __device__ void step(const spt_material& m, Draws& r) {
+    __device__ __forceinline__ void step(const spt_material& m, Draws& r) {
         const float inf = __builtin_inff();
         const spt_layer& l = m.layers[id];
         const BSample s = layer_sample(l, nwo, r);
@@ -310,7 +310,7 @@ struct Walk {
         nwo = -wi;
         ++bounce;
     }
-    __device__ void result(V3& bsdf, V3& refl, float& pdf) const {
+    __device__ __forceinline__ void result(V3& bsdf, V3& refl, float& pdf) const {
         if ((bounce < 500) && !reached_inf && (fp > 0.0f)) {
             pdf = fp;
             bsdf = fb;
@@ -323,7 +323,7 @@ struct Walk {
     }
 };
 
-__device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& refl, float& pdf, V3& wi,
+__device__ __forceinline__ void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& refl, float& pdf, V3& wi,
                                     Draws& r) {
     Walk k;
     k.wi = wi;
@@ -337,7 +337,7 @@ __device__ inline void layered_eval(const spt_material& m, V3 wo, V3& bsdf, V3& 
 // called twice per camera sample (pathtracer.cpp:110-111), x from the first
 // call and y from the second; each random call draws two numbers, the first
 // going to x.
-__device__ inline void pixel_offset(uint32_t type, uint32_t n, float w, uint32_t s, Draws& r, float& sx,
+__device__ __forceinline__ void pixel_offset(uint32_t type, uint32_t n, float w, uint32_t s, Draws& r, float& sx,
                                     float& sy) {
     if (type == SPT_PIXEL_REGULAR) {
         const float off = w * 0.5f;

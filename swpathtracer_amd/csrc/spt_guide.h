@@ -281,12 +281,15 @@ struct Lobe {
 
 // y: the 40 raw outputs (a float pointer, or a HalfRow).
 template <typename Row>
-__device__ inline void mixture_params(const Row& y, Lobe L[kLobes]) {
+__device__ __forceinline__ void mixture_params(const Row& y, Lobe L[kLobes]) {
     float amax = -3.0e38f;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) amax = fmaxf(amax, y[5 * i + 4]);
     float sum = 0.0f;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) sum += expf(y[5 * i + 4] - amax);
     const float lse = amax + logf(sum);
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) {
         const V3 raw{y[5 * i], y[5 * i + 1], y[5 * i + 2]};
         const float nr = sqrtf(dot(raw, raw) + 1e-12f);
@@ -302,22 +305,23 @@ __device__ inline void mixture_params(const Row& y, Lobe L[kLobes]) {
 }
 
 // log of kappa / (2 pi (1 - e^{-2 kappa})) exp(kappa (mu.d - 1))
-__device__ inline float log_vmf(const Lobe& L, V3 d) {
+__device__ __forceinline__ float log_vmf(const Lobe& L, V3 d) {
     return logf(L.kappa) - 1.8378770664093453f - logf(-expm1f(-2.0f * L.kappa)) + L.kappa * (dot(L.mu, d) - 1.0f);
 }
 
 // log of the vMF normalisation kappa / (2 pi (1 - e^{-2 kappa}))
-__device__ inline float log_vmf_norm(float k) { return logf(k) - 1.8378770664093453f - logf(-expm1f(-2.0f * k)); }
+__device__ __forceinline__ float log_vmf_norm(float k) { return logf(k) - 1.8378770664093453f - logf(-expm1f(-2.0f * k)); }
 
 // Product of the mixture with one vMF lobe (mb, kb), renormalised (product
 // importance sampling with vMF lobes, Herholz et al. 2016):
 // vMF(mu_i, k_i) vMF(mb, kb) = C_i C_b / C' e^{k' - k_i - kb} vMF(mu', k')
 // with k' mu' = k_i mu_i + kb mb. The result is again a mixture, so sampling
 // and density stay exact.
-__device__ inline void mixture_product(Lobe L[kLobes], V3 mb, float kb) {
+__device__ __forceinline__ void mixture_product(Lobe L[kLobes], V3 mb, float kb) {
     const float lcb = log_vmf_norm(kb);
     float lw[kLobes];
     float m = -3.0e38f;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) {
         const V3 v = L[i].mu * L[i].kappa + mb * kb;
         const float nv = sqrtf(dot(v, v));
@@ -328,13 +332,16 @@ __device__ inline void mixture_product(Lobe L[kLobes], V3 mb, float kb) {
         m = fmaxf(m, lw[i]);
     }
     float sum = 0.0f;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) sum += expf(lw[i] - m);
     const float lse = m + logf(sum);
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) L[i].logw = lw[i] - lse;
 }
 
-__device__ inline float mixture_pdf(const Lobe L[kLobes], V3 d) {
+__device__ __forceinline__ float mixture_pdf(const Lobe L[kLobes], V3 d) {
     float q = 0.0f;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) q += expf(L[i].logw + log_vmf(L[i], d));
     return q;
 }
@@ -349,17 +356,21 @@ __device__ inline void basis(V3 n, V3& t, V3& b) {
 }
 
 // Sample the mixture: lobe by weight (u0), then Jakob's stable vMF sampler.
-__device__ inline V3 mixture_sample(const Lobe L[kLobes], float u0, float u1, float u2) {
-    int k = kLobes - 1;
+__device__ __forceinline__ V3 mixture_sample(const Lobe L[kLobes], float u0, float u1, float u2) {
+    // the first lobe whose running weight exceeds u0 (else the last), carried
+    // along: an index would put the lobes into scratch memory
+    V3 mu = L[kLobes - 1].mu;
+    float kap = L[kLobes - 1].kappa;
     float c = 0.0f;
+    bool found = false;
+#pragma unroll
     for (int i = 0; i < kLobes; ++i) {
         c += expf(L[i].logw);
-        if (u0 < c) {
-            k = i;
-            break;
-        }
+        const bool here = !found && u0 < c;
+        mu = V3{here ? L[i].mu.x : mu.x, here ? L[i].mu.y : mu.y, here ? L[i].mu.z : mu.z};
+        kap = here ? L[i].kappa : kap;
+        found = found || here;
     }
-    const float kap = L[k].kappa;
     // for kappa above ~44, e^{-2 kappa} underflows and u1 = 0 gives log(0):
     // the exact limit is w = -1, so clamp (a NaN direction would make the
     // next ray visit every node of the tree)
@@ -367,8 +378,8 @@ __device__ inline V3 mixture_sample(const Lobe L[kLobes], float u0, float u1, fl
     const float st = sqrtf(fmaxf(0.0f, 1.0f - w * w));
     const float ph = 2.0f * kPi * u2;
     V3 t, b;
-    basis(L[k].mu, t, b);
-    return t * (st * cosf(ph)) + b * (st * sinf(ph)) + L[k].mu * w;
+    basis(mu, t, b);
+    return t * (st * cosf(ph)) + b * (st * sinf(ph)) + mu * w;
 }
 
 }  // namespace guide

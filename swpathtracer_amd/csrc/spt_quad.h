@@ -164,7 +164,10 @@ __device__ inline bool accept_near(V3 o, V3 d, float t, float u, float v, V3 v0,
 // from the others. Blocks go to the XCDs in turn, so a region's counter stays
 // in one XCD's L2. One counter for all rays was the limit of mid-sized
 // launches: about 10 ns per atomic on an address that all XCDs share, 160 us
-// for 1M rays in shares of 32 to 64.
+// for 1M rays in shares of 32 to 64. A share is a quarter of what an even split
+// of the region's rest would give each wave: long rays lie together in an
+// image, and with half of it the last waves held 1920x1080 primary rays up
+// from 0.33 to 0.41 ms (incoherent rays, 16.8M: 2.36 and 2.42 ms).
 constexpr uint32_t kRayCounters = 8, kRayCounterStride = 32;  // one 128-B line each
 constexpr uint32_t kRayCounterWords = kRayCounters * kRayCounterStride;
 struct RayShares {
@@ -346,7 +349,7 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                             while (tried < kRayCounters && sh.fixed < n) {
                                 const uint32_t region = (blockIdx.x + tried) % kRayCounters;
                                 const uint32_t take =
-                                    max((uint32_t)kQuadPool, min(left * kRayCounters / (2u * sh.waves), 512u) & ~31u);
+                                    max((uint32_t)kQuadPool, min(left * kRayCounters / (4u * sh.waves), 512u) & ~31u);
                                 uint32_t at = 0;
                                 if (lane == 0) at = atomicAdd(ray_counter + region * kRayCounterStride, take);
                                 at = __builtin_amdgcn_readfirstlane(at);

@@ -129,7 +129,7 @@ __device__ inline void count_done(const RenderArgs& a, uint32_t jid, uint32_t n)
 // per wave, whose addresses all XCDs share) when the jobs fit them.
 constexpr uint32_t kDoneJobs = 512;
 template <bool MULTI>
-__device__ inline void finish_path(const RenderArgs& a, const Job& jb, uint32_t jid, uint32_t pix, uint64_t local,
+__device__ __forceinline__ void finish_path(const RenderArgs& a, const Job& jb, uint32_t jid, uint32_t pix, uint64_t local,
                                    float4 L, uint32_t* done) {
     if (MULTI) {
         if (a.n_jobs <= kDoneJobs)
@@ -140,7 +140,7 @@ __device__ inline void finish_path(const RenderArgs& a, const Job& jb, uint32_t 
     if (jb.film32) {
         float* f = jb.film32 + 3 * (size_t)pix;
         // adding 0 changes nothing, and most paths end without light: 28M paths
-        // shaded in 1.37 ms instead of 1.65
+        // shaded in 1.37 ms instead of 1.65 (blocks of 256)
         if (L.x != 0.0f) unsafeAtomicAdd(f + 0, L.x);
         if (L.y != 0.0f) unsafeAtomicAdd(f + 1, L.y);
         if (L.z != 0.0f) unsafeAtomicAdd(f + 2, L.z);
@@ -422,7 +422,7 @@ __device__ inline float layer_density(const spt_layer& l, V3 wo, V3 wi) {
 // coat, and w2 is the direction that refracts to it (tangential part scaled
 // by 1/eta). p(w2) = p(exit) |d exit / d w2| = p(exit) eta^2 cos(w2) /
 // cos(exit). Directions past the critical angle are never proposed.
-__device__ inline float coat_guide_density(const guide::Lobe* lobes, const Frame& fr, V3 w2, float eta) {
+__device__ __forceinline__ float coat_guide_density(const guide::Lobe* lobes, const Frame& fr, V3 w2, float eta) {
     const float t2 = eta * eta * (w2.x * w2.x + w2.z * w2.z);
     if (w2.y <= 0.0f || t2 >= 1.0f) return 0.0f;
     const float cy = sqrtf(1.0f - t2);
@@ -457,7 +457,7 @@ __device__ inline void bsdf_lobe(const spt_layer& l, V3 wo, float widen, V3& mb,
 // has no density) use the layer's own sampler: mixing there would double the
 // weight of every such revisit. 'via' is set when the walk reached the
 // opaque layer.
-__device__ inline void layered_eval_guided(const spt_material& m, V3 wo, const Frame& frm, const guide::Lobe* lobes,
+__device__ __forceinline__ void layered_eval_guided(const spt_material& m, V3 wo, const Frame& frm, const guide::Lobe* lobes,
                                            float c, V3& bsdf, V3& refl, float& pdf, V3& wi, Draws& r, bool& via) {
     const spt_layer& coat = m.layers[0];
     const spt_layer& base = m.layers[1];
@@ -547,7 +547,7 @@ struct Survivor {
 };
 
 template <bool GUIDED>
-__device__ inline void store_survivor(const RenderArgs& a, const PathBuf& B, const Survivor& sv, uint32_t slot) {
+__device__ __forceinline__ void store_survivor(const RenderArgs& a, const PathBuf& B, const Survivor& sv, uint32_t slot) {
     B.o[slot] = sv.o;
     B.d[slot] = sv.d;
     B.thr[slot] = sv.thr;
@@ -559,7 +559,7 @@ __device__ inline void store_survivor(const RenderArgs& a, const PathBuf& B, con
 
 // A path's vertex at its hit: position, shading normal, local frame and
 // outgoing direction in it.
-__device__ inline void path_vertex(const RenderArgs& a, V3 o, V3 d, float4 hv, V3& pos, V3& nrm, Frame& fr, V3& wo) {
+__device__ __forceinline__ void path_vertex(const RenderArgs& a, V3 o, V3 d, float4 hv, V3& pos, V3& nrm, Frame& fr, V3& wo) {
     Hit h;
     h.t = hv.x;
     h.idx = __float_as_uint(hv.y);
@@ -574,7 +574,7 @@ __device__ inline void path_vertex(const RenderArgs& a, V3 o, V3 d, float4 hv, V
 // Shading of one vertex (integrators/pathtracer.cpp:21-54) of path j in
 // shading order; go_on(survivor) is called for a path that does not end here.
 template <bool MULTI, bool GUIDED, bool WALKS, typename GoOn>
-__device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const Work& w, const spt_material* smats,
+__device__ __forceinline__ void shade_path(const RenderArgs& a, const PathBuf& A, const Work& w, const spt_material* smats,
                                   bool lds_mats, uint32_t i, uint32_t* done, GoOn go_on) {
     const float4 hv = w.hit[i];
     float4 rad = A.rad[i];
@@ -768,7 +768,7 @@ __device__ inline void shade_path(const RenderArgs& a, const PathBuf& A, const W
 // ones once half of its lanes have finished; each round it steps the lanes at
 // a dielectric or the others, whichever are more, so that lanes line up.
 // 123M-path mesh image (28M live paths a launch): sort, walks and shading 2.5
-// -> 0.88 (walks) + 1.37 ms (k_shade), the rays of the unsorted queue 5% faster
+// -> 0.88 (walks) + 1.01 ms (k_shade), the rays of the unsorted queue 5% faster
 // as well. Bound by VALU issue at 20 lanes.
 template <bool MULTI>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(RenderArgs a, PathBuf A, Work w,
@@ -868,18 +868,61 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 
 // Shading of one bounce (integrators/pathtracer.cpp:21-54) for every live
 // path of A, in the queue's order; survivors are appended to B, with one atomic
-// on B's count per block and 256 paths: one per wave (the compiler's
-// aggregation) made that address the limit, about 10 ns per atomic that all
-// XCDs share (61M paths: 950k atomics in a 10.2-ms launch).
+// on B's count per block and turn: one per wave (the compiler's aggregation)
+// made that address the limit, about 10 ns per atomic that all XCDs share (61M
+// paths: 950k atomics in a 10.2-ms launch).
 // GUIDED instantiates the guide's sampling and record capture and walks in
 // place (a bounce's launches are shorter there, and a launch more costs the
 // length of its longest walk, 60 us); the plain instantiation carries none of
 // their registers and leaves layered materials to k_walk. Bound by the queue's
-// traffic, about 210 B a path (28M paths 1.37 ms, 4.4 TB/s); five or six waves
-// per SIMD instead of four do not change that (1.40, 1.56 ms).
+// traffic, about 200 B a path (28M paths 1.01 ms); five or six waves per SIMD
+// instead of four do not help.
+// Threads of a shading block, which takes its survivors' slots with one
+// atomic: 28M paths shaded in 1.45 ms with 256, 1.01 with 512, 1.09 with 1024.
+// Guided shading is bound by its own instructions and its waves wait for each
+// other less in smaller blocks (400x300, 36-sample pass 10.6 ms with 256, 11.0
+// with 512).
+template <bool GUIDED>
+constexpr uint32_t kShadeBlock = GUIDED ? 256 : 512;
+
+// Guided shading keeps the survivors of a block in LDS across the barriers:
+// held in registers they spill 72 of them.
+template <bool GUIDED>
+struct Park {
+    float4 o[kShadeBlock<true>], d[kShadeBlock<true>], thr[kShadeBlock<true>], rad[kShadeBlock<true>];
+    uint4 gr[kShadeBlock<true>];
+    uint64_t key[kShadeBlock<true>], local[kShadeBlock<true>];
+    __device__ __forceinline__ void put(const RenderArgs& a, const Survivor& sv) {
+        const uint32_t i = threadIdx.x;
+        o[i] = sv.o;
+        d[i] = sv.d;
+        thr[i] = sv.thr;
+        rad[i] = sv.rad;
+        key[i] = sv.key;
+        if (a.per_path) local[i] = sv.local;
+        if (a.train) gr[i] = sv.gr;
+    }
+    __device__ __forceinline__ void get(const RenderArgs& a, Survivor& sv) {
+        const uint32_t i = threadIdx.x;
+        sv.o = o[i];
+        sv.d = d[i];
+        sv.thr = thr[i];
+        sv.rad = rad[i];
+        sv.key = key[i];
+        if (a.per_path) sv.local = local[i];
+        if (a.train) sv.gr = gr[i];
+    }
+};
+template <>
+struct Park<false> {
+    __device__ void put(const RenderArgs&, const Survivor&) {}
+    __device__ void get(const RenderArgs&, Survivor&) {}
+};
+
 template <bool MULTI, bool GUIDED>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_shade(RenderArgs a, PathBuf A, PathBuf B, Work w,
+__global__ __launch_bounds__(kShadeBlock<GUIDED>) __attribute__((amdgpu_waves_per_eu(4))) void k_shade(RenderArgs a, PathBuf A, PathBuf B, Work w,
                                                   const uint32_t* __restrict__ cntA, uint32_t* __restrict__ cntB) {
+    constexpr uint32_t kThreads = kShadeBlock<GUIDED>;
     // the material table in LDS when it is small (each lane reads its
     // layered material field by field)
     __shared__ spt_material smats[kLdsMats];
@@ -888,34 +931,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const uint32_t words = a.sc.n_mats * (uint32_t)(sizeof(spt_material) / 4);
         const uint32_t* src = reinterpret_cast<const uint32_t*>(a.sc.mats);
         uint32_t* dst = reinterpret_cast<uint32_t*>(smats);
-        for (uint32_t k = threadIdx.x; k < words; k += kBlock) dst[k] = src[k];
+        for (uint32_t k = threadIdx.x; k < words; k += kThreads) dst[k] = src[k];
     }
     __shared__ uint32_t done[MULTI ? kDoneJobs : 1];  // finished paths of the block per job
     if (MULTI)
-        for (uint32_t k = threadIdx.x; k < kDoneJobs; k += kBlock) done[k] = 0;
+        for (uint32_t k = threadIdx.x; k < kDoneJobs; k += kThreads) done[k] = 0;
     __syncthreads();
-    // survivors of the block's four waves (two sets, used in turn) and their first slot
-    __shared__ uint32_t survivors[2][kBlock / 64 + 1];
+    __shared__ Park<GUIDED> park;
+    // survivors of the block's waves (two sets, used in turn) and their first slot
+    __shared__ uint32_t survivors[2][kThreads / 64 + 1];
     const uint32_t n = *cntA;
-    const uint32_t gthreads = gridDim.x * kBlock;
+    const uint32_t gthreads = gridDim.x * kThreads;
     const uint32_t wave = threadIdx.x / 64;
     uint32_t turn = 0;
-    for (uint32_t j0 = blockIdx.x * kBlock; j0 < n; j0 += gthreads, turn ^= 1u) {
+    for (uint32_t j0 = blockIdx.x * kThreads; j0 < n; j0 += gthreads, turn ^= 1u) {
         const uint32_t j = j0 + threadIdx.x;
-        if (GUIDED) {  // a slot per lane (per wave, as the compiler aggregates them): holding the survivors
-                       // across the barriers would spill 72 VGPRs instead of 22, which costs guided
-                       // passes as much as the shared address
-            if (j < n)
-                shade_path<MULTI, true, true>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& sv) {
-                    store_survivor<GUIDED>(a, B, sv, atomicAdd(cntB, 1u));
-                });
-            continue;
-        }
         Survivor sv;
         bool alive = false;
         if (j < n)
-            shade_path<MULTI, false, false>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& next) {
-                sv = next;
+            shade_path<MULTI, GUIDED, GUIDED>(a, A, w, smats, lds_mats, j, done, [&](const Survivor& next) {
+                if (GUIDED)
+                    park.put(a, next);
+                else
+                    sv = next;
                 alive = true;
             });
         const uint64_t am = __ballot(alive);
@@ -923,18 +961,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         __syncthreads();
         if (threadIdx.x == 0) {
             uint32_t sum = 0;
-            for (uint32_t v = 0; v < kBlock / 64; ++v) sum += survivors[turn][v];
-            survivors[turn][kBlock / 64] = sum ? atomicAdd(cntB, sum) : 0u;
+            for (uint32_t v = 0; v < kThreads / 64; ++v) sum += survivors[turn][v];
+            survivors[turn][kThreads / 64] = sum ? atomicAdd(cntB, sum) : 0u;
         }
         __syncthreads();
         if (!alive) continue;
-        uint32_t slot = survivors[turn][kBlock / 64] + (uint32_t)__popcll(am & __lanemask_lt());
+        uint32_t slot = survivors[turn][kThreads / 64] + (uint32_t)__popcll(am & __lanemask_lt());
         for (uint32_t v = 0; v < wave; ++v) slot += survivors[turn][v];
+        if (GUIDED) park.get(a, sv);
         store_survivor<GUIDED>(a, B, sv, slot);
     }
     if (MULTI && a.n_jobs <= kDoneJobs) {
         __syncthreads();
-        for (uint32_t k = threadIdx.x; k < a.n_jobs; k += kBlock)
+        for (uint32_t k = threadIdx.x; k < a.n_jobs; k += kThreads)
             if (done[k]) count_done(a, k, done[k]);
     }
 }
@@ -1218,7 +1257,10 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
                                  // the 1024-spp mesh image at 911, 948, 897, 914 Mpaths/s
         per_cu = std::min<int>(per_cu, tn.wavefronts == 2 ? 5 : 4);
     const uint32_t ext_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)(per_cu * ctx->num_cus));
-    const uint32_t shade_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * tn.shade_blocks_per_cu);
+    // tn.shade_blocks_per_cu counts blocks of kBlock threads
+    const uint32_t shade_block = a.guided ? kShadeBlock<true> : kShadeBlock<false>;
+    const uint32_t shade_grid = std::max<uint32_t>(
+        1, std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * tn.shade_blocks_per_cu) / (shade_block / kBlock));
     const uint32_t walk_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * 4);
     const uint32_t refill_grid = std::min<uint32_t>(blocks_for(cap), (uint32_t)ctx->num_cus * 8);
     hipStream_t st = ctx->stream;
@@ -1284,7 +1326,7 @@ spt_status run_paths(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tuni
             if (timed && !gev.empty()) (void)hipEventRecord(gev.back(), st);
         }
         if (a.walk) hipLaunchKernelGGL((k_walk<MULTI>), dim3(walk_grid), dim3(kBlock), 0, st, a, A, w, cntA);
-        hipLaunchKernelGGL((a.guided ? k_shade<MULTI, true> : k_shade<MULTI, false>), dim3(shade_grid), dim3(kBlock), 0, st, a, A, B, w, cntA, cntB);
+        hipLaunchKernelGGL((a.guided ? k_shade<MULTI, true> : k_shade<MULTI, false>), dim3(shade_grid), dim3(shade_block), 0, st, a, A, B, w, cntA, cntB);
         // regeneration: the survivors' buffer is topped up with new camera paths
         hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, st, cntA, cntB, w.cnt, w.rays, (uint32_t)cap, total, ctx->d_status,
                            a.job_clock);
