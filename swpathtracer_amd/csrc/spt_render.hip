@@ -787,17 +787,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     __syncthreads();
     const uint64_t lt = __lanemask_lt();
     const uint32_t n = *cntA, waves = gridDim.x * (kBlock / 64);
-    const uint32_t share = ((n + waves - 1) / waves + 63u) & ~63u;
     uint32_t* list = lists[threadIdx.x / 64];
-    uint32_t next = min(n, (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * share), found = 0;
-    const uint32_t end = min(n, next + share);
+    // 64 slots at a time, dealt to the waves in turn: layered paths lie together
+    uint32_t next = (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * 64, found = 0;
     uint32_t slot = kDone, mid = 0;
     bool walking = false;
     Walk wk{};
     Draws r{};
     while (true) {
         const uint64_t idle = __ballot(!walking);
-        if (idle == ~0ull || ((next < end || found) && __popcll(idle) >= kWalkRefill)) {
+        if (idle == ~0ull || ((next < n || found) && __popcll(idle) >= kWalkRefill)) {
             if (!walking && slot != kDone) {
                 V3 bsdf, refl;
                 float pdf;
@@ -820,14 +819,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 if (r.overflow) atomicAdd(&w.cnt[2], 1u);
                 slot = kDone;
             }
-            while (found < (uint32_t)__popcll(idle) && next < end) {
+            while (found < (uint32_t)__popcll(idle) && next < n) {
                 const uint32_t e = next + __lane_id();
-                const uint32_t k = e < end ? w.skey[e] : a.sc.n_mats;
+                const uint32_t k = e < n ? w.skey[e] : a.sc.n_mats;
                 const bool layered = k < a.sc.n_mats && (lds_mats ? smats[k] : a.sc.mats[k]).n_layers > 1;
                 const uint64_t lm = __ballot(layered);
                 if (layered) list[found + (uint32_t)__popcll(lm & lt)] = e;
                 found += (uint32_t)__popcll(lm);
-                next += 64;
+                next += 64 * waves;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             if (!walking) {
@@ -979,7 +978,7 @@ __global__ __launch_bounds__(kShadeBlock<GUIDED>) __attribute__((amdgpu_waves_pe
 }
 
 // Every path of buffer A (count *cntA) run to its end in one launch: a wave
-// owns a contiguous share of the paths, up to 64 at a time in its lanes, and
+// owns a share of the paths, up to 64 at a time in its lanes, and
 // alternates between tracing their rays with its 16 quads and shading them in
 // place, at its own pace. For the last paths of a call, and all paths of a
 // small one, whose bounces would each take seven launches and wait for the
@@ -1009,10 +1008,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     __syncthreads();
     const uint32_t n = *cntA;
     const uint32_t waves = gridDim.x * (kBlock / 64);
-    const uint32_t share = (n + waves - 1) / waves;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
-    uint32_t next = min(n, wave * share);
-    const uint32_t end = min(n, next + share);
+    // this wave's paths, in chunks dealt to the waves in turn: long ones lie together
+    const uint32_t chunk = min(16u, (n + waves - 1) / waves);
+    const uint32_t end = n ? (n + waves * chunk - 1) / (waves * chunk) * chunk : 0u;
+    uint32_t next = 0;
     uint32_t* mine = slots[threadIdx.x >> 6];
     const uint64_t lt = __lanemask_lt();
     bool overflow = false;
@@ -1022,14 +1022,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const uint64_t need = ballot(slot == kDone);
         if (slot == kDone) {
             const uint32_t k = next + (uint32_t)lanes(need & lt);
-            if (k < end) {
-                slot = k;
+            const uint32_t at = k < end ? ((k / chunk) * waves + wave) * chunk + k % chunk : n;
+            if (at < n) {
+                slot = at;
                 segments = 0;
             }
         }
         next = min(end, next + (uint32_t)lanes(need));
         const uint64_t live = ballot(slot != kDone);
-        if (!live) break;
+        if (!live) {
+            if (next < end) continue;
+            break;
+        }
         const uint32_t m = (uint32_t)lanes(live);
         rays += m;
         if (slot != kDone) mine[lanes(live & lt)] = slot;
