@@ -130,8 +130,14 @@ __global__ __launch_bounds__(kBlock) void k_raycast_block(DevScene sc, DevCamera
         [&](uint32_t i, const Hit& h, V3 o, V3 d) { put_pixel<KIND>(sc, out, base + i, h, o, d); });
 }
 
-// Intersection-test count ray caster (int_test_count_raycaster.cpp:75-85).
-__global__ __launch_bounds__(kBlock) void k_raycast_count(DevScene sc, DevCamera cam, uint32_t* __restrict__ out,
+// Intersection-test count ray caster (int_test_count_raycaster.cpp:75-85): the
+// boxes and primitives the reference tests for the ray of each pixel, i.e.
+// every box of the binary tree whose parent the ray's line meets (no pruning
+// by t, so the order does not matter and no primitive is read).
+//
+// A ray per lane: bound by the longest rays' chains of node loads, and by its
+// instructions in small trees.
+__global__ __launch_bounds__(kBlock) void k_raycast_count_lane(DevScene sc, DevCamera cam, uint32_t* __restrict__ out,
                                                           uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
     __shared__ uint32_t lds[kLdsStack * kBlock];
     const uint32_t gthreads = gridDim.x * kBlock;
@@ -146,6 +152,111 @@ __global__ __launch_bounds__(kBlock) void k_raycast_count(DevScene sc, DevCamera
         uint32_t tests, isects;
         trace_ray<true>(sc, o, d, st, h, tests, isects, overflow);
         out[i] = tests;
+    }
+    if (overflow) atomicOr(flags, 1u);
+}
+
+// The four lanes of a quad share a ray and its stack: each round they take its
+// four top entries, a node each, and push the children that are met, those of
+// deeper nodes on top. A wave's 16 rays are a tile of 4 x 4 pixels. Bound by
+// the longest rays' chains of node loads, which take a quarter of the rounds
+// this way. Mesh of 1M triangles, a ray per lane before: 64x48 266 -> 68 us,
+// 185x305 545 -> 105, 640x480 686 -> 170, 1920x1080 852 -> 260. Tiles of 8 x 8
+// pixels whose rays are set up once and taken by free quads: 72, 113, 217, 348
+// (longer chains per wave).
+//
+// Stack entries: pops take the deepest nodes, so entries of a level are only
+// added once none of it is left, at most 8, and at most 4 stay once a deeper
+// level has entries: 4 per level and 8 are never exceeded (kCountSlack).
+constexpr int kCountStack = 24;  // entries of a ray in LDS, deeper ones spill
+constexpr uint32_t kCountSlack = 8;
+__host__ __device__ inline uint32_t count_stack_cap(uint32_t stack_cap) { return 4u * stack_cap + kCountSlack; }
+
+// Words of spill space a block needs.
+inline size_t count_spill_words(uint32_t stack_cap) {
+    const uint32_t cap = count_stack_cap(stack_cap);
+    return cap > (uint32_t)kCountStack ? (size_t)(cap - kCountStack) * kQuadsPerBlock : 0;
+}
+
+// Whether a ray per lane counts faster: a root that is a leaf has no nodes to
+// share, and with a small tree (short chains) and enough pixels to fill the chip
+// the quads' extra instructions cost more than the chains. 1920x1080, lane
+// against quad: 4,746 nodes 128 and 150 us, 9,568 nodes 162 and 159, 19,923
+// nodes 209 and 160; 4,746 nodes, 1280x960 125 and 125, 960x720 109 and 80.
+inline bool count_by_lane(const DevScene& sc, uint64_t pixels) {
+    return sc.root_leaf != 0 || (sc.n_nodes < 8192u && pixels > (1u << 20));
+}
+
+__global__ __launch_bounds__(kBlock) void k_raycast_count(DevScene sc, DevCamera cam, uint32_t* __restrict__ out,
+                                                          uint32_t* __restrict__ spill, uint32_t* __restrict__ flags) {
+    __shared__ uint32_t lds[kQuadsPerBlock][kCountStack + 1];  // odd row stride: spread over the banks
+    const uint32_t lane = __lane_id(), q4 = lane & 3u, quad = threadIdx.x >> 2, ray = lane >> 2;
+    lds_u32* stk = (lds_u32*)lds[quad];
+    // entry k at (k - kCountStack) * kQuadsPerBlock
+    const int cap = (int)count_stack_cap(sc.stack_cap);
+    glb_u32* deep = (glb_u32*)(spill + blockIdx.x * (size_t)max(cap - kCountStack, 0) * kQuadsPerBlock) + quad;
+    const uint32_t after = (0xEu << q4) & 0xFu;  // lanes of the quad that hold entries further down
+    const V3 rmn{sc.rmin[0], sc.rmin[1], sc.rmin[2]}, rmx{sc.rmax[0], sc.rmax[1], sc.rmax[2]};
+    const uint64_t tiles_x = ((uint64_t)cam.width + 3) / 4, tiles = tiles_x * (((uint64_t)cam.height + 3) / 4);
+    const uint64_t waves = (uint64_t)gridDim.x * (kBlock / 64);
+    bool overflow = false;
+    for (uint64_t tile = (uint64_t)blockIdx.x * (kBlock / 64) + threadIdx.x / 64; tile < tiles; tile += waves) {
+        // a 32-bit division takes a fifth of the instructions
+        const uint64_t ty = tile >> 32 ? tile / tiles_x : (uint32_t)tile / (uint32_t)tiles_x;
+        const uint64_t x = (tile - ty * tiles_x) * 4 + (ray & 3u), y = ty * 4 + (ray >> 2);
+        const bool inside = x < cam.width && y < cam.height;
+        const uint64_t i = inside ? y * cam.width + x : 0;
+        V3 o, d;
+        pixel_ray(cam, i, o, d);
+        const V3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+        float tn, tf;
+        uint32_t tests = q4 == 0u ? 1u : 0u;
+        int sp = 0;
+        if (inside && slab(o, inv, rmn, rmx, tn, tf)) {
+            sp = 1;
+            if (q4 == 0u) stk[0] = 0u;
+        }
+        while (ballot(sp > 0)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            bool hl = false, hr = false;
+            uint4 r{};
+            if ((int)q4 < sp) {
+                const int at = sp - 1 - (int)q4;
+                const uint32_t node = at < kCountStack ? stk[at] : deep[(size_t)(at - kCountStack) * kQuadsPerBlock];
+                const float4* np = sc.nodes + 4 * (size_t)node;
+                const float4 a = np[0], b = np[1], c = np[2];
+                r = reinterpret_cast<const uint4*>(np)[3];
+                hl = slab(o, inv, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, tn, tf);
+                hr = slab(o, inv, V3{b.z, b.w, c.x}, V3{c.y, c.z, c.w}, tn, tf);
+                tests += 2u + (hl ? r.y : 0u) + (hr ? r.w : 0u);  // a leaf's primitives are all tested
+                hl = hl && r.y == 0u;
+                hr = hr && r.w == 0u;
+            }
+            const uint32_t ml = (uint32_t)(ballot(hl) >> (lane & 60u)) & 0xFu;
+            const uint32_t mr = (uint32_t)(ballot(hr) >> (lane & 60u)) & 0xFu;
+            sp = max(sp - 4, 0);
+            const int added = __popc(ml) + __popc(mr);
+            if (sp + added > cap) {
+                overflow = true;
+                sp = 0;
+                continue;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // all entries are read before their places are reused
+            int at = sp + __popc(ml & after) + __popc(mr & after);
+            auto put = [&](uint32_t node) {
+                if (at < kCountStack)
+                    stk[at] = node;
+                else
+                    deep[(size_t)(at - kCountStack) * kQuadsPerBlock] = node;
+                ++at;
+            };
+            if (hr) put(r.z);
+            if (hl) put(r.x);
+            sp += added;
+        }
+        tests += (uint32_t)__shfl_xor((int)tests, 1);
+        tests += (uint32_t)__shfl_xor((int)tests, 2);
+        if (inside && q4 == 0u) out[i] = tests;
     }
     if (overflow) atomicOr(flags, 1u);
 }
@@ -381,11 +492,21 @@ spt_status launch_raycast(spt_ctx* ctx, const spt_camera* cam, uint32_t kind, vo
                                    base, cnt, out, ctx->d_spill, ctx->d_flags, ctx->d_rays, refill_of(ctx));
             },
             "raycast launch");
-    const uint32_t grid = grid_for(ctx, n);
-    spt_status s = ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap > kLdsStack ? ctx->stack_cap - kLdsStack : 1));
-    if (s != SPT_OK) return s;
-    hipLaunchKernelGGL(k_raycast_count, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc,
-                       reinterpret_cast<uint32_t*>(d_out), ctx->d_spill, ctx->d_flags);
+    uint32_t* counts = reinterpret_cast<uint32_t*>(d_out);
+    if (count_by_lane(sc, n)) {
+        const uint32_t grid = grid_for(ctx, n);
+        spt_status s = ensure_spill(ctx, (size_t)grid * kBlock * (ctx->stack_cap > kLdsStack ? ctx->stack_cap - kLdsStack : 1));
+        if (s != SPT_OK) return s;
+        hipLaunchKernelGGL(k_raycast_count_lane, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, counts, ctx->d_spill,
+                           ctx->d_flags);
+    } else {
+        const uint64_t tiles = (((uint64_t)dc.width + 3) / 4) * (((uint64_t)dc.height + 3) / 4);
+        const uint32_t grid = (uint32_t)std::min<uint64_t>((tiles + kBlock / 64 - 1) / (kBlock / 64), (uint64_t)ctx->num_cus * 16);
+        spt_status s = ensure_spill(ctx, std::max<size_t>(1, grid * count_spill_words(sc.stack_cap)));
+        if (s != SPT_OK) return s;
+        hipLaunchKernelGGL(k_raycast_count, dim3(grid), dim3(kBlock), 0, ctx->stream, sc, dc, counts, ctx->d_spill,
+                           ctx->d_flags);
+    }
     return check_hip(ctx, hipGetLastError(), "raycast launch");
 }
 

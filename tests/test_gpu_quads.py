@@ -118,3 +118,27 @@ def test_scenes_of_one_block(device, spheres, triangles, distance):
         r[::9, 0:3] = rng.uniform(-0.3, 0.3, r[::9, 0:3].shape)
         r[::101, 5] = np.nan
         _check(device, v, r, kinds=kinds)
+
+
+@pytest.mark.parametrize("width, height", [(1, 1), (3, 5), (4, 4), (17, 2), (131, 67)])
+def test_count_caster_at_ragged_sizes(device, width, height):
+    """Tiles of 4 x 4 pixels and their remainders, stacks in LDS only and beyond
+    it, a scene whose root is a leaf. Counts are whole numbers: equal."""
+    cam = dict(position=(0.2, 0.3, 2.5), look_at=(0, 0, 0), fov=50.0)
+    mesh = scenes.displaced_mesh(rings=48, segments=96)
+    rng = np.random.default_rng(width * 1000 + height)
+    # long thin overlapping triangles: rays meet most boxes of the tree
+    heap = rng.uniform(-1, 1, (600, 3, 3)).astype(np.float32)
+    for verts in (mesh.verts, heap, mesh.verts.reshape(-1, 3, 3)[:2]):
+        device.set_scene(api.Bvh(verts))
+        c = api.pinhole(width, height, **cam)
+        assert np.array_equal(device.raycast(c, L.SPT_RAYCAST_COUNT), O.Scene(verts).raycast(c, 2))
+
+
+@pytest.mark.parametrize("width, height", [(1024, 1024), (1031, 1025)])
+def test_count_caster_around_the_pixel_limit(device, width, height):
+    """A small tree just below and above the size from which a lane counts a ray."""
+    verts = scenes.displaced_mesh(rings=12, segments=24).verts
+    device.set_scene(api.Bvh(verts))
+    c = api.pinhole(width, height, position=(0.2, 0.3, 2.5), look_at=(0, 0, 0), fov=50.0)
+    assert np.array_equal(device.raycast(c, L.SPT_RAYCAST_COUNT), O.Scene(verts).raycast(c, 2))
