@@ -314,8 +314,6 @@ def guide_experiment(args):
     # inference: one more 144-spp guided pass (trained guide, no capture) with
     # the inference launches timed by HIP events; 25,600 useful FLOP per query
     # (32x64 + 64x64 + 64x64 + 64x40 multiply-adds)
-    # (one wavefront, so that no other wavefront's kernels share the timed
-    # launches)
     dev.set_tuning(wavefronts=1, path_capacity=args.guide_capacity)
     p = integ.params()
     p.spp, p.seed = 144, 0x1FE12
@@ -326,10 +324,10 @@ def guide_experiment(args):
     rs = dev.render_stats()
     dev.set_tuning(path_capacity=args.guide_capacity)
     inf_tflops = rs["guide_queries"] * 25600 / max(rs["guide_ms"] * 1e-3, 1e-12) / 1e12
-    # its memory side: per query 104 B read (queue index 4, hit 16, sort key 4,
+    # its memory side: per query 100 B read (hit 16, material 4,
     # origin 16, direction 16, the triangle's shading record 48) and 80 B of
     # half-float outputs written
-    inf_gbs = rs["guide_queries"] * 184 / max(rs["guide_ms"] * 1e-3, 1e-12) / 1e9
+    inf_gbs = rs["guide_queries"] * 180 / max(rs["guide_ms"] * 1e-3, 1e-12) / 1e9
     infer = {"queries": int(rs["guide_queries"]), "kernel_ms": round(rs["guide_ms"], 3),
              "tflops": round(inf_tflops, 1), "mfma_util": round(inf_tflops / 2500.0, 4),
              "algorithmic_gbs": round(inf_gbs, 1), "hbm_frac": round(inf_gbs / HBM_PEAK_GBS, 4)}
@@ -519,25 +517,12 @@ def main():
     fs = dev.render_stats()
     per_ray_nodes = fs["node_fetches"] / fs["rays"]
     per_ray_tris = fs["tri_fetches"] / fs["rays"]
-    # per extension ray: queue index 4 + origin 16 + direction 16 in, hit 16 + sort key 4 out
-    bytes_per_ray = 56 + 32 * per_ray_nodes + 48 * per_ray_tris  # tree data counted in 32-B units
+    # per extension ray: origin 16 + direction 16 in, hit 16 + material 4 out
+    bytes_per_ray = 52 + 32 * per_ray_nodes + 48 * per_ray_tris  # tree data counted in 32-B units
     achieved = bytes_per_ray * rays / (ext_ms * 1e-3) / 1e9
-    # The renderer runs concurrent wavefronts, so an extension launch shares
-    # the GPU with another wavefront's shading and lasts longer than it would
-    # alone. Beside the per-launch figure: the extension rays' algorithmic
-    # bytes over the whole timed wall time, and one untimed step on a single
-    # wavefront (the kernel with the GPU to itself).
+    # Beside the per-launch figure: the extension rays' algorithmic bytes over
+    # the whole timed wall time (the launches between them are shading).
     aggregate = bytes_per_ray * rays / wall / 1e9
-    tn_default = dev.get_tuning()
-    dev.set_tuning(wavefronts=1)  # the other fields at their one-wavefront defaults
-    step(0, L.SPT_RENDER_FILM32 | L.SPT_RENDER_TIME_KERNELS)
-    dev.sync()
-    si = dev.render_stats()
-    dev.set_tuning()  # back to the library defaults
-    single = {"avg_launch_ms": round(si["extend_ms"] / max(si["extend_launches"], 1), 4),
-              "launches": int(si["extend_launches"]),
-              "achieved": round(bytes_per_ray * si["rays"] / (si["extend_ms"] * 1e-3) / 1e9, 1)}
-    single["frac"] = round(single["achieved"] / HBM_PEAK_GBS, 4)
 
     # HBM bytes per extension launch of this workload, from the committed
     # rocprofv3 FETCH_SIZE / WRITE_SIZE passes (copy-calibrated)
@@ -546,8 +531,8 @@ def main():
     if os.path.exists(tf) and args.rings == 512 and args.segments == 1024:
         with open(tf) as fh:
             tj = json.load(fh)
-        # measured on this workload's launches, with as many wavefronts
-        if tj.get("spp_per_step") == sps and tj.get("wavefronts", 1) == tn_default["wavefronts"]:
+        # measured on this workload's launches, on one wavefront (the default)
+        if tj.get("spp_per_step") == sps and tj.get("wavefronts", 1) == 1:
             traffic = tj["hbm_bytes_per_launch"]
 
     extra = {}
@@ -643,9 +628,8 @@ def main():
                      "bytes_per_ray": round(bytes_per_ray, 1), "tree_units_32B_per_ray": round(per_ray_nodes, 2),
                      "tri_fetches_per_ray": round(per_ray_tris, 2),
                      "avg_launch_ms": round(ext_ms / max(ext_n, 1), 4), "launches": ext_n,
-                     "wavefronts": tn_default["wavefronts"],
-                     "aggregate_achieved": round(aggregate, 1), "aggregate_frac": round(aggregate / HBM_PEAK_GBS, 4),
-                     "single_wavefront": single},
+                     "wavefronts": 1,
+                     "aggregate_achieved": round(aggregate, 1), "aggregate_frac": round(aggregate / HBM_PEAK_GBS, 4)},
         "cpu_baseline": cpu,
         "image_mean": [round(float(x), 5) for x in img.reshape(-1, 3).mean(0)],
     }

@@ -350,7 +350,7 @@ typedef struct spt_render_stats {
     uint64_t node_fetches;
     uint64_t tri_fetches;
     double guide_ms;       /* with SPT_RENDER_TIME_KERNELS and GUIDED: guide inference time */
-    uint64_t guide_queries; /* GUIDED with the material sort: hits the guide network evaluated */
+    uint64_t guide_queries; /* GUIDED: hits the guide network evaluated */
 } spt_render_stats;
 spt_status spt_render_get_stats(spt_ctx* ctx, spt_render_stats* out);
 
@@ -385,8 +385,8 @@ typedef struct spt_tuning {
                                       several; 20 in spt_trace) */
     uint32_t wavefronts;           /* independent wavefronts run at once on their own streams, each
                                       with a share of the paths and of the queue capacity, so
-                                      one's traversal overlaps another's shading (1..4, default 3;
-                                      left at the default, a plain render of one scene uses one) */
+                                      one's traversal overlaps another's shading (1..4; reported as 3
+                                      when left at zero, which runs one) */
 } spt_tuning;
 spt_status spt_set_tuning(spt_ctx* ctx, const spt_tuning* t);
 spt_status spt_get_tuning(spt_ctx* ctx, spt_tuning* t);
