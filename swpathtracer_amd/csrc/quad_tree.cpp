@@ -16,8 +16,9 @@
 // more than small triangles need: the traversal only has to reach every
 // candidate the reference would accept, and such a candidate lies on its
 // triangle up to the rounding of the triangle test. So the boxes here are the
-// given ones cut to the primitives' bounds plus a padding of their own
-// (prim_pad). The mesh in the box goes from 10.3 to 8.3 steps for rays off its
+// given ones cut to the triangles' bounds plus a padding of their own
+// (prim_pad); leaves with spheres keep theirs. The mesh in the box goes from
+// 10.3 to 8.3 steps for rays off its
 // surfaces, the longest of a million of them from 1036 to 651 (near the poles
 // of the displaced sphere hundreds of slivers are thinner than 1e-3).
 #include "quad_tree.h"
@@ -69,7 +70,7 @@ struct Box {
     float lo[3], hi[3];
 };
 
-// Padding of a primitive's box: how far the point where a ray crosses the
+// Padding of a triangle's box: how far the point where a ray crosses the
 // plane can be from the point (u, v, t) of a float triangle test that accepts
 // it. In units of 2^-24 |o - v0| |e1| |e2| / |det| the two are at most 2.7
 // apart in the plane and 5.3 along the ray (9 million accepted tests, grazing
@@ -78,9 +79,8 @@ struct Box {
 // of the root box: ray origins within one diagonal of its centre, unit
 // directions; the traversal widens the boxes for other rays) are
 // 0.5 * reach * |e1| |e2|. At least the rounding of the box tests themselves,
-// at most the reference's 1e-3. Spheres keep that.
+// at most the reference's 1e-3.
 float prim_pad(const spt_tri48& t, float reach, float least) {
-    if (t.pad[1] == SPT_PRIM_SPHERE) return 1e-3f;
     auto len = [](const float* e) { return std::sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]); };
     const float p = std::max(0.5f * reach * len(t.e1) * len(t.e2), least);
     return p < 1e-3f ? p : 1e-3f;
@@ -110,9 +110,9 @@ public:
         if (n_ == 0) {  // the root is a leaf: its box is the (unpadded) root box
             Part p;
             p.kind = Part::kRange;
-            for (int k = 0; k < 3; ++k) {  // all primitives are candidates: only their own bounds count
-                p.box.lo[k] = -std::numeric_limits<float>::infinity();
-                p.box.hi[k] = std::numeric_limits<float>::infinity();
+            for (int k = 0; k < 3; ++k) {  // hit points are accepted up to 1e-3 outside the box
+                p.box.lo[k] = std::nextafter(root_box[k] - 2e-3f, -std::numeric_limits<float>::infinity());
+                p.box.hi[k] = std::nextafter(root_box[3 + k] + 2e-3f, std::numeric_limits<float>::infinity());
             }
             p.first = 0;
             p.count = n_tris;
@@ -171,28 +171,31 @@ private:
         Part part;
     };
 
-    // A primitive's bounds and padding (in double, rounded outward).
+    // A triangle's bounds and padding (in double, rounded outward).
     void prim_box(uint32_t tri, Box& b) const {
         const spt_tri48& t = tris_[tri];
         const double pad = prim_pad(t, reach_, least_);
         for (int k = 0; k < 3; ++k) {
-            double lo, hi;
-            if (t.pad[1] == SPT_PRIM_SPHERE) {
-                lo = (double)t.v0[k] - t.e1[0];
-                hi = (double)t.v0[k] + t.e1[0];
-            } else {
-                const double v0 = t.v0[k], v1 = v0 + t.e1[k], v2 = v0 + t.e2[k];
-                lo = std::min(v0, std::min(v1, v2));
-                hi = std::max(v0, std::max(v1, v2));
-            }
+            const double v0 = t.v0[k], v1 = v0 + t.e1[k], v2 = v0 + t.e2[k];
+            const double lo = std::min(v0, std::min(v1, v2)), hi = std::max(v0, std::max(v1, v2));
             b.lo[k] = std::nextafter((float)(lo - pad), -std::numeric_limits<float>::infinity());
             b.hi[k] = std::nextafter((float)(hi + pad), std::numeric_limits<float>::infinity());
         }
     }
 
-    // Bounds of primitives [first, first + count).
+    // Bounds of primitives [first, first + count). None with spheres among them:
+    // their test accepts hit points off the sphere when the direction is not of
+    // unit length, anywhere in the box of the leaf.
     Box range_box(uint32_t first, uint32_t count) const {
         Box u;
+        for (uint32_t i = 0; i < count; ++i)
+            if (tris_[first + i].pad[1] == SPT_PRIM_SPHERE) {
+                for (int k = 0; k < 3; ++k) {
+                    u.lo[k] = -std::numeric_limits<float>::infinity();
+                    u.hi[k] = std::numeric_limits<float>::infinity();
+                }
+                return u;
+            }
         prim_box(first, u);
         for (uint32_t i = 1; i < count; ++i) {
             Box b;

@@ -142,3 +142,27 @@ def test_count_caster_around_the_pixel_limit(device, width, height):
     device.set_scene(api.Bvh(verts))
     c = api.pinhole(width, height, position=(0.2, 0.3, 2.5), look_at=(0, 0, 0), fov=50.0)
     assert np.array_equal(device.raycast(c, L.SPT_RAYCAST_COUNT), O.Scene(verts).raycast(c, 2))
+
+
+@pytest.mark.parametrize("n_spheres, n_tris", [(1, 9), (9, 3), (6, 40)])
+@pytest.mark.parametrize("length", [0.5, 1.0, 3.0])
+def test_spheres_in_large_leaves(device, n_spheres, n_tris, length):
+    """With directions that are not of unit length the sphere test accepts hit
+    points off the sphere, anywhere in its leaf's box: a leaf's parts that hold
+    spheres keep that box. Equal centroids make one leaf of all of them."""
+    rng = np.random.default_rng(100 * n_spheres + n_tris)
+    verts = np.zeros((n_spheres + n_tris, 9), np.float32)
+    kinds = np.zeros(n_spheres + n_tris, np.uint32)
+    verts[:n_spheres, 3] = rng.uniform(0.02, 0.3, n_spheres)
+    kinds[:n_spheres] = L.SPT_PRIM_SPHERE
+    a, b = rng.uniform(-1, 1, (2, n_tris, 3))
+    verts[n_spheres:] = np.concatenate([a, b, -a - b], axis=1)
+    hit = _check(device, verts, _rays(rng, 20000, -2, 2, length), kinds)
+    assert 0.0 < hit < 1.0
+    # the same beside a distant group, so that the leaf is not the root
+    far = verts.copy()
+    far[:n_spheres, 0:3] += 8
+    far[n_spheres:] += 8
+    rays = _rays(rng, 20000, -2, 2, length)
+    rays[::2, 0:3] += 8
+    _check(device, np.concatenate([verts, far]), rays, np.concatenate([kinds, kinds]))
