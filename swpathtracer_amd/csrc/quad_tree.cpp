@@ -18,9 +18,9 @@
 // triangle up to the rounding of the triangle test. So the boxes here are the
 // given ones cut to the triangles' bounds plus a padding of their own
 // (prim_pad); leaves with spheres keep theirs. The mesh in the box goes from
-// 10.3 to 8.3 steps for rays off its
-// surfaces, the longest of a million of them from 1036 to 651 (near the poles
-// of the displaced sphere hundreds of slivers are thinner than 1e-3).
+// 10.3 to 8.3 steps for rays off its surfaces, the longest of a million of them
+// from 1036 to 651 (near the poles of the displaced sphere hundreds of slivers
+// are thinner than 1e-3).
 #include "quad_tree.h"
 
 #include <algorithm>

@@ -150,14 +150,15 @@ __device__ inline bool accept_exact(const DevScene& sc, V3 o, V3 d, float t, uin
 // point at (u, v) of a triangle lies inside its leaf's box, which holds the
 // vertices, so a hit point within 5e-4 of it lies inside the box +-1e-3 (with
 // coordinates up to 1024 the rounding of the triangle's point is below 2e-4).
-// A sphere (u = v = 0, v0 = centre) reaches its radius further, as its box
-// does. Saves the load of the box, which the whole wave would wait for.
+// A sphere (u = v = 0, v0 = centre) reaches its radius, as its box does, and no
+// further: its hit point may lie off it, and a root leaf's box, which the ray has
+// to meet, has no padding. Saves the load of the box, which the whole wave would wait for.
 __device__ inline bool accept_near(V3 o, V3 d, float t, float u, float v, V3 v0, V3 e1, V3 e2, float radius) {
     const V3 p = o + d * t;
     const float x = p.x - fmaf(u, e1.x, fmaf(v, e2.x, v0.x));
     const float y = p.y - fmaf(u, e1.y, fmaf(v, e2.y, v0.y));
     const float z = p.z - fmaf(u, e1.z, fmaf(v, e2.z, v0.z));
-    return fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) <= 5e-4f + radius;
+    return fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) <= (radius > 0.0f ? radius : 5e-4f);
 }
 
 // How the waves of a launch share its rays: groups of `chunk` rays dealt to

@@ -166,3 +166,15 @@ def test_spheres_in_large_leaves(device, n_spheres, n_tris, length):
     rays = _rays(rng, 20000, -2, 2, length)
     rays[::2, 0:3] += 8
     _check(device, np.concatenate([verts, far]), rays, np.concatenate([kinds, kinds]))
+
+
+@pytest.mark.parametrize("n", [1, 4, 7])
+@pytest.mark.parametrize("length", [0.5, 1.0, 3.0])
+def test_spheres_in_a_root_leaf(device, n, length):
+    """The root's box has no padding: a hit point accepted off the sphere does
+    not mean that the ray meets it. Many rays pass close to the box."""
+    rng = np.random.default_rng(n)
+    verts = np.zeros((n, 9), np.float32)
+    verts[:, 3] = rng.uniform(0.2, 0.5, n)
+    kinds = np.full(n, L.SPT_PRIM_SPHERE, np.uint32)
+    _check(device, verts, _rays(rng, 400000, -1, 1, length), kinds)
