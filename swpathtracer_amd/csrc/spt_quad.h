@@ -570,22 +570,26 @@ __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray
 }
 
 // Rays 0 .. n - 1 against a scene whose tree is one block (at most four
-// primitives): a ray per lane, no tree, pool, stack or root box. The same candidates are
-// accepted as in the block step above. 185x305 depth image of a sphere
-// 4 us, 11.5 with the quads, whose set-up and rounds a wave are latency here;
-// 1900x1050 13 us. Bound by VALU issue.
+// primitives in a root leaf): a ray per lane, no tree, pool or stack. The same
+// candidates are accepted as in the block step above, and then the ray has to
+// meet the root's box, as the reference asks before it tests the leaf
+// (acceleration/sbvh.cpp:423-515): that box has no padding, so a ray towards a
+// vertex or edge on it may miss it by a rounding. Only hits pay for that test.
+// 185x305 depth image of a sphere 4 us, 11.5 with the quads, whose set-up and
+// rounds a wave are latency here; 1900x1050 13 us. Bound by VALU issue.
 template <typename GetRay, typename PutHit>
 __device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay get_ray, PutHit put_hit) {
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         V3 o, d;
         get_ray(i, o, d);
         const float sum = o.x + o.y + o.z + d.x + d.y + d.z;
-        Hit h;
-        h.t = __builtin_inff();
-        h.idx = kNoHit;
-        h.mat = 0;
-        h.u = h.v = 0.0f;
-        if (sum - sum == 0.0f) {  // the root box would cost more than the primitives
+        Hit miss;
+        miss.t = __builtin_inff();
+        miss.idx = kNoHit;
+        miss.mat = 0;
+        miss.u = miss.v = 0.0f;
+        Hit h = miss;
+        if (sum - sum == 0.0f) {
             const float4* tp = reinterpret_cast<const float4*>(sc.qprims);
             for (int k = 0; k < 4; ++k) {
                 const float4 a = tp[3 * k], b = tp[3 * k + 1], c = tp[3 * k + 2];
@@ -608,6 +612,9 @@ __device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay ge
                     h.v = v;
                 }
             }
+            const Root r = scene_root(sc);
+            float tn, tf;
+            if (h.idx != kNoHit && !slab(o, V3{1.0f / d.x, 1.0f / d.y, 1.0f / d.z}, r.mn, r.mx, tn, tf)) h = miss;
         }
         put_hit(i, h, o, d);
     }

@@ -1,0 +1,67 @@
+"""Rays that the acceptance rules decide by a rounding, ids and t bit for bit
+against the oracle (acceleration/sbvh.cpp:423-515): the root's box has no
+padding, so a ray towards a vertex or edge that spans it may miss the box and
+still pass the primitive's test."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from swpathtracer_amd import api, scenes
+import swpathtracer_amd._lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+def _towards(rng, points, distance, length=1.0):
+    """One ray per point, from `distance` away on average."""
+    r = np.zeros((len(points), 8), np.float32)
+    d = rng.normal(size=(len(points), 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    r[:, 0:3] = points - d * distance * rng.uniform(0.5, 1.5, (len(points), 1))
+    r[:, 4:7] = length * d
+    return r
+
+
+def _same(got, want):
+    (t, p), (t_c, p_c) = got, want
+    assert np.array_equal(p, p_c), f"{np.sum(p != p_c)} of {len(p)} ids differ"
+    hit = p_c != L.SPT_MISS
+    assert np.array_equal(t[hit].view(np.uint32), t_c[hit].view(np.uint32))
+    assert np.all(np.isinf(t[~hit]))
+    return hit.mean()
+
+
+def _check(device, verts, rays, kinds=None):
+    device.set_scene(api.Bvh(verts, kinds=kinds))
+    return _same(device.trace_host(rays), O.Scene(verts, kinds=kinds).trace(rays)[:2])
+
+
+def _vertices_and_edges(rng, verts, n):
+    """Half of the points on vertices, half on edges."""
+    v = verts.reshape(-1, 3, 3)[rng.integers(len(verts), size=n)]
+    a, b = v[np.arange(n), rng.integers(3, size=n)], v[np.arange(n), rng.integers(3, size=n)]
+    w = rng.uniform(0, 1, (n, 1)).astype(np.float32)
+    w[::2] = 0
+    return a + (b - a) * w
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_vertices_and_edges_in_one_block(device, n):
+    """Random triangles, and n pieces of a floor whose box is flat."""
+    rng = np.random.default_rng(n)
+    for _ in range(4):
+        v = rng.uniform(-1, 1, (n, 9)).astype(np.float32)
+        hit = _check(device, v, _towards(rng, _vertices_and_edges(rng, v, 50_000), 1.5))
+        assert 0.1 < hit < 0.9
+    floor = rng.uniform(-1, 1, (n, 3, 3)).astype(np.float32)
+    floor[:, :, 1] = 0.25
+    _check(device, floor.reshape(n, 9), _towards(rng, _vertices_and_edges(rng, floor, 50_000), 1.5))
+
+
+def test_ray_beside_a_root_leaf(device):
+    """A ray that meets the triangle by its own test and misses its box by 1e-7."""
+    v = np.array([[0.0442627668, -0.762663662, -0.288553238, 0.700170398, 0.0994391441, -0.193311572, -0.0341354012,
+                   0.456554413, -0.777606249]], np.float32)
+    r = np.array([[1.23511338, 1.47528875, -1.42693853, 0, -0.27806744, -0.715177178, 0.641248763, 0]], np.float32)
+    assert O.Scene(v).trace(r)[1][0] == L.SPT_MISS
+    _check(device, v, r)
