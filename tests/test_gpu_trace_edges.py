@@ -65,3 +65,15 @@ def test_ray_beside_a_root_leaf(device):
     r = np.array([[1.23511338, 1.47528875, -1.42693853, 0, -0.27806744, -0.715177178, 0.641248763, 0]], np.float32)
     assert O.Scene(v).trace(r)[1][0] == L.SPT_MISS
     _check(device, v, r)
+
+
+@pytest.mark.parametrize("n", [7, 60, 500])
+def test_vertices_that_span_the_root(device, n):
+    """The same in scenes with a tree: rays towards the extreme vertices."""
+    rng = np.random.default_rng(n)
+    v = rng.uniform(-0.7, 0.7, (n, 9)).astype(np.float32)
+    v[:6] *= np.float32(1.4)
+    p = v.reshape(-1, 3)
+    extreme = np.concatenate([p[p.argmin(0)], p[p.argmax(0)]])
+    hit = _check(device, v, _towards(rng, np.repeat(extreme, 20_000, axis=0), 1.5))
+    assert hit > 0.1
