@@ -117,16 +117,20 @@ __device__ inline bool root_test(V3 o, V3 d, V3 inv, V3 mn, V3 mx) {
 
 // What a ray adds to the tree's box paddings (prim_pad in quad_tree.cpp): they
 // cover rays of at most unit length whose origin is within a diagonal of the
-// root box of its centre. The error they stand for grows with the distance;
-// adding 1e-3 gives boxes no smaller than the reference's, and the second
-// term covers the rounding of the box tests at that distance.
+// root box of its centre. The error they stand for grows with the distance and
+// with the length; adding 1e-3 gives boxes no smaller than the reference's. The
+// rounding of the box tests grows with the distance whatever the length (the
+// second term: without it 25 of a million rays of length 2 from 60,000 away lost
+// their hit). It opens the more boxes the farther a ray starts: 65,536 rays
+// into the 1M-triangle mesh in the box, of size 2, 0.26 ms from 100 away, 0.81
+// from 5,000, 11 from 60,000.
 __device__ inline float ray_slack(const Root& r, V3 o, V3 d) {
-    if (!(dot(d, d) <= 1.002f)) return 1e-3f;
+    const bool longer = !(dot(d, d) <= 1.002f);
     const V3 e = r.mx - r.mn, c = o - (r.mn + e * 0.5f);
     const float diag2 = dot(e, e), far2 = dot(c, c);
-    if (far2 <= diag2) return 0.0f;
+    if (!(far2 > diag2)) return longer ? 1e-3f : 0.0f;
     const float far = sqrtf(far2);
-    return fminf(1e-3f, 1e-3f * (far / sqrtf(diag2) - 1.0f)) + 1e-6f * far;
+    return (longer ? 1e-3f : fminf(1e-3f, 1e-3f * (far / sqrtf(diag2) - 1.0f))) + 1e-6f * far;
 }
 
 template <int CTRL>

@@ -77,3 +77,15 @@ def test_vertices_that_span_the_root(device, n):
     extreme = np.concatenate([p[p.argmin(0)], p[p.argmax(0)]])
     hit = _check(device, v, _towards(rng, np.repeat(extreme, 20_000, axis=0), 1.5))
     assert hit > 0.1
+
+
+@pytest.mark.parametrize("distance, length", [(60.0, 2.0), (5000.0, 2.0), (60_000.0, 2.0), (60_000.0, 30.0),
+                                              (60_000.0, 1.0)])
+def test_far_rays_of_any_length(device, distance, length):
+    """The rounding of the box tests grows with the distance, whatever the
+    length of the direction."""
+    rng = np.random.default_rng(int(distance + length))
+    v = (rng.uniform(-1, 1, (4000, 1, 3)) + rng.uniform(-0.02, 0.02, (4000, 3, 3))).astype(np.float32).reshape(-1, 9)
+    c = v.reshape(-1, 3, 3).mean(1)
+    rays = _towards(rng, c[rng.integers(len(c), size=1_000_000)], distance, length)
+    assert _check(device, v, rays) > 0.3
