@@ -17,7 +17,10 @@
 // candidate the reference would accept, and such a candidate lies on its
 // triangle up to the rounding of the triangle test. So the boxes here are the
 // given ones cut to the triangles' bounds plus a padding of their own
-// (prim_pad); leaves with spheres keep theirs. The mesh in the box goes from
+// (prim_pad). Not so a leaf with spheres, or whose box does not hold its
+// primitives (an uploaded tree may clip them): there hits are accepted off the
+// primitive, or outside the box, so such leaves and the nodes above them get the
+// leaf's box and the 1e-3 around it that its acceptance allows. The mesh in the box goes from
 // 10.3 to 8.3 steps for rays off its surfaces, the longest of a million of them
 // from 1036 to 651 (near the poles of the displaced sphere hundreds of slivers
 // are thinner than 1e-3).
@@ -110,17 +113,15 @@ public:
         if (n_ == 0) {  // the root is a leaf: its box is the (unpadded) root box
             Part p;
             p.kind = Part::kRange;
-            for (int k = 0; k < 3; ++k) {  // hit points are accepted up to 1e-3 outside the box
-                p.box.lo[k] = std::nextafter(root_box[k] - 2e-3f, -std::numeric_limits<float>::infinity());
-                p.box.hi[k] = std::nextafter(root_box[3 + k] + 2e-3f, std::numeric_limits<float>::infinity());
+            for (int k = 0; k < 3; ++k) {
+                p.box.lo[k] = root_box[k];
+                p.box.hi[k] = root_box[3 + k];
             }
             p.first = 0;
             p.count = n_tris;
-            QuadBox b{};
-            std::memcpy(b.mn, root_box, sizeof(b.mn));
-            std::memcpy(b.mx, root_box + 3, sizeof(b.mx));
-            out_.boxes.push_back(b);
-            p.leaf_box = (uint32_t)out_.boxes.size() - 1;
+            p.loose = loose(p.box, 0, n_tris);
+            p.leaf_box = add_box(p.box, 0, n_tris);
+            widen(p.box);
             work.push_back({root, 1, 0, true, p});
         } else {
             plan();
@@ -164,6 +165,7 @@ private:
         uint32_t bin = 0;              // kInner, kMerged: binary node
         uint32_t first = 0, count = 0; // kRange (part of one leaf), kMerged (a subtree of several)
         uint32_t leaf_box = 0;         // kRange
+        bool loose = false;            // kRange: parts of it keep its box
     };
     struct Work {
         uint32_t slot, depth, bin;
@@ -183,19 +185,45 @@ private:
         }
     }
 
-    // Bounds of primitives [first, first + count). None with spheres among them:
-    // their test accepts hit points off the sphere when the direction is not of
-    // unit length, anywhere in the box of the leaf.
+    // Whether the box of a leaf reaches as far as its primitives (to 1e-4, which
+    // the rounding of v0 + e1 and the acceptance shortcut leave room for).
+    bool holds(const Item& e, uint32_t first, uint32_t count) const {
+        for (uint32_t i = first; i < first + count; ++i) {
+            const spt_tri48& t = tris_[i];
+            for (int k = 0; k < 3; ++k) {
+                double lo = t.v0[k], hi = lo;
+                if (t.pad[1] == SPT_PRIM_SPHERE) {
+                    lo -= std::fabs((double)t.e1[0]);
+                    hi += std::fabs((double)t.e1[0]);
+                } else {
+                    const double v1 = lo + t.e1[k], v2 = lo + t.e2[k];
+                    lo = std::min(lo, std::min(v1, v2));
+                    hi = std::max(hi, std::max(v1, v2));
+                }
+                if (!(lo >= (double)e.lo[k] - 1e-4 && hi <= (double)e.hi[k] + 1e-4)) return false;
+            }
+        }
+        return true;
+    }
+    // Whether hits in a leaf are not accepted at its primitives alone: a sphere's
+    // test accepts hit points off it when the direction is not of unit length.
+    bool loose(const Item& e, uint32_t first, uint32_t count) const {
+        for (uint32_t i = first; i < first + count; ++i)
+            if (tris_[i].pad[1] == SPT_PRIM_SPHERE) return true;
+        return !holds(e, first, count);
+    }
+    // Hit points are accepted up to 1e-3 outside their leaf's box.
+    template <typename E>
+    static void widen(E& e) {
+        for (int k = 0; k < 3; ++k) {
+            e.lo[k] = std::nextafter(e.lo[k] - 2e-3f, -std::numeric_limits<float>::infinity());
+            e.hi[k] = std::nextafter(e.hi[k] + 2e-3f, std::numeric_limits<float>::infinity());
+        }
+    }
+
+    // Bounds of triangles [first, first + count).
     Box range_box(uint32_t first, uint32_t count) const {
         Box u;
-        for (uint32_t i = 0; i < count; ++i)
-            if (tris_[first + i].pad[1] == SPT_PRIM_SPHERE) {
-                for (int k = 0; k < 3; ++k) {
-                    u.lo[k] = -std::numeric_limits<float>::infinity();
-                    u.hi[k] = std::numeric_limits<float>::infinity();
-                }
-                return u;
-            }
         prim_box(first, u);
         for (uint32_t i = 1; i < count; ++i) {
             Box b;
@@ -219,10 +247,20 @@ private:
         }
     }
 
-    // A child of a binary node with its cut box (after plan()).
+    // A child of a binary node with the box the traversal gets (after plan()).
     void item(uint32_t bin, int s, Item& e) const {
         load_item(nodes_[bin], s, e);
-        cut(e, boxes_[2 * (size_t)bin + s]);
+        settle(bin, s, e);
+    }
+    void settle(uint32_t bin, int s, Item& e) const {
+        const Box& u = boxes_[2 * (size_t)bin + s];
+        if (loose_[2 * (size_t)bin + s])
+            for (int k = 0; k < 3; ++k) {
+                e.lo[k] = u.lo[k];
+                e.hi[k] = u.hi[k];
+            }
+        else
+            cut(e, u);
     }
 
     float leaf_cost(float a, uint32_t cnt) const {
@@ -234,6 +272,7 @@ private:
     void plan() {
         plan_.resize(n_);
         boxes_.resize(2 * (size_t)n_);
+        loose_.resize(2 * (size_t)n_);
         for (uint32_t i = n_; i-- > 0;) {  // children come after their parent
             Plan& p = plan_[i];
             Item l, r, b;
@@ -241,9 +280,17 @@ private:
                 Item& e = s == 0 ? l : r;
                 load_item(nodes_[i], s, e);
                 Box& u = boxes_[2 * (size_t)i + s];
-                if (e.cnt) {
+                if (e.cnt && loose(e, e.ref, e.cnt)) {
+                    loose_[2 * (size_t)i + s] = true;
+                    for (int k = 0; k < 3; ++k) {
+                        u.lo[k] = e.lo[k];
+                        u.hi[k] = e.hi[k];
+                    }
+                    widen(u);
+                } else if (e.cnt) {
                     u = range_box(e.ref, e.cnt);
                 } else {
+                    loose_[2 * (size_t)i + s] = loose_[2 * (size_t)e.ref] || loose_[2 * (size_t)e.ref + 1];
                     Item cl, cr;
                     item(e.ref, 0, cl);
                     item(e.ref, 1, cr);
@@ -252,7 +299,7 @@ private:
                         u.hi[k] = std::max(cl.hi[k], cr.hi[k]);
                     }
                 }
-                cut(e, u);
+                settle(i, s, e);
             }
             for (int k = 0; k < 3; ++k) {
                 b.lo[k] = std::min(l.lo[k], r.lo[k]);
@@ -302,7 +349,8 @@ private:
             p.kind = Part::kRange;
             p.first = e.ref;
             p.count = e.cnt;
-            p.leaf_box = add_box(given);
+            p.loose = loose_[2 * (size_t)bin + s];
+            p.leaf_box = add_box(given, e.ref, e.cnt);
             parts.push_back(p);
             return;
         }
@@ -329,17 +377,18 @@ private:
             Part q = p;
             q.first = p.first + (uint32_t)at;
             q.count = (uint32_t)std::min<uint64_t>(step, p.count - at);
-            cut(q.box, range_box(q.first, q.count));
+            if (!p.loose) cut(q.box, range_box(q.first, q.count));
             parts.push_back(q);
         }
     }
 
-    uint32_t add_box(const Item& e) {
+    // Index of the box of leaf [first, first + count), as the primitives keep it.
+    uint32_t add_box(const Item& e, uint32_t first, uint32_t count) {
         QuadBox b{};
         std::memcpy(b.mn, e.lo, sizeof(b.mn));
         std::memcpy(b.mx, e.hi, sizeof(b.mx));
         out_.boxes.push_back(b);
-        return (uint32_t)out_.boxes.size() - 1;
+        return ((uint32_t)out_.boxes.size() - 1) | (holds(e, first, count) ? 0u : kQuadExact);
     }
 
     void put(QuadPrim* dst, uint32_t tri, uint32_t box) {
@@ -357,7 +406,7 @@ private:
             Item e;
             load_item(nodes_[bin], s, e);
             if (e.cnt) {
-                const uint32_t box = add_box(e);
+                const uint32_t box = add_box(e, e.ref, e.cnt);
                 for (uint32_t k = 0; k < e.cnt; ++k) put(at++, e.ref + k, box);
             } else {
                 emit_leaves(e.ref, at);
@@ -444,6 +493,7 @@ private:
     float reach_ = 0.0f, least_ = 0.0f;  // prim_pad
     std::vector<Plan> plan_;
     std::vector<Box> boxes_;  // [2 i + s]: what child s of binary node i holds
+    std::vector<bool> loose_;  // [2 i + s]: that child is its box, whatever the node gives it
 };
 
 }  // namespace

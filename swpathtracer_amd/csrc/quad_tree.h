@@ -33,6 +33,9 @@ static_assert(sizeof(QuadNode) == 64, "QuadNode layout");
 constexpr uint32_t kQuadLeaf = 0x80000000u;
 constexpr uint32_t kQuadNone = 0xFFFFFFFFu;
 constexpr uint32_t kQuadSphere = 0x80000000u;  // QuadPrim::kind_mat: sphere flag beside the material
+// QuadPrim::box: the leaf's box does not hold its primitives, every hit is
+// compared with it
+constexpr uint32_t kQuadExact = 0x80000000u;
 
 // One primitive of a block of four (192 B, a lane each): the geometry of
 // spt_tri48, its index in leaf order (kQuadNone: unused slot, a degenerate

@@ -149,6 +149,7 @@ __device__ inline float fma_half(uint32_t pair, int hi, float a, float b) {
 // Exact acceptance test of a candidate at t (sbvh.cpp:494-496) with the box
 // of its leaf, which the ray must also meet.
 __device__ inline bool accept_exact(const DevScene& sc, V3 o, V3 d, float t, uint32_t box) {
+    box &= ~kQuadExact;
     const float4 b0 = sc.qboxes[2 * (size_t)box], b1 = sc.qboxes[2 * (size_t)box + 1];
     const V3 mn{b0.x, b0.y, b0.z}, mx{b1.x, b1.y, b1.z};
     float tn, tf;
@@ -156,8 +157,8 @@ __device__ inline bool accept_exact(const DevScene& sc, V3 o, V3 d, float t, uin
 }
 
 // The same test answered from the primitive alone where that is certain: the
-// point at (u, v) of a triangle lies inside its leaf's box, which holds the
-// vertices, so a hit point within 5e-4 of it lies inside the box +-1e-3 (with
+// point at (u, v) of a triangle lies inside its leaf's box where that holds the
+// vertices (no kQuadExact), so a hit point within 5e-4 of it lies inside the box +-1e-3 (with
 // coordinates up to 1024 the rounding of the triangle's point is below 2e-4).
 // A sphere (u = v = 0, v0 = centre) reaches its radius, as its box does, and no
 // further: its hit point may lie off it, and a root leaf's box, which the ray has
@@ -537,7 +538,7 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
             pass = pass & (t > 0.0f) & ((t < best) | ((t == best) & (idx < best_idx)));
             if (ballot(pass)) {
                 bool ok = pass;
-                const bool sure = sc.small_coords &&
+                const bool sure = sc.small_coords && !(__float_as_uint(c.z) & kQuadExact) &&
                                   accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
                                               (km & kQuadSphere) ? a.w : 0.0f);
                 if (ballot(pass & !sure)) {
@@ -610,9 +611,12 @@ __device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay ge
                 else
                     pass = tri_test(o, d, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x}, t, u, v);
                 pass = pass & (t > 0.0f) & ((t < h.t) | ((t == h.t) & (idx < h.idx)));
-                if (pass && ((sc.small_coords && accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
-                                                             (km & kQuadSphere) ? a.w : 0.0f)) ||
-                             accept_exact(sc, o, d, t, __float_as_uint(c.z)))) {
+                if (!pass) continue;
+                const uint32_t box = __float_as_uint(c.z);
+                const bool sure = sc.small_coords && !(box & kQuadExact) &&
+                                  accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
+                                              (km & kQuadSphere) ? a.w : 0.0f);
+                if (sure || accept_exact(sc, o, d, t, box)) {
                     h.t = t;
                     h.idx = idx;
                     h.mat = km & ~kQuadSphere;

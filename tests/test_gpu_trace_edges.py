@@ -89,3 +89,26 @@ def test_far_rays_of_any_length(device, distance, length):
     c = v.reshape(-1, 3, 3).mean(1)
     rays = _towards(rng, c[rng.integers(len(c), size=1_000_000)], distance, length)
     assert _check(device, v, rays) > 0.3
+
+
+@pytest.mark.parametrize("n, kept", [(3, 0.6), (3, 0.9), (9, 0.5), (3000, 0.5)])
+@pytest.mark.parametrize("length", [1.0, 2.0])
+def test_boxes_that_cut_their_primitives(device, n, kept, length):
+    """An uploaded tree may clip primitives: hits are accepted inside their
+    leaf's box only. The general path is the one that visits the reference's
+    own nodes."""
+    rng = np.random.default_rng(n)
+    v = (rng.uniform(-1, 1, (n, 1, 3)) + rng.uniform(-0.3, 0.3, (n, 3, 3))).astype(np.float32).reshape(-1, 9)
+    nodes, tris, _, box = api.Bvh(v).export()
+    for side in ("l", "r"):  # every other leaf keeps a part of its box
+        leaf = (nodes[side + "cnt"] > 0) & (rng.random(len(nodes)) < 0.5)
+        mn, mx = nodes[side + "min"], nodes[side + "max"]
+        mx[leaf] = mn[leaf] + np.float32(kept) * (mx[leaf] - mn[leaf])
+    if len(nodes) == 0:
+        box[3:] = box[:3] + np.float32(kept) * (box[3:] - box[:3])
+    device._check(device.lib.spt_upload_scene(device.h, nodes.ctypes.data if len(nodes) else None, len(nodes),
+                                              tris.ctypes.data, n, box.ctypes.data, None))
+    rays = _towards(rng, (v.reshape(-1, 3, 3)[rng.integers(n, size=200_000)] *
+                          rng.dirichlet([1, 1, 1], 200_000)[:, :, None]).sum(1), 1.5, length)
+    whole = _same(device.trace_host(rays), device.trace_host(rays, L.SPT_TRACE_UNPRUNED))
+    assert whole < 1.0 and (whole > 0.05 or kept == 0.6)  # there all three are clipped away
