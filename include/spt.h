@@ -385,15 +385,17 @@ typedef struct spt_tuning {
                                       several; 20 in spt_trace) */
     uint32_t wavefronts;           /* independent wavefronts run at once on their own streams, each
                                       with a share of the paths and of the queue capacity, so
-                                      one's traversal overlaps another's shading (1..4; reported as 3
-                                      when left at zero, which runs one) */
+                                      one's traversal overlaps another's shading (1..4). Zero runs
+                                      one and is reported as 3 with their launch shapes (64
+                                      shading blocks, 20 refill lanes); these three set
+                                      again as spt_get_tuning reported them still run one */
 } spt_tuning;
 spt_status spt_set_tuning(spt_ctx* ctx, const spt_tuning* t);
 spt_status spt_get_tuning(spt_ctx* ctx, spt_tuning* t);
 /* Times candidate tunings on a sample of the given render (about sample_paths
  * paths per trial; outputs discarded), keeps the fastest in the context and
- * returns it. Coordinate descent over capacity, grids, graph and check
- * interval. */
+ * returns it. Coordinate descent over wavefronts, capacity, grids, graph and
+ * check interval, from what the context's tuning runs. */
 spt_status spt_autotune(spt_ctx* ctx, const spt_camera* cam, const spt_render_params* params, uint64_t sample_paths,
                         spt_tuning* out);
 

@@ -54,13 +54,22 @@ double time_ms(spt_ctx* ctx, F run, spt_status& s) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// Coordinate descent over the tuning fields: each field in turn takes the
-// candidate value with the lowest time (best of two runs) with the others
-// held at their current best.
+// Coordinate descent over the tuning fields, from what a call runs with the
+// context's tuning: each field in turn takes the candidate value with the lowest
+// time (best of two runs) with the others held at their current best. The number
+// of wavefronts comes first, each with its own launch shapes where the caller
+// left them open, since the other fields depend on it.
 template <typename F>
 spt_status tune(spt_ctx* ctx, bool batch, F run, spt_tuning* out) {
     const spt_tuning saved = ctx->tuning;
-    spt_tuning best = resolve_tuning(ctx->tuning);
+    // 24 refill lanes where the caller left them open: what one wavefront's 48 act
+    // as, and never the 20 of a reported default (returned_tuning)
+    auto shapes = [&](spt_tuning& t) {
+        resolve_front_defaults(saved, t, t.wavefronts);
+        if (saved.refill_lanes == 0) t.refill_lanes = kMaxRefillLanes;
+    };
+    spt_tuning best = running_tuning(saved);
+    shapes(best);
     spt_status s = SPT_OK;
     auto trial = [&](const spt_tuning& t) {
         ctx->tuning = t;
@@ -75,13 +84,13 @@ spt_status tune(spt_ctx* ctx, bool batch, F run, spt_tuning* out) {
         std::vector<uint32_t> values;
     };
     std::vector<Dim> dims = {
+        {&spt_tuning::wavefronts, {1u, 2u, 3u}},
         {&spt_tuning::path_capacity, {1u << 23, 1u << 24, 1u << 25, 1u << 26, 1u << 27}},
         {&spt_tuning::extend_blocks_per_cu, {0u, 6u, 4u, 3u, 2u}},
         {&spt_tuning::shade_blocks_per_cu, {16u, 32u, 64u, 128u}},
         {&spt_tuning::use_graph, {2u, 1u}},
         {&spt_tuning::check_every, {2u, 4u, 8u}},
         {&spt_tuning::refill_lanes, {8u, 16u, 24u}},
-        {&spt_tuning::wavefronts, {3u, 2u, 1u}},
     };
     if (batch) {
         dims.push_back({&spt_tuning::tile_pixels, {1024u, 4096u, 16384u, 65536u}});
@@ -92,6 +101,7 @@ spt_status tune(spt_ctx* ctx, bool batch, F run, spt_tuning* out) {
             if (best.*(d.field) == v) continue;
             spt_tuning t = best;
             t.*(d.field) = v;
+            if (d.field == &spt_tuning::wavefronts) shapes(t);
             const double ms = trial(t);
             if (s != SPT_OK) break;
             if (ms < best_ms) {
@@ -122,13 +132,14 @@ spt_status spt_set_tuning(spt_ctx* ctx, const spt_tuning* t) {
     if (t->path_capacity > (1u << 27) || t->use_graph > 2 || t->shade_blocks_per_cu > 1024 ||
         t->extend_blocks_per_cu > 64 || t->check_every > 64 || t->refill_lanes > 64 || t->wavefronts > 4)
         return set_error(ctx, SPT_ERR_INVALID, "tuning value out of range");
-    ctx->tuning = *t;
+    ctx->tuning = ctx->told_default ? returned_tuning(*t) : *t;
     return SPT_OK;
 }
 
 spt_status spt_get_tuning(spt_ctx* ctx, spt_tuning* t) {
     if (!ctx || !t) return SPT_ERR_INVALID;
     *t = resolve_tuning(ctx->tuning);
+    if (t->wavefronts == 3) ctx->told_default = ctx->tuning.wavefronts == 0;
     return SPT_OK;
 }
 

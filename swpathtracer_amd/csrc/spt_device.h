@@ -8,6 +8,7 @@
 
 #include "spt.h"
 #include "quad_tree.h"
+#include "spt_tuning.h"
 #include "spt_internal.h"
 #include "spt_math.h"
 
@@ -18,11 +19,6 @@ constexpr int kBlock = 256;       // threads per block of the ray kernels (4 wav
 constexpr uint32_t kShadeFlat = 0, kShadeSmooth = 1, kShadeSphere = 2;
 constexpr int kLdsStack = 16;     // traversal stack entries per lane kept in LDS
 constexpr uint32_t kNoHit = SPT_MISS;
-// Idle lanes (four per ray) that make a traversal wave take new rays: 16 to 24
-// measure best for every kind of ray (extension rays of a 123M-path render 8:
-// 87 ms, 16: 84, 24: 83, 48: 98), so a larger spt_tuning.refill_lanes acts
-// as 24.
-constexpr uint32_t kRefillLanes = 20, kMaxRefillLanes = 24;
 
 // Materials the learned guide samples: one Lambertian / importance-sampled
 // GGX layer (kGuideSingle), or such a layer under one smooth dielectric coat
@@ -403,6 +399,7 @@ struct spt_ctx {
     spt_render_stats stats{};
     spt::GuideState guide;
     spt_tuning tuning{};  // zero fields: defaults
+    bool told_default = false;  // the last three wavefronts spt_get_tuning reported were the default's
     int wall_clock_khz = 100000;
     void* h_pin = nullptr;  // kPinBytes of pinned host memory for small read-backs
     // mapped host memory the bounce loop reports its progress to (see k_plan)
@@ -475,7 +472,6 @@ spt_status guide_eval_launch(spt_ctx* ctx, const float* d_q, uint32_t stride, ui
 spt_status guide_train_launch(spt_ctx* ctx, const float* d_rec, uint32_t n, float* loss_out, uint32_t rs);
 spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_params* p, float* d_rgb32,
                          double* d_rgb64, float* d_path_rgb);
-spt_tuning resolve_tuning(const spt_tuning& t);
 void scene_arrays(const spt_bvh* bvh, const float* verts, const float* normals, const uint32_t* mat_ids,
                   std::vector<spt_tri48>& tris, std::vector<float>& sh);
 uint32_t tree_stack_cap(const spt_node64* nodes, uint32_t n);

@@ -1089,28 +1089,6 @@ size_t guide_paths_lds_bytes() {
 
 }  // namespace
 
-// Defaults for the zero fields of a tuning.
-// Shading grid by wavefront count: one wavefront shades with 128 blocks per
-// CU; with other wavefronts beside it a smaller grid measured faster (1024-spp
-// mesh image, three wavefronts: 64 blocks 910 Mpaths/s, 32 893, 128 891). The
-// refill threshold of one wavefront acts as kMaxRefillLanes.
-void resolve_front_defaults(const spt_tuning& raw, spt_tuning& r, uint32_t fronts) {
-    r.shade_blocks_per_cu = raw.shade_blocks_per_cu ? raw.shade_blocks_per_cu : (fronts > 1 ? 64u : 128u);
-    r.refill_lanes = raw.refill_lanes ? raw.refill_lanes : (fronts > 1 ? kRefillLanes : 48u);
-}
-
-spt_tuning resolve_tuning(const spt_tuning& t) {
-    spt_tuning r = t;
-    if (r.path_capacity == 0) r.path_capacity = 1u << 27;
-    if (r.use_graph == 0) r.use_graph = 2;
-    if (r.tile_pixels == 0) r.tile_pixels = 4096;
-    if (r.tile_samples == 0) r.tile_samples = 16;
-    if (r.check_every == 0) r.check_every = 4;
-    if (r.wavefronts == 0) r.wavefronts = 3;
-    resolve_front_defaults(t, r, r.wavefronts);
-    return r;
-}
-
 // Validates one render's parameters and fills its job (everything but the
 // tree root). total = paths of the call.
 spt_status make_job(spt_ctx* ctx, const spt_camera* cam, const spt_render_params* prm, float* d_rgb32, double* d_rgb64,
@@ -1513,11 +1491,6 @@ spt_status run_fronts(spt_ctx* ctx, RenderArgs& a, uint64_t total, const spt_tun
     spt_tuning t1 = tn;
     uint32_t k = std::max<uint32_t>(1, std::min<uint32_t>(4, tn.wavefronts));
     if (a.rec_ring) k = 1;  // in-call training trains from one wavefront's ring
-    // one wavefront unless the caller asks for more: its traversal and shading
-    // each fill the chip, and with other streams in the process several lose
-    // (1, 2, 3 of them: guided 800x600, 64 spp 63.9, 74.7, 72.5 ms, 400x300,
-    // 36 spp 11.5, 11.4, 11.6; batch of 12 scenes 59.3, 64.5, 66.3)
-    if (ctx->tuning.wavefronts == 0) k = 1;
     while (k > 1 && total / k < (1ull << 21)) --k;
     if (k == 1) {
         t1.wavefronts = 1;
@@ -1651,7 +1624,7 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
     if (ctx->guide.cand_per_path > 0.0 && ctx->guide.records_cap > 0) {
         double want = ctx->guide.cand_per_path * (double)total;
         if (a.rec_ring) {
-            const spt_tuning tn = resolve_tuning(ctx->tuning);
+            const spt_tuning tn = running_tuning(ctx->tuning);
             const double per_bounce = ctx->guide.cand_per_path / ctx->guide.rays_per_path *
                                       (double)std::min<uint64_t>(total, tn.path_capacity);
             want = per_bounce * (double)(ctx->guide.train_every + tn.check_every + 1) * 4.0;
@@ -1663,7 +1636,7 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
     a.walk = ctx->layered && !a.guided;
     spt_render_stats stats{};
     stats.paths = total;
-    s = run_fronts<false>(ctx, a, total, resolve_tuning(ctx->tuning), stats);
+    s = run_fronts<false>(ctx, a, total, running_tuning(ctx->tuning), stats);
     stats.ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     ctx->stats = stats;
     return s;
@@ -1671,7 +1644,7 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
 
 spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
     auto t0 = std::chrono::steady_clock::now();
-    const spt_tuning tn = resolve_tuning(ctx->tuning);
+    const spt_tuning tn = running_tuning(ctx->tuning);
     const uint32_t nj = (uint32_t)b.jobs.size();
     std::vector<Job> jobs = b.jobs;
     for (Job& jb : jobs) {
