@@ -85,8 +85,11 @@ constexpr int kTrainTile = 128, kTrainBlock = 512, kTrainRow = kTrainTile + 8;  
 struct TrainLds {
     FwdWeights fw;
     // W2^T, W3^T, W4^T as MFMA operands of the backward pass (as in FwdWeights,
-    // rows = inputs; W4 with 16 more outputs of weight 0: a v_mfma 16x16x16
-    // issued right behind the 16x16x32 whose result it adds to gave wrong rows)
+    // rows = inputs; W4 with 16 more outputs of weight 0). A third k-tile of 16
+    // as a v_mfma 16x16x16 is not safe here: the compiler puts no wait between it
+    // and a 16x16x32 whose result it adds to, and as a pair on one accumulator,
+    // two instructions apart, they give wrong sums (nearly every element off; exact
+    // with three other products in between, or with a second 16x16x32).
     uint4 w2t[4 * 2 * 64], w3t[4 * 2 * 64], w4t[4 * 2 * 64];
     unsigned short x[2][kEnc][kTrainRow];  // two tiles in turn
     unsigned short h1[kHid][kTrainRow], h2[kHid][kTrainRow], h3[kHid][kTrainRow];
