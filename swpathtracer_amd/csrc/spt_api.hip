@@ -197,8 +197,6 @@ void scene_arrays(const spt_bvh* bvh, const float* verts, const float* normals, 
     }
 }
 
-uint32_t tree_stack_cap(const spt_node64* nodes, uint32_t n) { return tree_depth(nodes, n) + 1; }
-
 // ---------------------------------------------------------------------------
 // The compressed four-wide tree spt_bvh_wide returns (for inspection; the
 // kernels read the quad tree).

@@ -15,8 +15,8 @@ namespace spt {
 namespace {
 
 void free_batch(BatchData& b) {
-    void* ptrs[] = {b.d_nodes, b.d_qnodes, b.d_qprims,     b.d_qboxes, b.d_tris, b.d_shading, b.d_mats,
-                    b.d_jobs,  b.d_tiles,  b.d_tile_start, b.d_done,   b.d_clock};
+    void* ptrs[] = {b.d_qnodes, b.d_qprims,     b.d_qboxes, b.d_shading, b.d_mats,
+                    b.d_jobs,   b.d_tiles,      b.d_tile_start, b.d_done,   b.d_clock};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     b = BatchData{};
@@ -175,9 +175,8 @@ spt_status spt_autotune(spt_ctx* ctx, const spt_camera* cam, const spt_render_pa
 spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_t n, spt_batch** out) {
     if (!ctx || !scenes || n == 0 || !out) return SPT_ERR_INVALID;
     *out = nullptr;
-    std::vector<spt_node64> nodes;
+    uint64_t node_base = 0, tri_base = 0;  // of the scenes so far
     QuadTree qt;
-    std::vector<spt_tri48> tris;
     std::vector<float> sh;
     std::vector<spt_material> mats;
     spt_batch* b = new (std::nothrow) spt_batch();
@@ -207,22 +206,16 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
         std::vector<spt_tri48> bt;
         std::vector<float> bs;
         scene_arrays(sc.bvh, sc.verts, sc.normals, sc.mat_ids, bt, bs);
-        const uint64_t node_base = nodes.size(), tri_base = tris.size(), mat_base = mats.size();
+        const uint64_t mat_base = mats.size();
         if (node_base + bn.size() >= (1u << 30) || tri_base + bt.size() >= (1ull << 32) || mat_base + sc.n_mats >= 65536)
             return fail(set_error(ctx, SPT_ERR_UNSUPPORTED, "batch exceeds 2^30 nodes / 2^32 triangles"));
         for (const spt_tri48& t : bt)
             if (t.pad[0] >= sc.n_mats) return fail(set_error(ctx, SPT_ERR_INVALID, "a triangle references a missing material"));
-        // rebase child references, triangle materials and shading materials
-        for (spt_node64 nd : bn) {
-            nd.lref += (nd.lcnt == 0) ? (uint32_t)node_base : (uint32_t)tri_base;
-            nd.rref += (nd.rcnt == 0) ? (uint32_t)node_base : (uint32_t)tri_base;
-            nodes.push_back(nd);
-        }
+        // rebase triangle and shading materials
         for (spt_tri48& t : bt) {
             t.pad[0] += (uint32_t)mat_base;
             d.has_spheres = d.has_spheres || t.pad[1] == SPT_PRIM_SPHERE;
         }
-        tris.insert(tris.end(), bt.begin(), bt.end());
         d.small_coords = d.small_coords && quad_small_coords(bt.data(), (uint32_t)bt.size());
         const float* rb = bvh_root_box(sc.bvh);
         const uint64_t qnode_base = qt.nodes.size();
@@ -244,16 +237,15 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
             jb.rmax[k] = rb[3 + k];
         }
         jb.node0 = (uint32_t)qnode_base;  // the traversal starts at the scene's root
-        d.stack_cap = std::max(d.stack_cap, tree_stack_cap(bn.data(), (uint32_t)bn.size()));
         d.jobs.push_back(jb);
+        node_base += bn.size();
+        tri_base += bt.size();
     }
     (void)hipSetDevice(ctx->device);
     uint64_t bytes = 0;
-    spt_status s = upload_vec(ctx, reinterpret_cast<spt_node64**>(&d.d_nodes), nodes, "batch nodes", bytes);
-    if (s == SPT_OK) s = upload_vec(ctx, &d.d_qnodes, qt.nodes, "batch quad nodes", bytes);
+    spt_status s = upload_vec(ctx, &d.d_qnodes, qt.nodes, "batch quad nodes", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, &d.d_qprims, qt.prims, "batch quad blocks", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, &d.d_qboxes, qt.boxes, "batch leaf boxes", bytes);
-    if (s == SPT_OK) s = upload_vec(ctx, reinterpret_cast<spt_tri48**>(&d.d_tris), tris, "batch triangles", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, reinterpret_cast<float**>(&d.d_shading), sh, "batch shading", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, &d.d_mats, mats, "batch materials", bytes);
     if (s == SPT_OK) s = upload_vec(ctx, &d.d_jobs, d.jobs, "batch jobs", bytes);
@@ -262,8 +254,7 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
     if (s != SPT_OK) return fail(s);
     d.small_tree = qt.small();
     d.layered = std::any_of(mats.begin(), mats.end(), [](const spt_material& m) { return m.n_layers > 1; });
-    d.n_nodes = (uint32_t)nodes.size();
-    d.n_tris = (uint32_t)tris.size();
+    d.n_tris = (uint32_t)tri_base;
     d.n_mats = (uint32_t)mats.size();
     d.device_bytes = bytes;
     *out = b;

@@ -249,15 +249,13 @@ struct BatchTile {
 
 // Device arrays and per-scene jobs of a batch (spt_batch_*).
 struct BatchData {
-    float4* d_nodes = nullptr;
     QuadNode* d_qnodes = nullptr;
     QuadPrim* d_qprims = nullptr;
     QuadBox* d_qboxes = nullptr;
-    float4* d_tris = nullptr;
     float4* d_shading = nullptr;
     spt_material* d_mats = nullptr;
     bool layered = false;  // some material has several layers
-    uint32_t n_nodes = 0, n_tris = 0, n_mats = 0, stack_cap = 0, stack_cap4 = 0;
+    uint32_t n_tris = 0, n_mats = 0, stack_cap4 = 0;
     bool has_spheres = false, small_coords = true, small_tree = false;
     std::vector<Job> jobs;  // host copy: sampling, outputs, roots
     Job* d_jobs = nullptr;
@@ -474,7 +472,6 @@ spt_status launch_render(spt_ctx* ctx, const spt_camera* cam, const spt_render_p
                          double* d_rgb64, float* d_path_rgb);
 void scene_arrays(const spt_bvh* bvh, const float* verts, const float* normals, const uint32_t* mat_ids,
                   std::vector<spt_tri48>& tris, std::vector<float>& sh);
-uint32_t tree_stack_cap(const spt_node64* nodes, uint32_t n);
 spt_status make_job(spt_ctx* ctx, const spt_camera* cam, const spt_render_params* prm, float* d_rgb32, double* d_rgb64,
                     float* d_path_rgb, Job& jb, uint64_t& total);
 // A multi-scene render (spt_batch_*): every job of the batch, or with

@@ -1715,21 +1715,17 @@ spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
     if (s == SPT_OK) s = check_hip(ctx, hipStreamSynchronize(st), "batch upload");  // host vectors go out of scope
     if (s != SPT_OK) return s;
 
-    RenderArgs a{};
-    a.sc.nodes = b.d_nodes;
+    RenderArgs a{};  // no binary tree: only casters and counting traversals read it
     a.sc.qnodes = reinterpret_cast<const uint32_t*>(b.d_qnodes);
     a.sc.qprims = reinterpret_cast<const float4*>(b.d_qprims);
     a.sc.qboxes = reinterpret_cast<const float4*>(b.d_qboxes);
     a.sc.small_coords = b.small_coords ? 1u : 0u;
     a.sc.small_tree = b.small_tree ? 1u : 0u;
     a.sc.stack_cap4 = b.stack_cap4;
-    a.sc.tris = b.d_tris;
     a.sc.shading = b.d_shading;
     a.sc.mats = b.d_mats;
     a.sc.n_tris = b.n_tris;
-    a.sc.n_nodes = b.n_nodes;
     a.sc.n_mats = b.n_mats;
-    a.sc.stack_cap = b.stack_cap;
     a.sc.has_spheres = b.has_spheres ? 1u : 0u;
     a.jobs = b.d_jobs;
     a.tiles = b.d_tiles;
