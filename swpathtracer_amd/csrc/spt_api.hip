@@ -218,18 +218,15 @@ constexpr uint32_t kNoChild = 0xFFFFFFFFu;
 // Compressed four-wide node (64 B):
 // each axis has a per-node grid origin + q * 2^e, and every child bound is
 // rounded outward to a byte q (lo down, hi up), so the decoded boxes contain
-// the exact padded child boxes (the traversal visits a superset of the exact
-// four-wide tree's boxes; results do not depend on visit order).
+// the exact padded child boxes.
 //   word 0-2: grid origin x y z (float); word 3: biased exponent bytes of
 //   2^e_x, 2^e_y, 2^e_z (float exponent field, bytes 0-2)
 //   words 4-9: q of lo.x, hi.x, lo.y, hi.y, lo.z, hi.z (byte i = child i)
 //   words 10-11: 16-bit triangle counts of the children (0: inner or unused;
 //   0xFFFF: 65535 or more, the full count is in the leaf's box record)
 //   words 12-15: children: NodeQ index (inner), first triangle (leaf), kNoChild
-// A leaf's range is read from the node that holds it, which the traversal
-// has just visited; its exact box (the reference's hit-point-inside-leaf
-// test) sits in a side array at 4 * node + slot and is read only when a
-// triangle of the leaf passes the t tests.
+// A leaf's exact box (the reference's hit-point-inside-leaf test) sits in a
+// side array at 4 * node + slot.
 struct NodeQ {
     float ox, oy, oz;
     uint32_t exps;
@@ -330,8 +327,7 @@ void collapse4(const spt_node64* nodes, uint32_t n, std::vector<Node4>& out) {
     }
 }
 
-// The value the traversal decodes for byte q (qdec): origin + q * scale in
-// float, q * scale exact.
+// The bound byte q stands for: origin + q * scale in float, q * scale exact.
 float grid_value(float origin, uint32_t q, float scale) {
     const volatile float p = (float)q * scale;
     return origin + p;
@@ -376,7 +372,7 @@ uint32_t quantize_axis(const float* lo, const float* hi, const bool* used, float
 // tri_base. Returns false when an index would not fit its field.
 bool compress4(const std::vector<Node4>& in, uint32_t tri_base, std::vector<NodeQ>& nodes, std::vector<LeafRec>& leaves) {
     const uint64_t node_base = nodes.size();
-    // leaf stack entries hold node << 2 | slot below kLeafBit
+    // leaf boxes are numbered 4 * node + slot in 31 bits
     if (node_base + in.size() > (1ull << 29)) return false;
     leaves.resize(4 * (node_base + in.size()), LeafRec{});
     for (size_t j = 0; j < in.size(); ++j) {

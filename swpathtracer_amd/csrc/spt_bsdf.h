@@ -45,7 +45,7 @@ __device__ __forceinline__ V3 schlick_r0(const float* r0, float c) {
 
 // Exact conductor Fresnel for complex IOR eta + i k from a medium of IOR 1
 // (textbook form, Pharr/Jakob/Humphreys PBR 3rd ed. sec. 8.2.1), with
-// dek = eta^2 - k^2 and fek = 4 eta^2 k^2 (prepare_layer).
+// dek = eta^2 - k^2 and fek = 4 eta^2 k^2 (prepare_material).
 __device__ __forceinline__ float fresnel_conductor(float ci, float dek, float fek) {
     ci = gmin(gmax(ci, -1.0f), 1.0f);
     const float c2 = ci * ci, s2 = 1.0f - c2;
@@ -82,7 +82,7 @@ __device__ __forceinline__ bool layer_opaque(const spt_layer& l) { return l.type
 
 __device__ __forceinline__ V3 layer_f(const spt_layer& l, V3 wo, V3 wi) {
     switch (l.type) {
-        case SPT_BSDF_LAMBERTIAN: {  // lambertian.cpp:9-16 (brdf_ = kd / pi: prepare_layer)
+        case SPT_BSDF_LAMBERTIAN: {  // lambertian.cpp:9-16 (brdf_ = kd / pi: prepare_material)
             if (wi.y > 0.0f) return V3{l.r0[0], l.r0[1], l.r0[2]};
             return V3{0.0f, 0.0f, 0.0f};
         }
@@ -208,7 +208,7 @@ __device__ __forceinline__ BSample layer_sample(const spt_layer& l, V3 wo, Draws
             if (l.sampler == SPT_SAMPLER_UNIFORM) return sample_uniform(r);
             return BSample{V3{-wo.x, wo.y, -wo.z}, 1.0f};  // smooth_specular_bsdf_sampler.cpp:5-7
         case SPT_BSDF_SMOOTH_DIELECTRIC: {                 // smooth_dielectric.cpp:30-51
-            // r0 = Schlick reflectance (fresnel_schlick.cpp:20-38), 1 / ior, 1 / ior^2 (prepare_layer)
+            // r0 = Schlick reflectance (fresnel_schlick.cpp:20-38), 1 / ior, 1 / ior^2 (prepare_material)
             const bool inside = wo.y < 0.0f;
             const float a = (inside ? l.ior * l.ior : l.r0[2]) * (1.0f - wo.y * wo.y);
             if (a > 1.0f) return BSample{V3{-wo.x, wo.y, -wo.z}, 1.0f};

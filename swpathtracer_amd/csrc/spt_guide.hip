@@ -17,7 +17,7 @@ namespace {
 // register-resident MLP on 4 groups of 16. Three blocks a CU, as many as their
 // LDS lets in at once (a million queries 51.7 us, with four 56.7, six 52.0,
 // sixteen 55.5), and no block-wide waits. Bound by the 196 B a query moves: a
-// million queries 48 us (before: 59), 41 at the rate of a large copy.
+// million queries 50 us (before: 62), 41 at the rate of a large copy.
 __global__ __launch_bounds__(kBlock) void k_guide_eval(const float* __restrict__ theta,
                                                        const unsigned short* __restrict__ wbf,
                                                        const float* __restrict__ q, uint32_t stride, uint32_t n,

@@ -21,8 +21,8 @@
 //
 // Measured on the 1M-triangle mesh in the box, a lane per ray before: rays off
 // its surfaces, 4,096: 294 -> 32 us, 65,536: 1409 -> 94 us, 1M: 1.67 -> 0.27
-// ms, 4.2M: 3.46 -> 0.73 ms, 16.8M: 7.3 -> 2.5 ms (2.3 -> 6.8 Grays/s);
-// 1920x1080 primary rays 1.00 -> 0.41 ms; the extension rays of a 123M-path
+// ms, 4.2M: 3.46 -> 0.70 ms, 16.8M: 7.3 -> 2.3 ms (2.3 -> 7.3 Grays/s);
+// 1920x1080 primary rays 1.00 -> 0.33 ms; the extension rays of a 123M-path
 // render 139 -> 84 ms. Bound by VALU issue (about 80% of the issue cycles at 42
 // of 64 lanes) once a launch has millions of rays, by the longest rays' chains
 // of loads below that.
