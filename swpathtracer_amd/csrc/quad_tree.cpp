@@ -205,6 +205,16 @@ private:
         }
         return true;
     }
+    bool small_coords(uint32_t first, uint32_t count) const {
+        for (uint32_t i = first; i < first + count; ++i) {
+            const spt_tri48& t = tris_[i];
+            for (int k = 0; k < 3; ++k)
+                if (!(std::fabs(t.v0[k]) <= 1024.0f && std::fabs(t.v0[k] + t.e1[k]) <= 1024.0f &&
+                      std::fabs(t.v0[k] + t.e2[k]) <= 1024.0f))
+                    return false;
+        }
+        return true;
+    }
     // Whether hits in a leaf are not accepted at its primitives alone: a sphere's
     // test accepts hit points off it when the direction is not of unit length.
     bool loose(const Item& e, uint32_t first, uint32_t count) const {
@@ -388,7 +398,8 @@ private:
         std::memcpy(b.mn, e.lo, sizeof(b.mn));
         std::memcpy(b.mx, e.hi, sizeof(b.mx));
         out_.boxes.push_back(b);
-        return ((uint32_t)out_.boxes.size() - 1) | (holds(e, first, count) ? 0u : kQuadExact);
+        const bool near = holds(e, first, count) && small_coords(first, count);
+        return ((uint32_t)out_.boxes.size() - 1) | (near ? 0u : kQuadExact);
     }
 
     void put(QuadPrim* dst, uint32_t tri, uint32_t box) {
@@ -501,17 +512,6 @@ private:
 uint32_t append_quad_tree(const spt_node64* nodes, uint32_t n_nodes, const spt_tri48* tris, uint32_t n_tris,
                           const float* root_box, uint32_t prim_base, QuadTree& out) {
     return Builder(nodes, n_nodes, tris, root_box, prim_base, out).run(n_tris, root_box);
-}
-
-bool quad_small_coords(const spt_tri48* tris, uint32_t n_tris) {
-    for (uint32_t i = 0; i < n_tris; ++i) {
-        const spt_tri48& t = tris[i];
-        for (int k = 0; k < 3; ++k)
-            if (!(std::fabs(t.v0[k]) <= 1024.0f && std::fabs(t.v0[k] + t.e1[k]) <= 1024.0f &&
-                  std::fabs(t.v0[k] + t.e2[k]) <= 1024.0f))
-                return false;
-    }
-    return true;
 }
 
 }  // namespace spt

@@ -33,8 +33,9 @@ static_assert(sizeof(QuadNode) == 64, "QuadNode layout");
 constexpr uint32_t kQuadLeaf = 0x80000000u;
 constexpr uint32_t kQuadNone = 0xFFFFFFFFu;
 constexpr uint32_t kQuadSphere = 0x80000000u;  // QuadPrim::kind_mat: sphere flag beside the material
-// QuadPrim::box: the leaf's box does not hold its primitives, every hit is
-// compared with it
+// QuadPrim::box: every hit is compared with the leaf's box, which does not hold
+// its primitives, or a coordinate of them exceeds 1024 (a float ulp, 6e-5 below
+// it, is far inside the 5e-4 margin of the traversal's acceptance shortcut)
 constexpr uint32_t kQuadExact = 0x80000000u;
 
 // One primitive of a block of four (192 B, a lane each): the geometry of
@@ -68,10 +69,5 @@ struct QuadTree {
 // entries a traversal of it can need, 0 when an index does not fit its field.
 uint32_t append_quad_tree(const spt_node64* nodes, uint32_t n_nodes, const spt_tri48* tris, uint32_t n_tris,
                           const float* root_box, uint32_t prim_base, QuadTree& out);
-
-// Whether every coordinate of the primitives is small enough for the
-// traversal's acceptance shortcut: at most 1024 in magnitude, where a float
-// ulp (6e-5 below it) is far inside the shortcut's 5e-4 margin.
-bool quad_small_coords(const spt_tri48* tris, uint32_t n_tris);
 
 }  // namespace spt

@@ -636,7 +636,6 @@ spt_status spt_upload_scene(spt_ctx* ctx, const spt_node64* nodes, uint32_t n_no
     ctx->root_leaf = n_nodes == 0 ? n_tris : 0;
     ctx->stack_cap = tree_depth(nodes, n_nodes) + 1;
     ctx->stack_cap4 = cap4;
-    ctx->small_coords = quad_small_coords(tris, n_tris);
     ctx->small_tree = qt.small();
     ctx->one_block = qt.prims.size() == 4;
     ctx->max_mat = 0;

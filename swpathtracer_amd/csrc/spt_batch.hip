@@ -216,7 +216,6 @@ spt_status spt_batch_create(spt_ctx* ctx, const spt_batch_scene* scenes, uint32_
             t.pad[0] += (uint32_t)mat_base;
             d.has_spheres = d.has_spheres || t.pad[1] == SPT_PRIM_SPHERE;
         }
-        d.small_coords = d.small_coords && quad_small_coords(bt.data(), (uint32_t)bt.size());
         const float* rb = bvh_root_box(sc.bvh);
         const uint64_t qnode_base = qt.nodes.size();
         const uint32_t cap4 = append_quad_tree(bn.data(), (uint32_t)bn.size(), bt.data(), (uint32_t)bt.size(), rb,

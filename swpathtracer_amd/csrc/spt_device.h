@@ -41,7 +41,6 @@ struct DevScene {
     uint32_t n_mats;
     uint32_t stack_cap;  // traversal stack entries a lane may need (inner-node depth + 1)
     uint32_t stack_cap4; // same for the quad traversal's tree (3 per level + 1)
-    uint32_t small_coords; // every coordinate at most 1024 (quad_small_coords)
     uint32_t small_tree;   // the quad nodes and blocks are under 4 GiB each (32-bit offsets)
     uint32_t has_spheres;  // some primitive record is a sphere (uniform branch in the leaf loops)
 };
@@ -256,7 +255,7 @@ struct BatchData {
     spt_material* d_mats = nullptr;
     bool layered = false;  // some material has several layers
     uint32_t n_tris = 0, n_mats = 0, stack_cap4 = 0;
-    bool has_spheres = false, small_coords = true, small_tree = false;
+    bool has_spheres = false, small_tree = false;
     std::vector<Job> jobs;  // host copy: sampling, outputs, roots
     Job* d_jobs = nullptr;
     BatchTile* d_tiles = nullptr;
@@ -374,7 +373,7 @@ struct spt_ctx {
     uint32_t root_leaf = 0;
     uint32_t stack_cap = 0;
     uint32_t max_mat = 0;  // largest material id referenced by a triangle
-    bool has_spheres = false, small_coords = false, small_tree = false;
+    bool has_spheres = false, small_tree = false;
     bool one_block = false;  // at most four primitives: closest hits without a tree
     bool has_scene = false;
     std::vector<spt_material> h_mats;
@@ -413,7 +412,6 @@ struct spt_ctx {
         s.qnodes = reinterpret_cast<const uint32_t*>(d_qnodes);
         s.qprims = reinterpret_cast<const float4*>(d_qprims);
         s.qboxes = reinterpret_cast<const float4*>(d_qboxes);
-        s.small_coords = small_coords ? 1u : 0u;
         s.small_tree = small_tree ? 1u : 0u;
         s.stack_cap4 = stack_cap4;
         s.tris = d_tris;

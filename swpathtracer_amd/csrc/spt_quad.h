@@ -125,12 +125,14 @@ __device__ inline bool root_test(V3 o, V3 d, V3 inv, V3 mn, V3 mx) {
 // into the 1M-triangle mesh in the box, of size 2, 0.26 ms from 100 away, 0.81
 // from 5,000, 11 from 60,000.
 __device__ inline float ray_slack(const Root& r, V3 o, V3 d) {
-    const bool longer = !(dot(d, d) <= 1.002f);
     const V3 e = r.mx - r.mn, c = o - (r.mn + e * 0.5f);
     const float diag2 = dot(e, e), far2 = dot(c, c);
-    if (!(far2 > diag2)) return longer ? 1e-3f : 0.0f;
-    const float far = sqrtf(far2);
-    return (longer ? 1e-3f : fminf(1e-3f, 1e-3f * (far / sqrtf(diag2) - 1.0f))) + 1e-6f * far;
+    float slack = dot(d, d) <= 1.002f ? 0.0f : 1e-3f;
+    if (far2 > diag2) {
+        const float far = sqrtf(far2);
+        slack = fminf(1e-3f, slack + 1e-3f * (far / sqrtf(diag2) - 1.0f)) + 1e-6f * far;
+    }
+    return slack;
 }
 
 template <int CTRL>
@@ -538,7 +540,7 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
             pass = pass & (t > 0.0f) & ((t < best) | ((t == best) & (idx < best_idx)));
             if (ballot(pass)) {
                 bool ok = pass;
-                const bool sure = sc.small_coords && !(__float_as_uint(c.z) & kQuadExact) &&
+                const bool sure = !(__float_as_uint(c.z) & kQuadExact) &&
                                   accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
                                               (km & kQuadSphere) ? a.w : 0.0f);
                 if (ballot(pass & !sure)) {
@@ -613,7 +615,7 @@ __device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay ge
                 pass = pass & (t > 0.0f) & ((t < h.t) | ((t == h.t) & (idx < h.idx)));
                 if (!pass) continue;
                 const uint32_t box = __float_as_uint(c.z);
-                const bool sure = sc.small_coords && !(box & kQuadExact) &&
+                const bool sure = !(box & kQuadExact) &&
                                   accept_near(o, d, t, u, v, V3{a.x, a.y, a.z}, V3{a.w, b.x, b.y}, V3{b.z, b.w, c.x},
                                               (km & kQuadSphere) ? a.w : 0.0f);
                 if (sure || accept_exact(sc, o, d, t, box)) {

@@ -1719,7 +1719,6 @@ spt_status launch_batch(spt_ctx* ctx, BatchData& b, uint32_t sample_div) {
     a.sc.qnodes = reinterpret_cast<const uint32_t*>(b.d_qnodes);
     a.sc.qprims = reinterpret_cast<const float4*>(b.d_qprims);
     a.sc.qboxes = reinterpret_cast<const float4*>(b.d_qboxes);
-    a.sc.small_coords = b.small_coords ? 1u : 0u;
     a.sc.small_tree = b.small_tree ? 1u : 0u;
     a.sc.stack_cap4 = b.stack_cap4;
     a.sc.shading = b.d_shading;

@@ -119,8 +119,9 @@ def _check(lib, nodes, tris, box, base=0, first_node=0, first_block=0):
         s = slice(first, first + cnt)
         assert np.all(leaf_of[s] == -1)
         leaf_of[s] = k
-        exact[s] = not (np.all(lo[s] >= mn - 1e-4) and np.all(hi[s] <= mx + 1e-4))
-        if exact[first] or sphere[s].any():
+        clips = not (np.all(lo[s] >= mn - 1e-4) and np.all(hi[s] <= mx + 1e-4))
+        exact[s] = clips or max(np.abs(lo[s]).max(), np.abs(hi[s]).max()) > 1024
+        if clips or sphere[s].any():
             need_lo[s], need_hi[s] = mn - 1e-3, mx + 1e-3
         else:
             m = (mn - 1e-3, mx + 1e-3) if len(nodes) == 0 else (mn, mx)
