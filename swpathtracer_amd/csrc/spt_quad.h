@@ -99,20 +99,15 @@ __host__ __device__ inline uint32_t quad_spill_words(uint32_t cap) {
 // becomes inf - inf.
 __device__ inline float safe_rcp(float d) { return (fabsf(d) > 0x1p-60f) ? rcp_rn(d) : copysignf(0x1p60f, d); }
 
-// Whether a hit can be accepted on the ray o + t d, t > 0, in a scene with the
-// root box [mn, mx]: the reference's own test of the ray's line against that box
-// (acceleration/aabb.cpp:31-99, quotients included: the box has no padding, and
-// rays towards a vertex or edge on it are decided by a rounding), unless the box
-// ends behind the origin. Not just behind it, where a rounding gives t its sign;
-// rays that leave a surface are moved 1e-3 along them, and those that leave the
-// scene (about 43% of 4.2M rays off the surfaces of the mesh in the box) end here: with
-// origins up to 1e-3 outside kept as well these rays took 823 us instead of 696.
-// inv = safe_rcp of d.
-__device__ inline bool root_test(V3 o, V3 d, V3 inv, V3 mn, V3 mx) {
-    if (__builtin_expect(fminf(fminf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)) <= 0x1p-60f, 0))
-        inv = V3{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
-    float tn, tf;
-    return slab(o, inv, mn, mx, tn, tf) && !(tf < -1e-4f);
+// Whether the ray meets the box [mn, mx] at t >= 0: one FMA per slab plane and
+// IEEE min/max (a NaN product keeps the box).
+__device__ inline bool root_test(V3 inv, V3 oi, V3 mn, V3 mx) {
+    const float t0x = fmaf(mn.x, inv.x, oi.x), t1x = fmaf(mx.x, inv.x, oi.x);
+    const float t0y = fmaf(mn.y, inv.y, oi.y), t1y = fmaf(mx.y, inv.y, oi.y);
+    const float t0z = fmaf(mn.z, inv.z, oi.z), t1z = fmaf(mx.z, inv.z, oi.z);
+    const float tmin = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fmaxf(fminf(t0z, t1z), 0.0f));
+    const float tmax = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fmaxf(t0z, t1z));
+    return tmin <= tmax && tmin < __builtin_inff();
 }
 
 // What a ray adds to the tree's box paddings (prim_pad in quad_tree.cpp): they
@@ -396,7 +391,8 @@ __device__ inline void trace_shares(const DevScene& sc, uint32_t n, RayShares sh
                         // a ray with a non-finite component cannot hit anything (every
                         // t comparison fails) but would pass every box test: a miss
                         const float sum = po.x + po.y + po.z + pd.x + pd.y + pd.z;
-                        keep = (sum - sum == 0.0f) && root_test(po, pd, pi, R.mn, R.mx);
+                        keep = (sum - sum == 0.0f) &&
+                               root_test(pi, V3{-po.x * pi.x, -po.y * pi.y, -po.z * pi.z}, R.mn, R.mx);
                         if (!keep) {
                             Hit h;
                             h.t = __builtin_inff();

@@ -67,18 +67,6 @@ def test_ray_beside_a_root_leaf(device):
     _check(device, v, r)
 
 
-@pytest.mark.parametrize("n", [7, 60, 500])
-def test_vertices_that_span_the_root(device, n):
-    """The same in scenes with a tree: rays towards the extreme vertices."""
-    rng = np.random.default_rng(n)
-    v = rng.uniform(-0.7, 0.7, (n, 9)).astype(np.float32)
-    v[:6] *= np.float32(1.4)
-    p = v.reshape(-1, 3)
-    extreme = np.concatenate([p[p.argmin(0)], p[p.argmax(0)]])
-    hit = _check(device, v, _towards(rng, np.repeat(extreme, 20_000, axis=0), 1.5))
-    assert hit > 0.1
-
-
 @pytest.mark.parametrize("distance, length", [(60.0, 2.0), (5000.0, 2.0), (60_000.0, 2.0), (60_000.0, 30.0),
                                               (60_000.0, 1.0)])
 def test_far_rays_of_any_length(device, distance, length):
