@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_camera_rays(DevCamera cam, float4* _
 }
 
 // Scratch of the allocation-free closest-hit entry point
-// (spt_trace_noalloc): word 0 holds the overflow flag, then come the
+// (spt_trace_noalloc) in scenes with a tree: word 0 holds the overflow flag, then come the
 // traversal's ray counters and the traversal stacks' spill area. Each device holds its own copy; host code reaches it
 // only through the address hipGetSymbolAddress returns for that device.
 static __device__ __align__(256) uint32_t scratch[SPT_NOALLOC_SCRATCH_WORDS];
@@ -426,6 +426,17 @@ spt_status launch_trace_noalloc(spt_ctx* ctx, const spt_ray32* d_rays, uint64_t 
         return set_error(ctx, SPT_ERR_INVALID, "spt_trace_noalloc: more than SPT_NOALLOC_MAX_RAYS rays");
     if (!ctx->scratch) return set_error(ctx, SPT_ERR_STATE, "spt_trace_noalloc: no static scratch on this device");
     if (n == 0) return SPT_OK;
+    if (ctx->one_block) {  // no stack, no counters: the kernel of spt_trace, and its results
+        const DevScene sc = ctx->scene();
+        return block_launches(
+            ctx, n,
+            [&](uint64_t base, uint32_t cnt, uint32_t grid) {
+                hipLaunchKernelGGL(k_trace_block, dim3(grid), dim3(kBlock), 0, ctx->stream, sc,
+                                   reinterpret_cast<const float4*>(d_rays) + 2 * base, cnt,
+                                   reinterpret_cast<uint2*>(d_hits) + base);
+            },
+            "trace (no allocation) launch");
+    }
     const void* kern = reinterpret_cast<const void*>(&k_trace_q<false, true>);
     // blocks whose stack entries beyond the LDS part fit the scratch
     const uint64_t per_block = quad_spill_words(ctx->stack_cap4);

@@ -36,6 +36,14 @@ def _check(device, verts, rays, kinds=None):
     return _same(device.trace_host(rays), O.Scene(verts, kinds=kinds).trace(rays)[:2])
 
 
+def _trace_noalloc(device, rays):
+    dr, dh = device.to_device(rays), device.alloc(8 * len(rays))
+    device._check(device.lib.spt_trace_noalloc(device.h, dr.ptr, len(rays), dh.ptr))
+    device.sync()
+    h = dh.download(np.uint32, (len(rays), 2))
+    return h[:, 0].view(np.float32).copy(), h[:, 1].copy()
+
+
 def _vertices_and_edges(rng, verts, n):
     """Half of the points on vertices, half on edges."""
     v = verts.reshape(-1, 3, 3)[rng.integers(len(verts), size=n)]
@@ -51,8 +59,10 @@ def test_vertices_and_edges_in_one_block(device, n):
     rng = np.random.default_rng(n)
     for _ in range(4):
         v = rng.uniform(-1, 1, (n, 9)).astype(np.float32)
-        hit = _check(device, v, _towards(rng, _vertices_and_edges(rng, v, 50_000), 1.5))
+        rays = _towards(rng, _vertices_and_edges(rng, v, 50_000), 1.5)
+        hit = _check(device, v, rays)
         assert 0.1 < hit < 0.9
+        _same(_trace_noalloc(device, rays), device.trace_host(rays))
     floor = rng.uniform(-1, 1, (n, 3, 3)).astype(np.float32)
     floor[:, :, 1] = 0.25
     _check(device, floor.reshape(n, 9), _towards(rng, _vertices_and_edges(rng, floor, 50_000), 1.5))
