@@ -582,8 +582,9 @@ __device__ inline void trace_quads(const DevScene& sc, uint32_t n, uint32_t* ray
 // meet the root's box, as the reference asks before it tests the leaf
 // (acceleration/sbvh.cpp:423-515): that box has no padding, so a ray towards a
 // vertex or edge on it may miss it by a rounding. Only hits pay for that test.
-// 185x305 depth image of a sphere 4 us, 11.5 with the quads, whose set-up and
-// rounds a wave are latency here; 1900x1050 13 us. Bound by VALU issue.
+// 185x305 depth image of a sphere 3.2 us, 11.5 with the quads, whose set-up and
+// rounds a wave are latency here; 1900x1050 10.3 us (9.7 without the root's box).
+// Bound by VALU issue.
 template <typename GetRay, typename PutHit>
 __device__ inline void trace_one_block(const DevScene& sc, uint32_t n, GetRay get_ray, PutHit put_hit) {
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
